@@ -43,7 +43,7 @@ constexpr int kQT = 64, kKB = 64, kKPad = kD + 8, kVPad = kKB + 8;  // MFMA pref
 constexpr int kMfmaAttnTokens = 320;   // prompts of this many tokens run attention_mfma
 constexpr int kMfmaAttnContext = 256;  // so do fewer tokens over this many positions of context
 constexpr int kMaxAttnChunks = 16;    // attention_mfma over key chunks: tiles x chunks at most
-constexpr int kSplitChunk = 64;   // split attention: positions per workgroup
+constexpr int kSplitChunk = 128;  // split attention: positions per workgroup
 constexpr int kSplitBelow = 32;   // fewer tokens than this use the split attention ...
 constexpr int kSplitContext = 128;  // ... over more than this many positions of context
 constexpr int kMaxSplit = 16;     // K splits of one GEMM (their partials are summed in a fixed order)
@@ -1110,93 +1110,220 @@ __global__ void __launch_bounds__(kD) attention_mfma_merge(const Tok* __restrict
   out[(size_t)t * kQS + h * kD + d] = (uint16_t)f32_to_bf16(y);
 }
 
-// Few tokens: the context of each (token, KV head) is split over workgroups of
-// kSplitChunk positions.  attn_split_scores writes the chunk's scores and its
-// (max m_j, sum l_j of exp(s - m_j)) per head; attn_split_pv takes the global
-// max M and the sum S = sum_j l_j * exp(m_j - M) (fixed order, identical in
-// every workgroup of the token), forms the probabilities and a partial P@V;
-// attn_split_merge adds the partials in chunk order.
-__global__ void __launch_bounds__(256) attn_split_scores(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok,
-                                                         int L, Cache c, float scale, int nch,
-                                                         float* __restrict__ scores, float2* __restrict__ ml) {
+// Context-split attention: one token per row of the launch (a batched decode step; a few tokens of a
+// prompt), its context in chunks of kSplitChunk positions, one workgroup of 4 waves per (chunk, KV
+// head, token), in HF's two passes over three launches:
+// - attn_chunk_scores requests the chunk's K rows (a lane row of 16 takes one position, so one wave
+//   instruction reads four whole rows), scores them as HF rounds them, stores the scores (fp32)
+//   and the chunk's (max m, sum l of exp(s - m)) per head.  RAW: q, k, v come as the q/k/v
+//   projection left them; each workgroup forms its q heads (head RMSNorm + RoPE) behind the K
+//   requests, and the chunk that holds the token's position also forms its k row, appends K and V
+//   and takes its own k from LDS, so no workgroup of the launch reads that cache row (valid only
+//   when no other token of the launch is of this sequence).  Otherwise Q is finished and K/V
+//   appended by an earlier launch;
+// - attn_chunk_pv requests the chunk's V rows, takes the global (M, L) from the chunks' pairs (one
+//   pair per lane, the same order in every workgroup of the token), forms the probabilities
+//   bf16(exp(s - M) * (1 / L)) one position per lane, and leaves the chunk's P@V partial;
+// - attn_chunk_merge adds the partials in a fixed order and rounds to bf16.
+// K and V are read once each, so HBM bounds it; what it is held to is that every chunk's rows are
+// requested at once (32 KB per workgroup) and that the work per position after the dot products
+// (exponentials, rounding) is done by one lane and not by the 16 that share a row.  A fixed chunk
+// rather than a fixed number of splits per token keeps the longest sequence of a ragged batch
+// from setting the time.  Qwen3-0.6B, us per layer for the three launches, against the forms it
+// replaced: 8 sequences of 5..1500 positions 32.3 -> 15.6, 3 of 5000..6100 74.7 -> 21.8, 48 of
+// 100..1000 86 -> 35.
+template <bool RAW>
+__global__ void __launch_bounds__(256) attn_chunk_scores(const uint16_t* __restrict__ src, const Tok* __restrict__ tok,
+                                                         int L, const uint16_t* __restrict__ q_norm,
+                                                         const uint16_t* __restrict__ k_norm,
+                                                         const uint16_t* __restrict__ cos_t,
+                                                         const uint16_t* __restrict__ sin_t, Cache c, float eps,
+                                                         float scale, int nch, float* __restrict__ scores,
+                                                         float2* __restrict__ ml) {
+  constexpr int NR = kSplitChunk / 16;  // 16-position rounds, all in flight
   __shared__ float sc[2][kSplitChunk];
-  __shared__ float red[2][4];
-  const int t = blockIdx.x, g = blockIdx.y, j = blockIdx.z, t16 = threadIdx.x & 15;
+  __shared__ __align__(16) uint16_t qs[2][kD], kn[kD];
+  __shared__ float wm[4], wl[4];
+  const int j = blockIdx.x, g = blockIdx.y, t = blockIdx.z;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, slot = lane >> 4,
+            t16 = lane & 15;
   const Tok tk = tok[t];
-  const int C = tk.valid ? tk.pos + 1 : 0;
-  const int c0 = j * kSplitChunk;
-  if (c0 >= C) return;
-  const int n = min(C - c0, kSplitChunk);
+  const int pos = tk.pos, c0 = j * kSplitChunk, n = min(pos + 1 - c0, kSplitChunk);
+  if (!tk.valid || n <= 0) return;
   const size_t base = cache_base(c, tk, L, g);
+  const uint16_t* kc = c.k + base;
+  const bool own = RAW && n <= kSplitChunk && pos < c0 + kSplitChunk;  // the chunk of the token's own position
   u32x4 qv[2];
+  // waves 0, 1: q heads 2g, 2g+1; wave 2: k head g; wave 3: v head g
+  const int h = w < 2 ? 2 * g + w : (w == 2 ? kNQ + g : kNQ + kNKV + g);
+  uint32_t x0b = 0, x1b = 0, w0b = 0, w1b = 0, c0b = 0, c1b = 0, s0b = 0, s1b = 0;
+  if constexpr (RAW) {  // a CU returns loads in order, so these go out ahead of the K rows
+    const uint16_t* xs = src + (size_t)t * kNQKV + h * kD;
+    const uint16_t* nw = w < 2 ? q_norm : k_norm;
+    const uint16_t* cr = cos_t + (size_t)pos * kD;
+    const uint16_t* sr = sin_t + (size_t)pos * kD;
+    x0b = ldu16(xs + lane), x1b = ldu16(xs + lane + 64);
+    w0b = ldu16(nw + lane), w1b = ldu16(nw + lane + 64);
+    c0b = ldu16(cr + lane), c1b = ldu16(cr + lane + 64);
+    s0b = ldu16(sr + lane), s1b = ldu16(sr + lane + 64);
+  } else {
 #pragma unroll
-  for (int h = 0; h < 2; h++) qv[h] = ld16(Q + (size_t)t * kQS + (2 * g + h) * kD + 8 * t16);
-  float m[2] = {-INFINITY, -INFINITY};
-  score_chunk(c.k + base, qv, scale, c0, c0 + n, sc[0], sc[1], m);
-  block_max2(m, red);
-  float l[2] = {0.f, 0.f};
-  const size_t ncap = (size_t)nch * kSplitChunk;
-  for (int i = threadIdx.x; i < n; i += 256) {
+    for (int hh = 0; hh < 2; hh++) qv[hh] = ld16(src + (size_t)t * kQS + (2 * g + hh) * kD + 8 * t16);
+  }
+  // positions past the token's own repeat the last one before it (masked below); its own row is not
+  // in the cache yet (RAW)
+  const int plast = RAW ? max(pos - 1, 0) : pos;
+  u32x4 kx[NR];
 #pragma unroll
-    for (int h = 0; h < 2; h++) {
-      const float s = sc[h][i];
-      scores[((size_t)t * kNQ + 2 * g + h) * ncap + c0 + i] = s;
-      l[h] += exp_acc(s - m[h]);
+  for (int r = 0; r < NR; r++) kx[r] = ld16(kc + (size_t)min(c0 + 16 * r + 4 * w + slot, plast) * kD + 8 * t16);
+  u32x4 k_now = u32x4{0, 0, 0, 0};
+  if constexpr (RAW) {
+    if (w == 3) {
+      if (own) {
+        c.v[base + (size_t)pos * kD + lane] = (uint16_t)x0b;
+        c.v[base + (size_t)pos * kD + lane + 64] = (uint16_t)x1b;
+      }
+    } else {
+      const float x0 = bf16_to_f32(x0b), x1 = bf16_to_f32(x1b);
+      const float ss = wave_sum(x0 * x0 + x1 * x1);
+      const float rstd = rcp_sqrt_torch(__fdiv_rn(ss, (float)kD) + eps);
+      const float n0 = bf16r(bf16_to_f32(w0b) * bf16r(x0 * rstd));
+      const float n1 = bf16r(bf16_to_f32(w1b) * bf16r(x1 * rstd));
+      const float cc0 = bf16_to_f32(c0b), cc1 = bf16_to_f32(c1b), ss0 = bf16_to_f32(s0b), ss1 = bf16_to_f32(s1b);
+      const uint16_t y0 = (uint16_t)f32_to_bf16(bf16r(bf16r(n0 * cc0) + bf16r(-n1 * ss0)));
+      const uint16_t y1 = (uint16_t)f32_to_bf16(bf16r(bf16r(n1 * cc1) + bf16r(n0 * ss1)));
+      uint16_t* dst = w < 2 ? qs[w] : kn;
+      dst[lane] = y0;
+      dst[lane + 64] = y1;
+      if (w == 2 && own) {
+        c.k[base + (size_t)pos * kD + lane] = y0;
+        c.k[base + (size_t)pos * kD + lane + 64] = y1;
+      }
     }
-  }
-  block_sum2(l, red);
-  if (threadIdx.x < 2)
-    ml[((size_t)t * kNQ + 2 * g + threadIdx.x) * nch + j] = make_float2(m[threadIdx.x], l[threadIdx.x]);
-}
-
-__global__ void __launch_bounds__(256) attn_split_pv(const Tok* __restrict__ tok, int L, Cache c, int nch,
-                                                     const float* __restrict__ scores, const float2* __restrict__ ml,
-                                                     float* __restrict__ pvp) {
-  __shared__ float pr[2][kSplitChunk];
-  __shared__ float pv[4][2][kD];
-  const int t = blockIdx.x, g = blockIdx.y, j = blockIdx.z;
-  const Tok tk = tok[t];
-  const int C = tk.valid ? tk.pos + 1 : 0;
-  const int c0 = j * kSplitChunk;
-  if (c0 >= C) return;
-  const int n = min(C - c0, kSplitChunk), used = (C + kSplitChunk - 1) / kSplitChunk;
-  const size_t ncap = (size_t)nch * kSplitChunk;
-  float M[2], inv[2];
+    __syncthreads();
 #pragma unroll
-  for (int h = 0; h < 2; h++) {
-    const float2* mlh = ml + ((size_t)t * kNQ + 2 * g + h) * nch;
-    float mx = -INFINITY;
-    for (int q = 0; q < used; q++) mx = fmaxf(mx, mlh[q].x);
-    float s = 0.f;
-    for (int q = 0; q < used; q++) s += mlh[q].y * exp_acc(mlh[q].x - mx);
-    M[h] = mx;
-    inv[h] = __fdiv_rn(1.0f, s);
+    for (int hh = 0; hh < 2; hh++) qv[hh] = *reinterpret_cast<const u32x4*>(&qs[hh][8 * t16]);
+    k_now = *reinterpret_cast<const u32x4*>(&kn[8 * t16]);
   }
-  for (int i = threadIdx.x; i < n; i += 256) {
 #pragma unroll
-    for (int h = 0; h < 2; h++)
-      pr[h][i] = bf16r(exp_acc(scores[((size_t)t * kNQ + 2 * g + h) * ncap + c0 + i] - M[h]) * inv[h]);
+  for (int r = 0; r < NR; r++) {
+    const int i = 16 * r + 4 * w + slot;
+    const u32x4 kr = RAW && c0 + i == pos ? k_now : kx[r];
+    const float s0 = row16_sum(dot8(kr, qv[0], 0.f)), s1 = row16_sum(dot8(kr, qv[1], 0.f));
+    if (t16 < 2) sc[t16][i] = t16 ? s1 : s0;
   }
   __syncthreads();
-  float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-  pv_chunk(c.v + cache_base(c, tk, L, g) + (size_t)c0 * kD, pr[0], pr[1], n, acc);
-  const float y = pv_merge_waves(acc, pv);
-  pvp[(((size_t)t * nch + j) * kNQ + 2 * g) * kD + threadIdx.x] = y;
+  // one (head, position) per thread: the score as HF rounds it, the chunk's maximum and sum
+  static_assert(kSplitChunk == 128, "256 threads: 2 heads x 128 positions, two waves per head");
+  const int hh = w >> 1, i = threadIdx.x & (kSplitChunk - 1);
+  const float s = bf16r(bf16r(sc[hh][i]) * scale);
+  if (i < n) scores[((size_t)t * kNQ + 2 * g + hh) * ((size_t)nch * kSplitChunk) + c0 + i] = s;
+  const float m = wave_max_all(i < n ? s : -INFINITY);
+  const float l = wave_total(i < n && m > -INFINITY ? exp_acc(s - m) : 0.f);
+  if (lane == 0) {
+    wm[w] = m;
+    wl[w] = l;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    const int q = 2 * threadIdx.x;
+    const float ma = wm[q], mb = wm[q + 1], mx = fmaxf(ma, mb);
+    const float la = ma == -INFINITY ? 0.f : wl[q] * exp_acc(ma - mx);
+    const float lb = mb == -INFINITY ? 0.f : wl[q + 1] * exp_acc(mb - mx);
+    ml[((size_t)t * kNQ + 2 * g + threadIdx.x) * nch + j] = make_float2(mx, la + lb);
+  }
 }
 
-// out[t][i] = bf16(sum over the token's chunks of the partial P@V), i over
-// the 16 x 128 head outputs; grid (token, 8 slices of 256).
-__global__ void __launch_bounds__(256) attn_split_merge(const Tok* __restrict__ tok, int nch,
-                                                        const float* __restrict__ pvp, uint16_t* __restrict__ out) {
-  const int t = blockIdx.x, i = blockIdx.y * 256 + threadIdx.x;
+__global__ void __launch_bounds__(256) attn_chunk_pv(const Tok* __restrict__ tok, int L, Cache c, int nch,
+                                                     const float* __restrict__ scores, const float2* __restrict__ ml,
+                                                     float* __restrict__ pvp) {
+  constexpr int NR = kSplitChunk / 16;
+  __shared__ float pr[2][kSplitChunk];
+  __shared__ float wacc[4][2][kD];
+  const int j = blockIdx.x, g = blockIdx.y, t = blockIdx.z;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, slot = lane >> 4,
+            t16 = lane & 15;
   const Tok tk = tok[t];
-  const int C = tk.valid ? tk.pos + 1 : 0;
-  const int used = (C + kSplitChunk - 1) / kSplitChunk;
-  const float* src = pvp + (size_t)t * nch * kQS + i;
-  float y = 0.f;
-#pragma unroll 8
-  for (int q = 0; q < used; q++) y += src[(size_t)q * kQS];
-  out[(size_t)t * kQS + i] = (uint16_t)f32_to_bf16(y);
+  const int pos = tk.pos, c0 = j * kSplitChunk, n = min(pos + 1 - c0, kSplitChunk);
+  if (!tk.valid || n <= 0) return;
+  const uint16_t* vc = c.v + cache_base(c, tk, L, g);
+  // this thread's score (head w / 2, position i of the chunk) and its head's pairs, then the V rows
+  const int hh = w >> 1, i = threadIdx.x & (kSplitChunk - 1), used = pos / kSplitChunk + 1;
+  const size_t row = (size_t)t * kNQ + 2 * g + hh;
+  const float s = scores[row * ((size_t)nch * kSplitChunk) + c0 + min(i, n - 1)];
+  const float2* mlh = ml + row * nch;
+  const float2 first = lane < used ? mlh[lane] : make_float2(-INFINITY, 0.f);
+  u32x4 vx[NR];
+#pragma unroll
+  for (int r = 0; r < NR; r++) vx[r] = ld16(vc + (size_t)min(c0 + 16 * r + 4 * w + slot, pos) * kD + 8 * t16);
+  float mx = first.x;
+  for (int q = 64 + lane; q < used; q += 64) mx = fmaxf(mx, mlh[q].x);
+  mx = wave_max_all(mx);
+  float ls = first.x == -INFINITY ? 0.f : first.y * exp_acc(first.x - mx);
+  for (int q = 64 + lane; q < used; q += 64) {
+    const float2 e = mlh[q];
+    ls += e.x == -INFINITY ? 0.f : e.y * exp_acc(e.x - mx);
+  }
+  const float inv = __fdiv_rn(1.0f, wave_total(ls));
+  pr[hh][i] = i < n ? bf16r(exp_acc(s - mx) * inv) : 0.f;
+  __syncthreads();
+  float acc[2][8];
+#pragma unroll
+  for (int q = 0; q < 2; q++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[q][e] = 0.f;
+#pragma unroll
+  for (int r = 0; r < NR; r++) {
+    const int p = 16 * r + 4 * w + slot;
+    // rows past the last position carry probability 0 and a repeated row; taken as zeros, so that
+    // an infinity in that row is not counted twice (0 * inf)
+    const bool live = p < n;
+    const u32x4 vr = u32x4{live ? vx[r].x : 0u, live ? vx[r].y : 0u, live ? vx[r].z : 0u, live ? vx[r].w : 0u};
+    const float vf[8] = {lo_bf16(vr.x), hi_bf16(vr.x), lo_bf16(vr.y), hi_bf16(vr.y),
+                         lo_bf16(vr.z), hi_bf16(vr.z), lo_bf16(vr.w), hi_bf16(vr.w)};
+    const float p0 = pr[0][p], p1 = pr[1][p];
+#pragma unroll
+    for (int e = 0; e < 8; e++) {
+      acc[0][e] = __builtin_fmaf(p0, vf[e], acc[0][e]);
+      acc[1][e] = __builtin_fmaf(p1, vf[e], acc[1][e]);
+    }
+  }
+  // the wave's four lane rows, then the four waves in order
+#pragma unroll
+  for (int q = 0; q < 2; q++) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[q][e] = rows_sum4(acc[q][e]);
+    if (lane < 16) {
+      *reinterpret_cast<f32x4*>(&wacc[w][q][8 * t16]) = f32x4{acc[q][0], acc[q][1], acc[q][2], acc[q][3]};
+      *reinterpret_cast<f32x4*>(&wacc[w][q][8 * t16 + 4]) = f32x4{acc[q][4], acc[q][5], acc[q][6], acc[q][7]};
+    }
+  }
+  __syncthreads();
+  const int d = threadIdx.x & 127, ho = threadIdx.x >> 7;  // 256 threads: both heads' dims
+  pvp[(((size_t)t * nch + j) * kNQ + 2 * g) * kD + threadIdx.x] =
+      ((wacc[0][ho][d] + wacc[1][ho][d]) + wacc[2][ho][d]) + wacc[3][ho][d];
+}
+
+// The output of (token t, head): its used chunks' partials added, rounded to bf16 (zeros for an invalid
+// token).  Thread (q, c4) adds every eighth chunk from q for dims 4c4..+3, then the eight sums in order.
+__global__ void __launch_bounds__(256) attn_chunk_merge(const Tok* __restrict__ tok, int nch,
+                                                        const float* __restrict__ pvp, uint16_t* __restrict__ out) {
+  __shared__ f32x4 part[8][32];
+  const int t = blockIdx.x, h = blockIdx.y, q = threadIdx.x >> 5, c4 = threadIdx.x & 31;
+  const Tok tk = tok[t];
+  const int used = tk.valid ? tk.pos / kSplitChunk + 1 : 0;
+  const float* src = pvp + ((size_t)t * nch * kNQ + h) * kD + 4 * c4;
+  f32x4 y = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+  for (int j = q; j < used; j += 8) y += *reinterpret_cast<const f32x4*>(src + (size_t)j * kQS);
+  part[q][c4] = y;
+  __syncthreads();
+  if (q == 0) {
+#pragma unroll
+    for (int k = 1; k < 8; k++) y += part[k][c4];
+    *reinterpret_cast<uint2*>(out + (size_t)t * kQS + h * kD + 4 * c4) =
+        make_uint2(pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]));
+  }
 }
 
 // ---------------------------------------------------------------- LM head
@@ -1458,13 +1585,11 @@ __global__ void __launch_bounds__(kLmWaves * 64) lm_head_rows(const uint16_t* __
 // ---------------------------------------------------------------- decode step, few sequences
 //
 // One token per sequence, at most 16 sequences (one MFMA row tile), contexts
-// up to kFusedCtx: seven launches per layer instead of eleven.
+// of any length: seven launches per layer instead of eleven.
 //
 //   gemm_rows<NORM>(q,k,v)   input RMSNorm in the prologue, bf16 q|k|v out
-//   attention_split          q/k head norm + RoPE, K/V append, scores and each
-//                            position split's (max, sum) over all CUs;
-//                            attention_pv the probabilities (HF's rounding) times
-//                            V per split; attention_merge adds the splits
+//   attn_chunk_scores<RAW>   q/k head norm + RoPE, K/V append, the chunks' scores;
+//   attn_chunk_pv, _merge    probabilities times V per chunk, the chunks' sum
 //   gemm_rows(o)             epilogue: residual add into the hidden rows
 //   gemm_rows<NORM>(g|u)     post-attention RMSNorm in the prologue, SiLU(g)*u out
 //   gemm_rows(down)          epilogue: residual add
@@ -1476,8 +1601,6 @@ __global__ void __launch_bounds__(kLmWaves * 64) lm_head_rows(const uint16_t* __
 
 constexpr int kRowWaves = 16;
 constexpr int kMaxRowsH = 2048;   // largest hidden size a NORM prologue stages in LDS
-constexpr int kFusedCtx = 4096;   // longest context of the fused decode attention
-constexpr int kAttnRounds = 4;    // fused attention: 64-position rounds of K or V loads in flight per wave
 
 enum RowEpi : int { kEpiStore = 0, kEpiResidual = 1, kEpiSiluMul = 2 };
 
@@ -1642,268 +1765,6 @@ __global__ void __launch_bounds__(NW * 64) gemm_rows(const uint16_t* __restrict_
   else *dst = (uint16_t)f32_to_bf16(y);
 }
 
-// Decode-step attention, split over positions: S workgroups of kSplitWaves
-// waves per (sequence's token, KV head), S * T * 8 >= 256, so that every CU
-// streams K/V (one workgroup per (token, KV head) left 224 of 256 CUs idle at
-// four sequences), in HF's two passes over three launches:
-// - attention_split requests the token's q/k/v head values, norm weights and
-//   RoPE row, then every K row of its positions [pb, pe) (a CU returns loads in
-//   order, so the small loads come first); forms the q heads 2g, 2g+1 and k head
-//   g (head RMSNorm + RoPE, as HF), and split 0 appends the token's K/V at its
-//   position (the token's own K is used from LDS, so no workgroup of this launch
-//   reads that cache row); scores its positions as HF rounds them, stores them
-//   (fp32) and writes the split's (max m, sum l of exp(s - m)) per head;
-// - attention_pv merges the S (m, l) pairs into the global (M, L) in split order
-//   (the same in every workgroup of the token), forms the probabilities
-//   bf16(exp(s - M) * (1 / L)) as HF rounds them, and multiplies them with the V
-//   rows of its positions: a partial P@V per split;
-// - attention_merge adds the S partials in split order and rounds to bf16.
-// Valid only when no other token of the launch writes this sequence's cache
-// (one token per sequence).
-constexpr int kSplitWaves = 4;    // waves per workgroup
-constexpr int kSplitRounds = 8;   // 16-position rounds of K (or V) rows in flight per wave
-constexpr int kMaxAttnSplit = 32;
-
-struct AttnPart {
-  float acc[2][kD];  // P@V of heads 2g, 2g+1 over the split's positions (probabilities normalised)
-  float m[2], l[2];  // the split's maximum score and sum of exp(s - m)
-};
-
-// position splits per (token, KV head) for T tokens
-int attn_splits(int T) { return std::min(kMaxAttnSplit, std::max(1, 256 / (kNKV * T))); }
-
-// scores[(t * kNQ + head) * cap + p] of token t's positions p: written by attention_split, read
-// by attention_pv
-__global__ void __launch_bounds__(kSplitWaves * 64) attention_split(
-    const uint16_t* __restrict__ QKV, const Tok* __restrict__ tok, int L, const uint16_t* q_norm,
-    const uint16_t* k_norm, const uint16_t* cos_t, const uint16_t* sin_t, Cache c, float eps, float scale,
-    AttnPart* __restrict__ part, float* __restrict__ scores, int cap, uint16_t* __restrict__ out) {
-  __shared__ uint16_t qs[2][kD], kn[kD];
-  __shared__ float wm[kSplitWaves][2], wl[kSplitWaves][2];
-  const int t = blockIdx.x, g = blockIdx.y, sp = blockIdx.z, S = gridDim.z;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, slot = lane >> 4, t16 = lane & 15;
-  const Tok tk = tok[t];
-  if (!tk.valid) {
-    if (sp == 0 && threadIdx.x < 2 * kD) out[(size_t)t * kQS + 2 * g * kD + threadIdx.x] = 0;
-    return;
-  }
-  const int pos = tk.pos, C = pos + 1;
-  const int chunk = (C + S - 1) / S;
-  const int pb = min(C, sp * chunk), pe = min(C, pb + chunk);
-  const size_t base = cache_base(c, tk, L, g);
-  const uint16_t* kc = c.k + base;
-  // waves 0, 1: q heads 2g, 2g+1; wave 2: k head g; wave 3: v head g
-  const int h = w < 2 ? 2 * g + w : (w == 2 ? kNQ + g : kNQ + kNKV + g);
-  const uint16_t* src = QKV + (size_t)t * kNQKV + h * kD;
-  const uint16_t* nw = w < 2 ? q_norm : k_norm;
-  const uint32_t x0b = ldu16(src + lane), x1b = ldu16(src + lane + 64);
-  const uint32_t w0b = ldu16(nw + lane), w1b = ldu16(nw + lane + 64);
-  const uint16_t* cr = cos_t + (size_t)pos * kD;
-  const uint16_t* sr = sin_t + (size_t)pos * kD;
-  const uint32_t c0b = ldu16(cr + lane), c1b = ldu16(cr + lane + 64);
-  const uint32_t s0b = ldu16(sr + lane), s1b = ldu16(sr + lane + 64);
-  // lane (slot, t16) of wave w takes dims 8*t16..+7 of position p0 + 16r + 4w + slot in round r;
-  // positions outside [pb, pe) and pos itself load row 0 (every cache has it) and are masked
-  u32x4 kx[kSplitRounds];
-  auto issue = [&](int p0) {
-#pragma unroll
-    for (int r = 0; r < kSplitRounds; r++) {
-      const int p = p0 + 16 * r + 4 * w + slot;
-      kx[r] = ld16(kc + (size_t)((p < pe && p != pos) ? p : 0) * kD + 8 * t16);
-    }
-  };
-  issue(pb);
-  {
-    const float x0 = bf16_to_f32(x0b), x1 = bf16_to_f32(x1b);
-    if (w == 3) {
-      if (sp == 0) {
-        c.v[base + (size_t)pos * kD + lane] = (uint16_t)x0b;
-        c.v[base + (size_t)pos * kD + lane + 64] = (uint16_t)x1b;
-      }
-    } else {
-      const float ss = wave_sum(x0 * x0 + x1 * x1);
-      const float rstd = rcp_sqrt_torch(__fdiv_rn(ss, (float)kD) + eps);
-      const float n0 = bf16r(bf16_to_f32(w0b) * bf16r(x0 * rstd));
-      const float n1 = bf16r(bf16_to_f32(w1b) * bf16r(x1 * rstd));
-      const float c0 = bf16_to_f32(c0b), c1 = bf16_to_f32(c1b), s0 = bf16_to_f32(s0b), s1 = bf16_to_f32(s1b);
-      const uint16_t y0 = (uint16_t)f32_to_bf16(bf16r(bf16r(n0 * c0) + bf16r(-n1 * s0)));
-      const uint16_t y1 = (uint16_t)f32_to_bf16(bf16r(bf16r(n1 * c1) + bf16r(n0 * s1)));
-      if (w < 2) {
-        qs[w][lane] = y0;
-        qs[w][lane + 64] = y1;
-      } else {
-        kn[lane] = y0;
-        kn[lane + 64] = y1;
-        if (sp == 0) {
-          c.k[base + (size_t)pos * kD + lane] = y0;
-          c.k[base + (size_t)pos * kD + lane + 64] = y1;
-        }
-      }
-    }
-  }
-  __syncthreads();
-  u32x4 qv[2];
-#pragma unroll
-  for (int hh = 0; hh < 2; hh++) qv[hh] = *reinterpret_cast<const u32x4*>(&qs[hh][8 * t16]);
-  const u32x4 k_now = *reinterpret_cast<const u32x4*>(&kn[8 * t16]);
-  float* const sc_out = scores + ((size_t)t * kNQ + 2 * g) * cap;
-  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};
-  for (int p0 = pb; p0 < pe; p0 += 16 * kSplitRounds) {
-    if (p0 != pb) issue(p0);  // positions beyond the first 16 * kSplitRounds of the split
-    float sc[kSplitRounds][2], bm[2] = {-INFINITY, -INFINITY};
-#pragma unroll
-    for (int r = 0; r < kSplitRounds; r++) {
-      const int p = p0 + 16 * r + 4 * w + slot;
-      const u32x4 kr = p == pos ? k_now : kx[r];
-#pragma unroll
-      for (int hh = 0; hh < 2; hh++) {
-        const float x = bf16r(bf16r(row16_sum(dot8(kr, qv[hh], 0.f))) * scale);
-        sc[r][hh] = p < pe ? x : -INFINITY;
-        bm[hh] = fmaxf(bm[hh], sc[r][hh]);
-        if (t16 == 0 && p < pe) sc_out[(size_t)hh * cap + p] = x;
-      }
-    }
-#pragma unroll
-    for (int hh = 0; hh < 2; hh++) {
-      float a, b;
-      swap16(bm[hh], a, b);
-      bm[hh] = fmaxf(a, b);
-      swap32(bm[hh], a, b);
-      bm[hh] = fmaxf(a, b);
-      // rescale the running sum to the new maximum
-      const float mn = fmaxf(m[hh], bm[hh]);
-      l[hh] *= m[hh] == -INFINITY ? 0.f : exp_acc(m[hh] - mn);
-      m[hh] = mn;
-    }
-#pragma unroll
-    for (int r = 0; r < kSplitRounds; r++)
-#pragma unroll
-      for (int hh = 0; hh < 2; hh++) l[hh] += sc[r][hh] == -INFINITY ? 0.f : exp_acc(sc[r][hh] - m[hh]);
-  }
-  // the wave's four rows summed (every lane of a row holds the same terms; lane 0 speaks for them)
-#pragma unroll
-  for (int hh = 0; hh < 2; hh++) {
-    l[hh] = rows_sum4(l[hh]);
-    if (lane == 0) {
-      wm[w][hh] = m[hh];
-      wl[w][hh] = l[hh];
-    }
-  }
-  __syncthreads();
-  // this workgroup's (max, sum): the waves rescaled to its maximum, in wave order
-  AttnPart* pt = part + ((size_t)t * kNKV + g) * S;
-  if (threadIdx.x < 2) {
-    const int hh = threadIdx.x;
-    float mx = -INFINITY;
-#pragma unroll
-    for (int q = 0; q < kSplitWaves; q++) mx = fmaxf(mx, wm[q][hh]);
-    float ls = 0.f;
-#pragma unroll
-    for (int q = 0; q < kSplitWaves; q++) ls += wm[q][hh] == -INFINITY ? 0.f : wl[q][hh] * exp_acc(wm[q][hh] - mx);
-    pt[sp].m[hh] = mx;
-    pt[sp].l[hh] = ls;
-  }
-}
-
-// The second pass of a split: the global (max, sum) of (token t, KV head g) from its S splits' pairs
-// in split order, the probabilities bf16(exp(s - M) * (1 / L)) of the split's positions (HF rounds
-// them to bf16), and their product with V: AttnPart::acc of this split.
-__global__ void __launch_bounds__(kSplitWaves * 64) attention_pv(const Tok* __restrict__ tok, int L, Cache c,
-                                                                 AttnPart* __restrict__ part,
-                                                                 const float* __restrict__ scores, int cap) {
-  __shared__ float wacc[kSplitWaves][2][kD];
-  const int t = blockIdx.x, g = blockIdx.y, sp = blockIdx.z, S = gridDim.z;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63, slot = lane >> 4, t16 = lane & 15;
-  const Tok tk = tok[t];
-  if (!tk.valid) return;  // attention_split wrote the zeros
-  const int C = tk.pos + 1;
-  const int chunk = (C + S - 1) / S;
-  const int pb = min(C, sp * chunk), pe = min(C, pb + chunk);
-  const uint16_t* vc = c.v + cache_base(c, tk, L, g);
-  // lane (slot, t16) of wave w takes dims 8*t16..+7 of position p0 + 16r + 4w + slot in round r;
-  // positions outside [pb, pe) load row 0 and are masked
-  u32x4 vx[kSplitRounds];
-  auto issue = [&](int p0) {
-#pragma unroll
-    for (int r = 0; r < kSplitRounds; r++) {
-      const int p = p0 + 16 * r + 4 * w + slot;
-      vx[r] = ld16(vc + (size_t)(p < pe ? p : 0) * kD + 8 * t16);
-    }
-  };
-  issue(pb);
-  AttnPart* pt = part + ((size_t)t * kNKV + g) * S;
-  float M[2], inv[2];
-#pragma unroll
-  for (int hh = 0; hh < 2; hh++) {
-    float mx = -INFINITY;
-    for (int q = 0; q < S; q++) mx = fmaxf(mx, pt[q].m[hh]);
-    float ls = 0.f;
-    for (int q = 0; q < S; q++) {
-      const float mq = pt[q].m[hh];
-      ls += mq == -INFINITY ? 0.f : pt[q].l[hh] * exp_acc(mq - mx);
-    }
-    M[hh] = mx;
-    inv[hh] = __fdiv_rn(1.0f, ls);
-  }
-  const float* sc_in = scores + ((size_t)t * kNQ + 2 * g) * cap;
-  float acc[2][8];
-#pragma unroll
-  for (int hh = 0; hh < 2; hh++)
-#pragma unroll
-    for (int i = 0; i < 8; i++) acc[hh][i] = 0.f;
-  for (int p0 = pb; p0 < pe; p0 += 16 * kSplitRounds) {
-    if (p0 != pb) issue(p0);
-#pragma unroll
-    for (int r = 0; r < kSplitRounds; r++) {
-      const int p = p0 + 16 * r + 4 * w + slot;
-      const u32x4 vr = vx[r];
-      const float vf[8] = {lo_bf16(vr.x), hi_bf16(vr.x), lo_bf16(vr.y), hi_bf16(vr.y),
-                           lo_bf16(vr.z), hi_bf16(vr.z), lo_bf16(vr.w), hi_bf16(vr.w)};
-#pragma unroll
-      for (int hh = 0; hh < 2; hh++) {
-        const float pr = p < pe ? bf16r(exp_acc(sc_in[(size_t)hh * cap + p] - M[hh]) * inv[hh]) : 0.f;
-        // a masked position (it loaded cache row 0, which the caller may not have written) leaves the
-        // sum untouched, so that a NaN there cannot enter it through 0 * NaN
-#pragma unroll
-        for (int i = 0; i < 8; i++) acc[hh][i] = p < pe ? __builtin_fmaf(pr, vf[i], acc[hh][i]) : acc[hh][i];
-      }
-    }
-  }
-  // the wave's four rows summed; lanes 0..15 hold dims 8*t16..+7
-#pragma unroll
-  for (int hh = 0; hh < 2; hh++) {
-#pragma unroll
-    for (int i = 0; i < 8; i++) acc[hh][i] = rows_sum4(acc[hh][i]);
-    if (lane < 16) {
-#pragma unroll
-      for (int i = 0; i < 8; i++) wacc[w][hh][8 * t16 + i] = acc[hh][i];
-    }
-  }
-  __syncthreads();
-  // this split's partial: the waves' in wave order
-  {
-    const int hh = threadIdx.x >> 7, d = threadIdx.x & 127;  // 256 threads: both heads' dims
-    float a = 0.f;
-#pragma unroll
-    for (int q = 0; q < kSplitWaves; q++) a += wacc[q][hh][d];
-    pt[sp].acc[hh][d] = a;
-  }
-}
-
-// The attention output of (token t, KV head g): its S partials added in split order.  256 threads:
-// thread i takes head 2g + i / 128, dim i % 128.
-__global__ void __launch_bounds__(256) attention_merge(const Tok* __restrict__ tok, int S,
-                                                       const AttnPart* __restrict__ part, uint16_t* __restrict__ out) {
-  const int t = blockIdx.x, g = blockIdx.y;
-  if (!tok[t].valid) return;  // attention_split wrote the zeros
-  const AttnPart* pt = part + ((size_t)t * kNKV + g) * S;
-  uint16_t* dst = out + (size_t)t * kQS + 2 * g * kD;
-  const int hh = threadIdx.x >> 7, d = threadIdx.x & 127;
-  float y = 0.f;
-  for (int q = 0; q < S; q++) y += pt[q].acc[hh][d];
-  dst[threadIdx.x] = (uint16_t)f32_to_bf16(y);
-}
-
 // ---------------------------------------------------------------- self-test
 
 // C[16][16] = A[16][32] . B[16][32]^T through one MFMA with the operand
@@ -2010,8 +1871,8 @@ size_t part_floats(int T, int N, int K) { return (size_t)plan_gemm(T, N, K).kspl
 
 int split_chunks(int max_context) { return (max_context + kSplitChunk - 1) / kSplitChunk; }
 
-// The context-split attention (three launches, each token's context over workgroups of 64
-// positions) for few tokens over a longer context; the row kernel (one launch) for few tokens over
+// The context-split attention (three launches, each token's context over workgroups of
+// kSplitChunk positions) for a batched step and for few tokens over a longer context; the row kernel (one launch) for few tokens over
 // a short one.  Qwen3-0.6B prefills, split against rows, same box: from position 0, 1 token 1.31 /
 // 1.21 ms and 31 tokens 1.45 / 1.35; from 96, 1.41 / 1.39; from 192, 1.46 / 1.56; from 500, 1.45 /
 // 2.14.  Its work grows with tokens x context, attention_mfma's with the context alone (a 64-token
@@ -2020,10 +1881,12 @@ int split_chunks(int max_context) { return (max_context + kSplitChunk - 1) / kSp
 // tokens after 600 positions 1.55 / 1.62 ms; 2 after 1500 1.61 / 1.64, 8 after 1500 1.83 / 1.68;
 // 1 after 4000 2.01 / 2.07, 2 after 4000 2.12 / 2.08; 1 after 7000 2.60 / 2.38; 31 after 7000
 // 17.96 / 2.42).  A batched decode step (one token per sequence, whose tiles hold several
-// sequences and would fall back to the row kernel) keeps the split form.
+// sequences and would fall back to the row kernel) takes the split form at any batch: 48 sequences of
+// 100..1000 positions ran attention_mfma over no tile and then the row kernel, 86 us per layer
+// against 35.
 constexpr int kSplitWork = 6144;
 bool split_attention(int T, int max_context, bool one_per_seq) {
-  return T < kSplitBelow && max_context > kSplitContext && (one_per_seq || (long long)T * max_context < kSplitWork);
+  return max_context > kSplitContext && (one_per_seq || (T < kSplitBelow && (long long)T * max_context < kSplitWork));
 }
 
 // attention_mfma pays off from about 320 tokens or 256 positions of context (below that the row
@@ -2032,7 +1895,8 @@ bool split_attention(int T, int max_context, bool one_per_seq) {
 // 3.67, 768 tokens 5.85 / 4.45; with its keys in chunks (below), after 400 positions: 32 tokens
 // 2.01 / 1.78, 256 tokens 3.57 / 2.45; after 950: 64 tokens 3.06 / 1.99.
 bool mfma_attention(int T, int max_context, bool one_per_seq) {
-  return !split_attention(T, max_context, one_per_seq) && (T >= kMfmaAttnTokens || max_context >= kMfmaAttnContext);
+  return !one_per_seq && !split_attention(T, max_context, false) &&
+         (T >= kMfmaAttnTokens || max_context >= kMfmaAttnContext);
 }
 
 // attention_mfma's keys in chunks of ck blocks (nch > 1: the split passes) when its tile pairs would
@@ -2062,16 +1926,16 @@ AttnSplit attn_mfma_split(int T, int max_context) {
 }
 
 struct Layout {
-  size_t tok, erow, keys, x, n, q, att, m, qkv, apart, part, scores, ml, pv, redo, mml, mpart, total;
+  size_t tok, erow, keys, x, n, q, att, m, qkv, part, scores, ml, pv, redo, mml, mpart, total;
 };
 
 constexpr int kLmTiles(int V) { return V / 64; }
 
 // The decode step of few sequences (one token each) takes the fused path.
-bool fused_decode(int T, int max_context) { return T <= 16 && max_context <= kFusedCtx; }
+bool fused_decode(int T) { return T <= 16; }
 
 template <class M>
-Layout layout(int T, int R, int max_context, bool one_per_seq = false) {
+Layout layout(int T, int R, int max_context, bool one_per_seq) {
   using Dm = Dims<M>;
   auto al = [](size_t b) { return (b + 255) & ~(size_t)255; };
   Layout l{};
@@ -2088,10 +1952,14 @@ Layout layout(int T, int R, int max_context, bool one_per_seq = false) {
   take(l.q, (size_t)T * kQS * 2);
   take(l.att, (size_t)T * kQS * 2);
   take(l.m, (size_t)T * Dm::I * 2);
-  if (one_per_seq && fused_decode(T, max_context)) {
+  if (split_attention(T, max_context, one_per_seq) || (one_per_seq && fused_decode(T))) {
+    const int nch = split_chunks(max_context);
+    take(l.scores, (size_t)T * kNQ * nch * kSplitChunk * 4);
+    take(l.ml, (size_t)T * kNQ * nch * 8);
+    take(l.pv, (size_t)T * nch * kQS * 4);
+  }
+  if (one_per_seq && fused_decode(T)) {
     take(l.qkv, (size_t)T * kNQKV * 2);
-    take(l.apart, (size_t)T * kNKV * attn_splits(T) * sizeof(AttnPart));
-    take(l.scores, (size_t)T * kNQ * max_context * 4);
     l.total = off;
     return l;
   }
@@ -2100,17 +1968,9 @@ Layout layout(int T, int R, int max_context, bool one_per_seq = false) {
   pf = std::max(pf, part_floats(T, 2 * Dm::I, Dm::H));
   pf = std::max(pf, part_floats(T, Dm::H, Dm::I));
   take(l.part, pf * 4);
-  // the buffers of every attention form the forward may pick for these sizes (one token per
-  // sequence or not: the workspace size query does not say)
-  if (split_attention(T, max_context, true)) {
-    const int nch = split_chunks(max_context);
-    take(l.scores, (size_t)T * kNQ * nch * kSplitChunk * 4);
-    take(l.ml, (size_t)T * kNQ * nch * 8);
-    take(l.pv, (size_t)T * nch * kQS * 4);
-  }
   take(l.redo, (size_t)((T + kQT - 1) / kQT) * 4);
   const AttnSplit sp = attn_mfma_split(T, max_context);
-  if (mfma_attention(T, max_context, false) && sp.nch > 1) {  // attention_mfma's chunks: (max, sum), partials
+  if (mfma_attention(T, max_context, one_per_seq) && sp.nch > 1) {  // attention_mfma's chunks: (max, sum), partials
     const size_t rows = (size_t)((T + kQT - 1) / kQT) * kNQ * sp.nch * kQT;
     take(l.mml, rows * sizeof(float2));
     take(l.mpart, rows * kD * 4);
@@ -2201,6 +2061,30 @@ void launch_rows(int tiles, const uint16_t* X, const uint16_t* nw, float eps, in
   }
 }
 
+// The context-split attention of one layer: RAW from the q/k/v projection's output, else from
+// finished q rows.
+struct AttnChunks {
+  int nch;
+  float* scores;
+  float2* ml;
+  float* pvp;
+};
+AttnChunks attn_chunks(const Args& a, const Layout& l) {
+  return {split_chunks(a.max_context), reinterpret_cast<float*>(a.ws + l.scores),
+          reinterpret_cast<float2*>(a.ws + l.ml), reinterpret_cast<float*>(a.ws + l.pv)};
+}
+
+template <bool RAW>
+void launch_attn_chunks(const Args& a, const AttnChunks& ac, const uint16_t* src, const Tok* tok, int L,
+                        const LDGLayerWeights& w, float eps, uint16_t* out, hipStream_t s) {
+  const dim3 grid(ac.nch, kNKV, a.T);
+  hipLaunchKernelGGL(attn_chunk_scores<RAW>, grid, dim3(256), 0, s, src, tok, L,
+                     static_cast<const uint16_t*>(w.q_norm_weight), static_cast<const uint16_t*>(w.k_norm_weight),
+                     a.cos_t, a.sin_t, a.cache, eps, a.attn_scale, ac.nch, ac.scores, ac.ml);
+  hipLaunchKernelGGL(attn_chunk_pv, grid, dim3(256), 0, s, tok, L, a.cache, ac.nch, ac.scores, ac.ml, ac.pvp);
+  hipLaunchKernelGGL(attn_chunk_merge, dim3(a.T, kNQ), dim3(256), 0, s, tok, ac.nch, ac.pvp, out);
+}
+
 template <class M>
 int forward_fused(const Args& a, hipStream_t s) {
   using Dm = Dims<M>;
@@ -2220,9 +2104,7 @@ int forward_fused(const Args& a, hipStream_t s) {
   static_assert(Dm::H == 1024 || Dm::H == 2048, "K splits of the hidden size");
   static_assert(Dm::I == 3072 || Dm::I == 6144, "K splits of the MLP size");
   static_assert(kQS == 2048 && Dm::H <= kMaxRowsH, "K splits of the attention output");
-  AttnPart* apart = reinterpret_cast<AttnPart*>(a.ws + l.apart);
-  float* ascores = reinterpret_cast<float*>(a.ws + l.scores);
-  const int nsplit = attn_splits(T);
+  const AttnChunks ac = attn_chunks(a, l);
   hipLaunchKernelGGL(prep_tokens, dim3((std::max(T, R) + 255) / 256), dim3(256), 0, s, a.tokens, a.seqs, a.pos, T,
                      a.emit, R, a.num_seqs, a.max_context, Dm::V, tok, erow);
   hipLaunchKernelGGL(embed_rows, dim3(T), dim3(256), 0, s, a.embed, tok, Dm::H, X);
@@ -2230,12 +2112,7 @@ int forward_fused(const Args& a, hipStream_t s) {
     const LDGLayerWeights& w = a.layers[L];
     const Seg qkv{{u16(w.q_proj_weight), u16(w.k_proj_weight), u16(w.v_proj_weight)}, {kQS, kNKV * kD, kNKV * kD}};
     launch_rows<kEpiStore, true, 16>(kNQKV / 16, X, u16(w.input_layernorm_weight), eps, T, Dm::H, qkv, QKV, kNQKV, s);
-    hipLaunchKernelGGL(attention_split, dim3(T, kNKV, nsplit), dim3(kSplitWaves * 64), 0, s, QKV, tok, L,
-                       u16(w.q_norm_weight), u16(w.k_norm_weight), a.cos_t, a.sin_t, a.cache, eps, a.attn_scale,
-                       apart, ascores, a.max_context, ATT);
-    hipLaunchKernelGGL(attention_pv, dim3(T, kNKV, nsplit), dim3(kSplitWaves * 64), 0, s, tok, L, a.cache, apart,
-                       ascores, a.max_context);
-    hipLaunchKernelGGL(attention_merge, dim3(T, kNKV), dim3(256), 0, s, tok, nsplit, apart, ATT);
+    launch_attn_chunks<true>(a, ac, QKV, tok, L, w, eps, ATT, s);
     const Seg o{{u16(w.o_proj_weight), nullptr, nullptr}, {Dm::H, 0, 0}};
     launch_rows<kEpiResidual, false, 16, true>(Dm::H / 8, ATT, nullptr, eps, T, kQS, o, X, Dm::H, s);
     const Seg gu{{u16(w.gate_proj_weight), u16(w.up_proj_weight), nullptr}, {Dm::I, Dm::I, 0}};
@@ -2253,8 +2130,8 @@ template <class M>
 int forward(const Args& a, hipStream_t s) {
   using Dm = Dims<M>;
   const int T = a.T, R = a.R;
-  if (a.one_per_seq && fused_decode(T, a.max_context)) return forward_fused<M>(a, s);
-  const Layout l = layout<M>(T, R, a.max_context);
+  if (a.one_per_seq && fused_decode(T)) return forward_fused<M>(a, s);
+  const Layout l = layout<M>(T, R, a.max_context, a.one_per_seq);
   Tok* tok = reinterpret_cast<Tok*>(a.ws + l.tok);
   int* erow = reinterpret_cast<int*>(a.ws + l.erow);
   auto* keys = reinterpret_cast<unsigned long long*>(a.ws + l.keys);
@@ -2266,7 +2143,6 @@ int forward(const Args& a, hipStream_t s) {
   float* part = reinterpret_cast<float*>(a.ws + l.part);
   const float eps = 1e-6f;
   const bool split = split_attention(T, a.max_context, a.one_per_seq);
-  const int nch = split ? split_chunks(a.max_context) : 0;
   const bool mfma_attn = mfma_attention(T, a.max_context, a.one_per_seq);
   const AttnSplit asp = attn_mfma_split(T, a.max_context);
   auto blocks = [](size_t n) { return dim3((unsigned)((n + 255) / 256)); };
@@ -2285,13 +2161,7 @@ int forward(const Args& a, hipStream_t s) {
     launch_gemm(N, T, Dm::H, qkv, kNQKV, part, s, &ks, kEpiQkv, &qo);
     if (ks) hipLaunchKernelGGL(qkv_finish, dim3(T, kNQ + 2 * kNKV), dim3(64), 0, s, part, ks, T, qo);
     if (split) {
-      float* scores = reinterpret_cast<float*>(a.ws + l.scores);
-      float2* ml = reinterpret_cast<float2*>(a.ws + l.ml);
-      float* pvp = reinterpret_cast<float*>(a.ws + l.pv);
-      hipLaunchKernelGGL(attn_split_scores, dim3(T, kNKV, nch), dim3(256), 0, s, Qb, tok, L, a.cache, a.attn_scale,
-                         nch, scores, ml);
-      hipLaunchKernelGGL(attn_split_pv, dim3(T, kNKV, nch), dim3(256), 0, s, tok, L, a.cache, nch, scores, ml, pvp);
-      hipLaunchKernelGGL(attn_split_merge, dim3(T, kQS / 256), dim3(256), 0, s, tok, nch, pvp, ATT);
+      launch_attn_chunks<false>(a, attn_chunks(a, l), Qb, tok, L, w, eps, ATT, s);
     } else {
       if (mfma_attn) {
         // tiles of one sequence's consecutive tokens on MFMA; any other tile row by row
@@ -2345,8 +2215,8 @@ extern "C" {
 
 size_t qmk_forward_workspace_bytes(int model, int num_tokens, int num_emit, int max_context) {
   if (num_tokens < 1 || num_emit < 1 || num_emit > batch::kMaxEmit || max_context < 1) return 0;
-  if (model == QMK_MODEL_QWEN3_1_7B) return batch::layout<Qwen3_1_7B>(num_tokens, num_emit, max_context).total;
-  if (model == QMK_MODEL_QWEN3_0_6B) return batch::layout<Qwen3_0_6B>(num_tokens, num_emit, max_context).total;
+  if (model == QMK_MODEL_QWEN3_1_7B) return batch::layout<Qwen3_1_7B>(num_tokens, num_emit, max_context, false).total;
+  if (model == QMK_MODEL_QWEN3_0_6B) return batch::layout<Qwen3_0_6B>(num_tokens, num_emit, max_context, false).total;
   return 0;
 }
 
