@@ -22,7 +22,7 @@
 //                         is not split)
 //   gemm_tiled(down)   -> residual_norm (residual add, next layer's input RMSNorm
 //                                        or the final norm)
-// then lm_head_gemm over the emitted rows (bf16 logits, per-tile argmax keys)
+// then the LM head over the emitted rows (bf16 logits, argmax keys)
 // -> keys_reduce (per-row argmax).
 
 #include <hip/hip_runtime.h>
@@ -322,6 +322,17 @@ constexpr int kTM = 128, kTK = 64;
 // is the same for every lane of the wave)
 __device__ __forceinline__ void dma16(const void* src, void* lds) {
   __builtin_amdgcn_global_load_lds(as_global<void>(src), (__attribute__((address_space(3))) void*)lds, 16, 0, 0);
+}
+
+// Barrier of a ring of DMA stages: at most N of this wave's requests are still in flight, its LDS
+// reads so far have returned, and every wave of the workgroup has come this far.  (__syncthreads
+// would do for the order, but the count of requests left in flight has to be exact.)
+template <int N>
+__device__ __forceinline__ void ring_barrier() {
+  wait_vmcnt_upto<N>();
+  __builtin_amdgcn_s_waitcnt(kWaitLgkm0);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
 }
 
 template <int TN, int EPI = kEpiPart>
@@ -1328,86 +1339,128 @@ __global__ void __launch_bounds__(256) attn_chunk_merge(const Tok* __restrict__ 
 
 // ---------------------------------------------------------------- LM head
 //
-// The LM head runs as lm_head_gemm (the GEMM above over the full K, one wave
-// per 16-row x 64-column tile) whose epilogue rounds each logit to bf16,
-// optionally writes its fp32 copy, and keeps, per row and tile, the largest
-// key (orderable bf16 logit << 32 | ~index): the first index of the maximum,
-// HF's greedy argmax.  keys_reduce then takes each row's largest key over the
-// tiles; no atomics, so the result is independent of scheduling.
+// The LM head kernels round each logit to bf16, optionally write its fp32 copy, and keep, per row
+// and wave or workgroup, the largest key (orderable bf16 logit << 32 | ~index): the first index of
+// the maximum, HF's greedy argmax.  keys_reduce then takes each row's largest key; no atomics, so
+// the result is independent of scheduling.
 
 __device__ __forceinline__ unsigned long long key_max(unsigned long long a, unsigned long long b) { return a > b ? a : b; }
 
-__global__ void __launch_bounds__(256) lm_head_gemm(const uint16_t* __restrict__ X, const int* __restrict__ rows,
-                                                    int R, const uint16_t* __restrict__ W, int K, int V,
-                                                    unsigned long long* __restrict__ keys_part,
-                                                    float* __restrict__ logits) {
-  constexpr int NB = 4;
-  const int nblk = gridDim.x;
-  const int b = blockIdx.x;
-  const int lb = (nblk % kGroups == 0) ? (b % kGroups) * (nblk / kGroups) + b / kGroups : b;
-  const int wave = lb * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  const int mtiles = (R + 15) / 16, ntiles = V / (16 * NB);
-  const int mt = wave % mtiles, nt = wave / mtiles;
-  if (nt >= ntiles) return;
-  const int kq = 8 * (lane >> 4);
-  const int xr = max(rows[min(mt * 16 + (lane & 15), R - 1)], 0);
-  const uint16_t* xa = X + (size_t)xr * K + kq;
-  const uint16_t* wb[NB];
+// lm_head_tiled: the LM head of more than 16 emitted rows.  A persistent grid of two workgroups per
+// CU; a workgroup of 4 waves takes the 64-row vocabulary tiles blockIdx.x, + gridDim.x, ... against
+// 16 MT emitted rows (blockIdx.y the group of rows), walking them as one sequence of 64-K steps
+// through a ring of four LDS stages: both operands go from global memory straight into LDS three
+// steps ahead, across tile boundaries, so every weight row is read once per group of rows, in whole
+// 128-byte lines, and 48 KB of weights per CU are in flight.  Wave w takes columns 16w..+15 of the
+// tile.  Stage rows are swizzled as gemm_tiled's.  Each lane keeps its rows' best (logit, index)
+// over its tiles (its columns come in increasing order, so the first of equal logits stays).
+// HBM bounds it (311 MB of Qwen3-0.6B weights, plus the fp32 logits).  48 rows: one wave per 16-row
+// tile, operands straight from global memory and weights re-read per 16 rows, 187 us -> 76.
+constexpr int kLmTileWGs = 512, kLmStages = 4;
+
+template <int MT, int K>
+__global__ void __launch_bounds__(256, 2) lm_head_tiled(const uint16_t* __restrict__ X, const int* __restrict__ rows,
+                                                        int R, const uint16_t* __restrict__ W, int V,
+                                                        unsigned long long* __restrict__ keys_part,
+                                                        float* __restrict__ logits) {
+  constexpr int AR = MT <= 2 ? 32 : 64;               // emitted rows staged (clamped past R)
+  constexpr int NA = AR / 32, NB = 2, KS = K / 64;    // 1 KB DMA blocks (8 rows) per wave and stage
+  constexpr int StB = (AR + 64) * 128;
+  static_assert(MT <= 4 && 16 * MT <= AR && K % 64 == 0, "row tiles");
+  static_assert(kLmStages * StB >= 4 * 16 * MT * 8, "the keys' exchange fits the stages");
+  __shared__ __align__(1024) unsigned char sm[kLmStages * StB];
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int l16 = lane & 15, lq = lane >> 4;
+  const int r0 = blockIdx.y * 16 * MT, ntiles = V / 64, step0 = gridDim.x;
+  const int mine = (int)blockIdx.x < ntiles ? (ntiles - (int)blockIdx.x + step0 - 1) / step0 : 0;
+  const int nsteps = mine * KS;
+  const uint16_t* asrc[NA];
+  const uint16_t* bsrc[NB];
 #pragma unroll
-  for (int j = 0; j < NB; j++) wb[j] = W + (size_t)(nt * 16 * NB + 16 * j + (lane & 15)) * K + kq;
-  f32x4 acc[NB];
-#pragma unroll
-  for (int j = 0; j < NB; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 a0 = ld_bf16x8(xa), a1 = ld_bf16x8(xa + 32), b0[NB], b1[NB];
-#pragma unroll
-  for (int j = 0; j < NB; j++) {
-    b0[j] = ld_bf16x8_stream(wb[j]);
-    b1[j] = ld_bf16x8_stream(wb[j] + 32);
+  for (int q = 0; q < NA; q++) {
+    const int row = 8 * (NA * w + q) + (lane >> 3), c = (lane & 7) ^ (row & 7);
+    asrc[q] = X + (size_t)max(rows[min(r0 + row, R - 1)], 0) * K + 8 * c;
   }
-  for (int k = 0; k < K; k += 64) {
-    bf16x8 na0, na1, nb0[NB], nb1[NB];
-    const bool more = k + 64 < K;
-    if (more) {
-      na0 = ld_bf16x8(xa + k + 64);
-      na1 = ld_bf16x8(xa + k + 96);
 #pragma unroll
-      for (int j = 0; j < NB; j++) {
-        nb0[j] = ld_bf16x8_stream(wb[j] + k + 64);
-        nb1[j] = ld_bf16x8_stream(wb[j] + k + 96);
+  for (int q = 0; q < NB; q++) {
+    const int row = 8 * (NB * w + q) + (lane >> 3), c = (lane & 7) ^ (row & 7);
+    bsrc[q] = W + ((size_t)blockIdx.x * 64 + row) * K + 8 * c;
+  }
+  // steps past the last are requested too (the last one again, into stages no one reads), so that
+  // the count of requests in flight is the same at every step
+  auto issue = [&](int step) {
+    const int sc = min(step, nsteps - 1), k = (sc % KS) * 64;
+    const size_t tb = (size_t)(sc / KS) * step0 * 64 * K + k;
+    unsigned char* base = sm + (step % kLmStages) * StB;
+#pragma unroll
+    for (int q = 0; q < NA; q++) dma16(asrc[q] + k, base + 1024 * (NA * w + q));
+#pragma unroll
+    for (int q = 0; q < NB; q++) dma16(bsrc[q] + tb, base + AR * 128 + 1024 * (NB * w + q));
+  };
+  f32x4 acc[MT];
+  uint32_t bval[MT][4], bidx[MT][4];
+#pragma unroll
+  for (int i = 0; i < MT; i++) {
+    acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 4; r++) bval[i][r] = 0, bidx[i][r] = 0xffffffffu;
+  }
+  if (nsteps > 0) {
+#pragma unroll
+    for (int u = 0; u < kLmStages - 1; u++) issue(u);
+  }
+  for (int st = 0; st < nsteps; st++) {
+    // step st has landed (two younger steps may be in flight) in every wave, and its predecessor's
+    // stage is read
+    ring_barrier<(kLmStages - 2) * (NA + NB)>();
+    issue(st + kLmStages - 1);
+    const unsigned char* base = sm + (st % kLmStages) * StB;
+#pragma unroll
+    for (int kc = 0; kc < 8; kc += 4) {
+      const int brow = 16 * w + l16;
+      const bf16x8 b = *reinterpret_cast<const bf16x8*>(base + AR * 128 + brow * 128 + 16 * ((kc + lq) ^ (brow & 7)));
+#pragma unroll
+      for (int i = 0; i < MT; i++) {
+        const int row = 16 * i + l16;
+        const bf16x8 a = *reinterpret_cast<const bf16x8*>(base + row * 128 + 16 * ((kc + lq) ^ (row & 7)));
+        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[i], 0, 0, 0);
       }
     }
+    if (st % KS == KS - 1) {  // the tile is complete
+      const uint32_t n = (uint32_t)(((st / KS) * step0 + blockIdx.x) * 64 + 16 * w + l16);
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0, b0[j], acc[j], 0, 0, 0);
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1, b1[j], acc[j], 0, 0, 0);
-    }
-    if (more) {
-      a0 = na0;
-      a1 = na1;
+      for (int i = 0; i < MT; i++) {
 #pragma unroll
-      for (int j = 0; j < NB; j++) {
-        b0[j] = nb0[j];
-        b1[j] = nb1[j];
+        for (int r = 0; r < 4; r++) {
+          const int t = r0 + 16 * i + 4 * lq + r;
+          const uint32_t hb = f32_to_bf16(acc[i][r]), o = orderable16(hb);
+          if (logits && t < R) logits[(size_t)t * V + n] = bf16_to_f32(hb);
+          if (o > bval[i][r] || bidx[i][r] == 0xffffffffu) {
+            bval[i][r] = o;
+            bidx[i][r] = n;
+          }
+        }
+        acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
       }
     }
   }
+  // each row's best over the 16 lanes that hold its columns, then over the waves
+  ring_barrier<0>();  // the last requests have landed, the last stage is read
+  auto red = reinterpret_cast<unsigned long long(*)[16 * MT]>(sm);
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
-    const int t = mt * 16 + 4 * (lane >> 4) + i;
-    unsigned long long best = 0;
+  for (int i = 0; i < MT; i++)
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-      const int n = nt * 16 * NB + 16 * j + (lane & 15);
-      const uint32_t hb = f32_to_bf16(acc[j][i]);
-      if (logits && t < R) logits[(size_t)t * V + n] = bf16_to_f32(hb);
-      best = key_max(best, ((unsigned long long)orderable16(hb) << 32) | (unsigned long long)(0xffffffffu - (uint32_t)n));
+    for (int r = 0; r < 4; r++) {
+      unsigned long long best = ((unsigned long long)bval[i][r] << 32) | (unsigned long long)(0xffffffffu - bidx[i][r]);
+#pragma unroll
+      for (int o = 1; o < 16; o <<= 1) best = key_max(best, __shfl_xor(best, o));
+      if (l16 == 0) red[w][16 * i + 4 * lq + r] = best;
     }
-    // max over the 16 lanes that hold row t
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) best = key_max(best, __shfl_xor(best, o));
-    if ((lane & 15) == 0 && t < R) keys_part[(size_t)t * ntiles + nt] = best;
-  }
+  __syncthreads();
+  const int t = r0 + (int)threadIdx.x;
+  if ((int)threadIdx.x < 16 * MT && t < R)
+    keys_part[(size_t)t * gridDim.x + blockIdx.x] =
+        key_max(key_max(red[0][threadIdx.x], red[1][threadIdx.x]), key_max(red[2][threadIdx.x], red[3][threadIdx.x]));
 }
 
 // LM head for at most 16 emitted rows, streamed by a persistent grid: 256
@@ -1929,8 +1982,6 @@ struct Layout {
   size_t tok, erow, keys, x, n, q, att, m, qkv, part, scores, ml, pv, redo, mml, mpart, total;
 };
 
-constexpr int kLmTiles(int V) { return V / 64; }
-
 // The decode step of few sequences (one token each) takes the fused path.
 bool fused_decode(int T) { return T <= 16; }
 
@@ -1946,7 +1997,8 @@ Layout layout(int T, int R, int max_context, bool one_per_seq) {
   };
   take(l.tok, (size_t)T * sizeof(Tok));
   take(l.erow, (size_t)R * 4);
-  take(l.keys, (size_t)R * std::max(kLmTiles(Dm::V), kLmBlocks * kLmWaves) * 8);
+  take(l.keys, (size_t)R * kLmBlocks * kLmWaves * 8);
+  static_assert(kLmBlocks * kLmWaves >= kLmTileWGs && Dm::V % 64 == 0, "LM head keys and tiles");
   take(l.x, (size_t)T * Dm::H * 2);
   take(l.n, (size_t)T * Dm::H * 2);
   take(l.q, (size_t)T * kQS * 2);
@@ -1993,8 +2045,8 @@ struct Args {
   char* ws;
 };
 
-// LM head + argmax of R emitted rows: the streamed persistent form for R <= 16,
-// the tiled GEMM above that.
+// LM head + argmax of R emitted rows: whole vocabulary rows for R <= 4, the streamed MFMA form up to
+// 16, tiles through LDS above that.
 template <class M>
 void launch_lm_head(const uint16_t* N, const int* erow, int R, const uint16_t* W, unsigned long long* keys,
                     float* logits, const Tok* tok, int* out, hipStream_t s) {
@@ -2017,10 +2069,14 @@ void launch_lm_head(const uint16_t* N, const int* erow, int R, const uint16_t* W
     hipLaunchKernelGGL(keys_reduce, dim3(R), dim3(256), 0, s, keys, kLmBlocks * kLmWaves, erow, tok, out);
     return;
   }
-  const int lm_waves = ((R + 15) / 16) * kLmTiles(Dm::V);
-  hipLaunchKernelGGL(lm_head_gemm, dim3((lm_waves + 3) / 4), dim3(256), 0, s, N, erow, R, W, Dm::H, Dm::V, keys,
-                     logits);
-  hipLaunchKernelGGL(keys_reduce, dim3(R), dim3(256), 0, s, keys, kLmTiles(Dm::V), erow, tok, out);
+  // two workgroups per CU, shared by the groups of up to 64 rows
+  const int groups = (R + 63) / 64;
+  const dim3 grid(kLmTileWGs / groups, groups);
+  if (R <= 32)
+    hipLaunchKernelGGL((lm_head_tiled<2, Dm::H>), grid, dim3(256), 0, s, N, erow, R, W, Dm::V, keys, logits);
+  else
+    hipLaunchKernelGGL((lm_head_tiled<4, Dm::H>), grid, dim3(256), 0, s, N, erow, R, W, Dm::V, keys, logits);
+  hipLaunchKernelGGL(keys_reduce, dim3(R), dim3(256), 0, s, keys, (int)grid.x, erow, tok, out);
 }
 
 // gemm_rows over `tiles` 16-column tiles (NB = 1), NW waves each taking

@@ -51,3 +51,45 @@ def test_decode_batch_attention_chunk_edges(shape, exact06, weights_gpu, c0s):
     """attn_chunk_*: contexts ending at, before and after a chunk's edge, a token in a chunk of its own,
     more than 64 chunks (two rounds of pairs), from raw projections (up to 16 sequences) and finished q."""
     _decode_steps(shape, exact06, weights_gpu, c0s, layers=2, max_seq=(max(c0s) + 2 + 63) // 64 * 64)
+
+
+@pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 200])
+def test_lm_head_row_groups(weights_gpu, rows):
+    """lm_head_tiled (more than 16 emitted rows, groups of 32 or 64): logits within one bf16 ulp of the
+    same rows emitted four at a time (lm_head_rows, another order of the same fp32 sums of bf16 products:
+    both round to a neighbour of the exact sum), and each token the first index of its own maximum.  One
+    emitted row is outside the batch: it emits -1."""
+    from qwen_megakernel.model import _Forward, _ops
+
+    V, T = 151936, 200
+    fwd = _Forward(_ops(), weights_gpu, 1)
+    k = torch.zeros(1, 1, 8, 256, 128, dtype=torch.bfloat16, device="cuda")
+    v = torch.zeros_like(k)
+
+    def i32(x):
+        return torch.tensor(x, dtype=torch.int32, device="cuda")
+
+    g = torch.Generator().manual_seed(rows)
+    ids = i32(torch.randint(0, V, (T,), generator=g).tolist())
+    seqs, pos = i32([0] * T), torch.arange(T, dtype=torch.int32, device="cuda")
+
+    def emit(which):
+        out = torch.empty(len(which), dtype=torch.int32, device="cuda")
+        logits = torch.empty(len(which), V, dtype=torch.float32, device="cuda")
+        fwd(ids, seqs, pos, i32(which), out, logits, k, v, T)
+        return out.cpu(), logits
+
+    which = torch.randperm(T, generator=g)[:rows].tolist()
+    which[rows // 2] = T + 5
+    out, logits = emit(which)
+    assert int(out[rows // 2]) == -1
+    for r0 in range(0, rows, 4):
+        o4, l4 = emit(which[r0:r0 + 4])
+        for r in range(len(o4)):
+            if which[r0 + r] >= T:
+                assert int(o4[r]) == -1
+                continue
+            x, y = logits[r0 + r], l4[r]
+            ulp = torch.exp2(torch.floor(torch.log2(y.abs().clamp_min(1e-3))) - 7)
+            assert ((x - y).abs() <= 1.01 * ulp).all()
+            assert int(out[r0 + r]) == int(torch.argmax(x.cpu()))
