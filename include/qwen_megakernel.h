@@ -363,7 +363,7 @@ size_t qmk_decode_batch_workspace_bytes(int model, int batch, int max_context);
  * next token, logits_out[b][vocab] its logits when not NULL.  Sequence b's
  * cache is the [num_layers][8][max_seq_len][128] block at k_cache + b *
  * seq_stride.  The same as qmk_forward_tokens with seq_ids = emit_rows =
- * 0..batch-1, but since each sequence has one token, batches of up to 16 run
+ * 0..batch-1, but since each sequence has one token, batches of up to 32 run
  * seven fused launches per layer (RMSNorm in the GEMM prologues, q/k norm +
  * RoPE + K/V append inside attention, residual and SiLU*up in the GEMM
  * epilogues).  Invalid ids or positions emit -1.

@@ -12,7 +12,8 @@
 // The reference prefills one token per step() (qwen_megakernel/model.py:210-211)
 // and decodes one sequence; the batched forward is an addition.
 //
-// Per layer (kernels in launch order):
+// At most kRowsMax tokens take gemm_rows and its fused prologues and epilogues ("few tokens" below).
+// Per layer above that (kernels in launch order):
 //   gemm_tiled(qkv)    -> qkv_finish (split-K sum, q/k RMSNorm + RoPE, K/V append;
 //                         in the GEMM's epilogue when K is not split)
 //   attention          (one kernel per (token, KV head) for many tokens; a
@@ -52,7 +53,7 @@ constexpr int kMaxEmit = 256;
 static_assert(Qwen3_0_6B::D == kD && Qwen3_0_6B::NQ == kNQ && Qwen3_0_6B::NKV == kNKV, "head layout");
 static_assert(Qwen3_1_7B::D == kD && Qwen3_1_7B::NQ == kNQ && Qwen3_1_7B::NKV == kNKV, "head layout");
 
-// Per-token metadata, checked once (prep_tokens).  An invalid token (id outside
+// Per-token metadata, checked once (embed_tokens).  An invalid token (id outside
 // the vocabulary, sequence or position out of range) reads embedding row 0,
 // writes nothing into any cache and emits -1.
 struct Tok {
@@ -106,28 +107,51 @@ __device__ __forceinline__ void block_max2(float (&v)[2], float (*red)[4]) {
 
 // ---------------------------------------------------------------- tokens
 
-__global__ void __launch_bounds__(256) prep_tokens(const int* __restrict__ tokens, const int* __restrict__ seqs,
-                                                   const int* __restrict__ pos, int T, const int* __restrict__ emit,
-                                                   int R, int num_seqs, int max_context, int vocab,
-                                                   Tok* __restrict__ tok, int* __restrict__ erow) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i < T) {
-    const int id = tokens[i], sq = seqs ? seqs[i] : i, p = pos[i];
-    const bool ok = id >= 0 && id < vocab && sq >= 0 && sq < num_seqs && p >= 0 && p < max_context;
-    tok[i] = Tok{ok ? id : 0, ok ? sq : 0, ok ? p : 0, ok ? 1 : 0};
+// One workgroup per token t: its checked record, X[t] = embed[token], and what the first layer's q/k/v
+// projection needs of it: N[t] = RMSNorm(X[t]) (NORM), or the row's sum of squares for gemm_rows,
+// ssq[t][0] (its other partials 0).  Workgroup 0 also checks the emit rows.  (Token records,
+// embedding and norm as three launches took 4.5 us each.)
+template <int H, bool NORM>
+__global__ void __launch_bounds__(256) embed_tokens(const int* __restrict__ tokens, const int* __restrict__ seqs,
+                                                    const int* __restrict__ pos, int T, const int* __restrict__ emit,
+                                                    int R, int num_seqs, int max_context, int vocab,
+                                                    const uint16_t* __restrict__ embed, Tok* __restrict__ tok,
+                                                    int* __restrict__ erow, uint16_t* __restrict__ X,
+                                                    const uint16_t* __restrict__ norm_w, float eps,
+                                                    uint16_t* __restrict__ Nout, float* __restrict__ ssq) {
+  constexpr int J = H / 256, JW = J / 2;  // elements and bf16 pairs per thread
+  typedef unsigned words_t __attribute__((ext_vector_type(JW)));
+  __shared__ float red[4];
+  const int t = blockIdx.x, i0 = J * threadIdx.x;
+  const int id = tokens[t], sq = seqs ? seqs[t] : t, p = pos[t];
+  const bool ok = id >= 0 && id < vocab && sq >= 0 && sq < num_seqs && p >= 0 && p < max_context;
+  if (threadIdx.x == 0) tok[t] = Tok{ok ? id : 0, ok ? sq : 0, ok ? p : 0, ok ? 1 : 0};
+  if (t == 0)
+    for (int i = threadIdx.x; i < R; i += 256) {
+      const int e = emit ? emit[i] : i;
+      erow[i] = (e >= 0 && e < T) ? e : -1;
+    }
+  const words_t xw = *reinterpret_cast<const words_t*>(embed + (size_t)(ok ? id : 0) * H + i0);
+  *reinterpret_cast<words_t*>(X + (size_t)t * H + i0) = xw;
+  float ss = 0.f;
+#pragma unroll
+  for (int e = 0; e < JW; e++) ss += lo_bf16(xw[e]) * lo_bf16(xw[e]) + hi_bf16(xw[e]) * hi_bf16(xw[e]);
+  ss = wave_sum(ss);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = ss;
+  __syncthreads();
+  ss = (red[0] + red[1]) + (red[2] + red[3]);
+  if constexpr (NORM) {
+    const float rstd = rcp_sqrt_torch(__fdiv_rn(ss, (float)H) + eps);
+    const words_t ww = *reinterpret_cast<const words_t*>(norm_w + i0);
+    words_t out;
+#pragma unroll
+    for (int e = 0; e < JW; e++)
+      out[e] = pack_bf16x2(bf16r(lo_bf16(ww[e]) * bf16r(lo_bf16(xw[e]) * rstd)),
+                           bf16r(hi_bf16(ww[e]) * bf16r(hi_bf16(xw[e]) * rstd)));
+    *reinterpret_cast<words_t*>(Nout + (size_t)t * H + i0) = out;
+  } else {
+    for (int i = threadIdx.x; i < H / 8; i += 256) ssq[(size_t)t * (H / 8) + i] = i == 0 ? ss : 0.f;
   }
-  if (i < R) {
-    const int e = emit ? emit[i] : i;
-    erow[i] = (e >= 0 && e < T) ? e : -1;
-  }
-}
-
-// X[t] = embed[token[t]]
-__global__ void __launch_bounds__(256) embed_rows(const uint16_t* __restrict__ embed, const Tok* __restrict__ tok,
-                                                  int H, uint16_t* __restrict__ X) {
-  const int t = blockIdx.x;
-  const uint16_t* e = embed + (size_t)tok[t].token * H;
-  for (int i = threadIdx.x; i < H / 8; i += 256) reinterpret_cast<u32x4*>(X + (size_t)t * H)[i] = ld16(e + 8 * i);
 }
 
 // ---------------------------------------------------------------- GEMM
@@ -1635,25 +1659,35 @@ __global__ void __launch_bounds__(kLmWaves * 64) lm_head_rows(const uint16_t* __
   }
 }
 
-// ---------------------------------------------------------------- decode step, few sequences
+// ---------------------------------------------------------------- few tokens
 //
-// One token per sequence, at most 16 sequences (one MFMA row tile), contexts
-// of any length: seven launches per layer instead of eleven.
+// At most kRowsMax tokens (a batched step, a short prompt): the projections run as gemm_rows, whole K
+// in one workgroup, with the work between them in their prologues and epilogues.  Per layer:
 //
-//   gemm_rows<NORM>(q,k,v)   input RMSNorm in the prologue, bf16 q|k|v out
-//   attn_chunk_scores<RAW>   q/k head norm + RoPE, K/V append, the chunks' scores;
-//   attn_chunk_pv, _merge    probabilities times V per chunk, the chunks' sum
-//   gemm_rows(o)             epilogue: residual add into the hidden rows
-//   gemm_rows<NORM>(g|u)     post-attention RMSNorm in the prologue, SiLU(g)*u out
-//   gemm_rows(down)          epilogue: residual add
+//   gemm_rows<NORM>(q,k,v)   input RMSNorm on the operands, bf16 q|k|v out
+//   attention                one token per sequence: attn_chunk_* straight from q|k|v; else
+//                            qkv_rows_finish (q/k norm + RoPE, K/V append), then any form
+//   gemm_rows(o)             epilogue: residual add into the hidden rows, their squares summed
+//   gemm_rows<NORM>(g|u)     post-attention RMSNorm on the operands, SiLU(g)*u out
+//   gemm_rows(down)          epilogue as o's
 //
-// gemm_rows: one workgroup of 16 waves per 16*NB-column tile; wave w takes
-// K/16 of the K range (the MFMA operand layout above) and the
-// 16 partial tiles are summed in LDS in wave order, so every column is one
-// fp32 sum rounded once, with no partials in memory and no finish kernel.
-
-constexpr int kRowWaves = 16;
-constexpr int kMaxRowsH = 2048;   // largest hidden size a NORM prologue stages in LDS
+// gemm_rows: one workgroup of NW waves per tile of 16 NB output columns (8: HALF, whose MFMA columns
+// 8-15 repeat rows 0-7, loads that the same instruction makes anyway: twice the workgroups for the
+// narrow o and down) and all T rows (MT MFMA row tiles).  Wave w takes K / NW of the K range: its
+// whole weight slice is requested at once, straight from the row-major rows in the MFMA operand
+// layout, behind the small loads (vector memory returns in order), and the waves' partial tiles are
+// summed in LDS in wave order, so every column is one fp32 sum rounded once.
+// RMSNorm needs each row's sum of squares before the product: the kernels that write the hidden rows
+// (embed_tokens, the residual epilogues) leave partial sums per 8 columns (ssq[t][H / 8]), a wave
+// adds each row's, and every wave normalises its own operands in registers, bf16(w * bf16(x *
+// rstd)) as HF; so no workgroup stages whole rows in LDS first.
+// It is bound by latency (dispatch, one round trip for rows and weights, two barriers), not by its
+// bytes: 4-6 us for the 4-13 MB of a Qwen3-0.6B projection.  Against
+// split-K gemm_tiled with finishing kernels (us per forward of 4 layers from position 0): Qwen3-0.6B 8
+// tokens 194 -> 175, 16 202 -> 187, 32 211 -> 203; Qwen3-1.7B 8 tokens 332 -> 279, 32 363 -> 339.
+// Every workgroup of a NORM product normalises all T rows, so above 32 it loses (48 tokens 224 ->
+// 236).
+constexpr int kRowsMax = 32;
 
 enum RowEpi : int { kEpiStore = 0, kEpiResidual = 1, kEpiSiluMul = 2 };
 
@@ -1662,160 +1696,164 @@ enum RowEpi : int { kEpiStore = 0, kEpiResidual = 1, kEpiSiluMul = 2 };
 // columns NC/2..NC-1; otherwise the seg rows in order.
 template <int EPI, int NC>
 __device__ __forceinline__ const uint16_t* tile_row(const Seg& seg, int tile, int col, int K) {
-  if (EPI == kEpiSiluMul) return seg.w[col / (NC / 2)] + (size_t)(tile * (NC / 2) + col % (NC / 2)) * K;
+  if (EPI == kEpiSiluMul) {
+    const uint16_t* base = col < NC / 2 ? seg.w[0] : seg.w[1];
+    return base + (size_t)(tile * (NC / 2) + col % (NC / 2)) * K;
+  }
   return seg_row(seg, tile * NC + col, K);
 }
 
-// Dynamic LDS of gemm_rows: the normalised input rows (NORM), then the NW
-// partial tiles, then the per-wave sums of squares.
-template <int NB, int NW, bool NORM>
-constexpr size_t rows_lds(int T, int K) {
-  return (NORM ? (size_t)((T * K * 2 + 15) / 16 * 16) : 0) + (size_t)NW * 16 * 16 * NB * 4 + (size_t)NW * 16 * 4 + 64;
+// LDS of gemm_rows: the waves' partial tiles of one row tile, and the rows' rstd
+template <int MT, int NC, int NW>
+constexpr size_t rows_lds() {
+  return (size_t)NW * 16 * NC * 4 + 16 * MT * 4;
 }
 
-// HALF: 8 output columns per tile (the MFMA's columns 8-15 repeat rows 0-7,
-// whose loads the same instruction already makes), twice the workgroups of an
-// N / 16 grid for the narrow o and down projections.
-template <int NB, int EPI, bool NORM, int NW, int ITERS, int MAXT, bool HALF = false>
-__global__ void __launch_bounds__(NW * 64) gemm_rows(const uint16_t* __restrict__ X, const uint16_t* __restrict__ norm_w,
-                                                     float eps, int T, int K, Seg seg, uint16_t* __restrict__ Y,
-                                                     int ldy) {
+// (four waves per SIMD: one workgroup of 16 waves or two of 8 per CU.  Told no occupancy, the
+// compiler splits the requests to fit eight.)
+template <int MT, int NB, int EPI, bool NORM, int NW, int K, bool HALF>
+__global__ void __launch_bounds__(NW * 64)
+    __attribute__((amdgpu_waves_per_eu(4, 4)))
+    gemm_rows(const uint16_t* __restrict__ X, const uint16_t* __restrict__ norm_w, const float* __restrict__ ssq_in,
+              float eps, int T, Seg seg, uint16_t* __restrict__ Y, int ldy, float* __restrict__ ssq_out) {
+  constexpr int ITERS = K / (64 * NW);  // 64-K steps per wave
   constexpr int NC = 16 * NB;
-  constexpr int NO = HALF ? 8 : NC;  // output columns per tile
+  constexpr int NO = HALF ? 8 : NC;  // product columns per tile
   static_assert(!HALF || (NB == 1 && EPI != kEpiSiluMul), "half tiles: one 16-column MFMA tile, plain rows");
   extern __shared__ __align__(16) unsigned char smem[];
-  uint16_t* xs = reinterpret_cast<uint16_t*>(smem);
-  const size_t xs_bytes = NORM ? (size_t)((T * K * 2 + 15) / 16 * 16) : 0;
-  float (*red)[16][NC] = reinterpret_cast<float (*)[16][NC]>(smem + xs_bytes);
-  float (*ssr)[16] = reinterpret_cast<float (*)[16]>(smem + xs_bytes + (size_t)NW * 16 * NC * 4);
-  float* rstd_s = reinterpret_cast<float*>(smem + xs_bytes + (size_t)NW * 16 * NC * 4 + (size_t)NW * 16 * 4);
-  const int tile = blockIdx.x;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int kq = 8 * (lane >> 4);
-  const int k0 = w * (64 * ITERS);
-  const int row = min(lane & 15, T - 1);
-  // NORM: the T input rows in 16-byte chunks (chunk c = thread + NT * q covers row 8c / K) and
-  // their norm weights are requested first, then the wave's whole weight slice, so that waiting
-  // for the rows (vector memory returns in order) never waits for the weights
-  constexpr int NT = NW * 64, MAXQ = NORM ? (MAXT * kMaxRowsH / 8 + NT - 1) / NT : 1;  // T <= MAXT
-  const int nchunks = T * K / 8;
-  u32x4 xr[MAXQ], wr[MAXQ];
-  if (NORM) {
+  float (*red)[16][NO] = reinterpret_cast<float (*)[16][NO]>(smem);
+  float* rstd_s = reinterpret_cast<float*>(smem + (size_t)NW * 16 * NO * 4);
+  const int tile = blockIdx.x, tb = blockIdx.y * 16 * MT;  // rows tb .. tb + 16 MT - 1
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15;
+  const int kq = 8 * (lane >> 4), k0 = w * (64 * ITERS);
+  // the rows' partial sums of squares (row w, w + NW, ..), then this wave's operand rows
+  constexpr int NR = NORM ? (16 * MT + NW - 1) / NW : 1;
+  constexpr int nss = K / 8;  // partials per row: 128 or 256
+  f32x4 sv[NR];
+  if constexpr (NORM) {
 #pragma unroll
-    for (int q = 0; q < MAXQ; q++) {
-      const int c = threadIdx.x + NT * q;
-      if (c < nchunks) {
-        xr[q] = ld16(X + (size_t)c * 8);
-        wr[q] = ld16(norm_w + (c * 8) % K);
-      }
+    for (int q = 0; q < NR; q++) {
+      const float* sp = ssq_in + (size_t)min(tb + w + NW * q, T - 1) * nss;
+      sv[q] = 4 * lane < nss ? *reinterpret_cast<const f32x4*>(sp + 4 * lane) : f32x4{0.f, 0.f, 0.f, 0.f};
     }
+  }
+  u32x4 a[MT][ITERS][2], wn[NORM ? ITERS : 1][2];
+#pragma unroll
+  for (int it = 0; it < ITERS; it++)
+#pragma unroll
+    for (int hf = 0; hf < 2; hf++) {
+      const int k = k0 + 64 * it + 32 * hf + kq;
+      if constexpr (NORM) wn[it][hf] = ld16(norm_w + k);
+#pragma unroll
+      for (int i = 0; i < MT; i++) a[i][it][hf] = ld16(X + (size_t)min(tb + 16 * i + l16, T - 1) * K + k);
+    }
+  // this thread's outputs of one row tile (16 rows x OC columns), and their elements of the hidden
+  // rows (residual)
+  constexpr int OC = EPI == kEpiSiluMul ? NC / 2 : NO;  // output columns per tile
+  static_assert(16 * OC <= NW * 64, "one output per thread and row tile");
+  const int rt = threadIdx.x / OC, rc = threadIdx.x % OC;
+  uint32_t xold[MT];
+  if constexpr (EPI == kEpiResidual) {
+#pragma unroll
+    for (int i = 0; i < MT; i++) xold[i] = ldu16(Y + (size_t)min(tb + 16 * i + rt, T - 1) * ldy + tile * OC + rc);
   }
   bf16x8 b[ITERS][2][NB];
 #pragma unroll
   for (int j = 0; j < NB; j++) {
     const uint16_t* wrow = (HALF ? tile_row<EPI, NO>(seg, tile, lane & 7, K)
-                                 : tile_row<EPI, NC>(seg, tile, 16 * j + (lane & 15), K)) + kq + k0;
+                                 : tile_row<EPI, NC>(seg, tile, 16 * j + l16, K)) + kq + k0;
 #pragma unroll
     for (int it = 0; it < ITERS; it++) {
       b[it][0][j] = ld_bf16x8_stream(wrow + 64 * it);
       b[it][1][j] = ld_bf16x8_stream(wrow + 64 * it + 32);
     }
   }
-  if (NORM) {
-    // RMSNorm of the rows into LDS, bf16(w * bf16(x * rstd)) as HF.  A wave's 64 chunks of one q
-    // lie in one row (K / 8 is a multiple of 64), so each wave sum belongs to one row.
-    float (*ssq)[NW] = reinterpret_cast<float (*)[NW]>(&ssr[0][0]);  // [MAXQ][NW] <= [16][NW]
+  if constexpr (NORM) {
 #pragma unroll
-    for (int q = 0; q < MAXQ; q++) {
-      const int c0 = w * 64 + NT * q;  // the wave's first chunk of this q
-      if (c0 < nchunks) {
-        float part = 0.f;
-        const u32x4 v = xr[q];
-        const uint32_t u4[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float lo = lo_bf16(u4[e]), hi = hi_bf16(u4[e]);
-          part += lo * lo + hi * hi;
-        }
-        part = wave_sum(part);
-        if (lane == 0) ssq[q][w] = part;
-      }
-    }
-    __syncthreads();
-    if ((int)threadIdx.x < T) {
-      // row t's wave sums, in (q, wave) order
-      float ss = 0.f;
-      for (int q = 0; q < MAXQ; q++)
-        for (int ww = 0; ww < NW; ww++) {
-          const int c0 = ww * 64 + NT * q;
-          if (c0 < nchunks && (c0 * 8) / K == (int)threadIdx.x) ss += ssq[q][ww];
-        }
-      rstd_s[threadIdx.x] = rcp_sqrt_torch(__fdiv_rn(ss, (float)K) + eps);
+    for (int q = 0; q < NR; q++) {
+      const float ss = wave_sum((sv[q][0] + sv[q][1]) + (sv[q][2] + sv[q][3]));
+      if (lane == 0 && w + NW * q < 16 * MT) rstd_s[w + NW * q] = rcp_sqrt_torch(__fdiv_rn(ss, (float)K) + eps);
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < MAXQ; q++) {
-      const int c = threadIdx.x + NT * q;
-      if (c < nchunks) {
-        const float r = rstd_s[(c * 8) / K];
-        const uint32_t xv[4] = {xr[q].x, xr[q].y, xr[q].z, xr[q].w};
-        const uint32_t wv[4] = {wr[q].x, wr[q].y, wr[q].z, wr[q].w};
-        uint32_t o[4];
+    for (int i = 0; i < MT; i++) {
+      const float r = rstd_s[16 * i + l16];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const float n0 = bf16r(lo_bf16(wv[e]) * bf16r(lo_bf16(xv[e]) * r));
-          const float n1 = bf16r(hi_bf16(wv[e]) * bf16r(hi_bf16(xv[e]) * r));
-          o[e] = f32_to_bf16(n0) | (f32_to_bf16(n1) << 16);
+      for (int it = 0; it < ITERS; it++)
+#pragma unroll
+        for (int hf = 0; hf < 2; hf++) {
+          u32x4 v = a[i][it][hf];
+          const u32x4 n = wn[it][hf];
+#pragma unroll
+          for (int e = 0; e < 4; e++) {
+            const uint32_t y = pack_bf16x2(lo_bf16(v[e]) * r, hi_bf16(v[e]) * r);
+            v[e] = pack_bf16x2(lo_bf16(n[e]) * lo_bf16(y), hi_bf16(n[e]) * hi_bf16(y));
+          }
+          a[i][it][hf] = v;
         }
-        *reinterpret_cast<u32x4*>(xs + (size_t)c * 8) = u32x4{o[0], o[1], o[2], o[3]};
-      }
     }
-    __syncthreads();
   }
-  auto load_a = [&](int k) -> bf16x8 {
-    if (NORM) return *reinterpret_cast<const bf16x8*>(xs + row * K + kq + k);
-    return ld_bf16x8(X + (size_t)row * K + kq + k);
-  };
-  bf16x8 a[ITERS][2];
+  f32x4 acc[MT][NB];
 #pragma unroll
-  for (int it = 0; it < ITERS; it++) {
-    a[it][0] = load_a(k0 + 64 * it);
-    a[it][1] = load_a(k0 + 64 * it + 32);
-  }
-  f32x4 acc[NB];
+  for (int i = 0; i < MT; i++)
 #pragma unroll
-  for (int j = 0; j < NB; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NB; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int it = 0; it < ITERS; it++)
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[it][0], b[it][0][j], acc[j], 0, 0, 0);
-      acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[it][1], b[it][1][j], acc[j], 0, 0, 0);
+    for (int hf = 0; hf < 2; hf++)
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int i = 0; i < MT; i++)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a[i][it][hf]), b[it][hf][j],
+                                                              acc[i][j], 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < MT; i++) {  // one row tile at a time through LDS
+    if (i) __syncthreads();
+    if (!HALF || l16 < 8) {
+#pragma unroll
+      for (int j = 0; j < NB; j++)
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[w][4 * (lane >> 4) + r][16 * j + l16] = acc[i][j][r];
     }
+    __syncthreads();
+    const int t = tb + 16 * i + rt;
+    if (rt >= 16) continue;  // whole waves
+    auto col_sum = [&](int cc) {
+      float y = 0.f;
 #pragma unroll
-  for (int j = 0; j < NB; j++)
-#pragma unroll
-    for (int i = 0; i < 4; i++) red[w][4 * (lane >> 4) + i][16 * j + (lane & 15)] = acc[j][i];
-  __syncthreads();
-  const int t = threadIdx.x / NO, c = threadIdx.x % NO;
-  if (t >= T || t >= 16) return;
-  auto col_sum = [&](int cc) {
-    float y = 0.f;
-#pragma unroll
-    for (int q = 0; q < NW; q++) y += red[q][t][cc];  // wave order
-    return y;
-  };
-  if (EPI == kEpiSiluMul) {
-    if (c >= NC / 2) return;
-    const float g = bf16r(col_sum(c)), u = bf16r(col_sum(c + NC / 2));
-    const float sg = bf16r(__fdiv_rn(g, 1.0f + expf(-g)));
-    Y[(size_t)t * ldy + tile * (NC / 2) + c] = (uint16_t)f32_to_bf16(bf16r(sg * u));
-    return;
+      for (int k = 0; k < NW; k++) y += red[k][rt][cc];  // wave order
+      return y;
+    };
+    uint16_t* dst = Y + (size_t)t * ldy + tile * OC + rc;
+    if constexpr (EPI == kEpiSiluMul) {
+      const float g = bf16r(col_sum(rc)), u = bf16r(col_sum(rc + NC / 2));
+      if (t < T) *dst = (uint16_t)f32_to_bf16(silu_mul(g, u));
+    } else if constexpr (EPI == kEpiResidual) {
+      const float x = bf16r(bf16_to_f32(xold[i]) + bf16r(col_sum(rc)));
+      // 8 columns of row t are 8 neighbouring lanes: one partial sum of squares
+      float ss = x * x;
+      ss = dpp_add<0xB1>(ss);   // quad_perm [1,0,3,2]
+      ss = dpp_add<0x4E>(ss);   // quad_perm [2,3,0,1]
+      ss = dpp_add<0x141>(ss);  // row_half_mirror
+      if (t < T) {
+        *dst = (uint16_t)f32_to_bf16(x);
+        if (rc % 8 == 0) ssq_out[(size_t)t * (ldy / 8) + (tile * OC + rc) / 8] = ss;
+      }
+    } else {
+      const float y = col_sum(rc);
+      if (t < T) *dst = (uint16_t)f32_to_bf16(y);
+    }
   }
-  const float y = bf16r(col_sum(c));
-  uint16_t* dst = Y + (size_t)t * ldy + tile * NO + c;
-  if (EPI == kEpiResidual) *dst = (uint16_t)f32_to_bf16(bf16r(bf16_to_f32(*dst) + y));
-  else *dst = (uint16_t)f32_to_bf16(y);
+}
+
+// q/k norm + RoPE and K/V append from gemm_rows' bf16 q|k|v rows: one wave per (token, head)
+__global__ void __launch_bounds__(256) qkv_rows_finish(const uint16_t* __restrict__ QKV, QkvOut o) {
+  const int t = blockIdx.x, h = blockIdx.y * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const uint16_t* x = QKV + (size_t)t * kNQKV + h * kD + lane;
+  const uint32_t x0 = ldu16(x), x1 = ldu16(x + 64);
+  qkv_head(o, t, h, lane, bf16_to_f32(x0), bf16_to_f32(x1));
 }
 
 // ---------------------------------------------------------------- self-test
@@ -1979,11 +2017,8 @@ AttnSplit attn_mfma_split(int T, int max_context) {
 }
 
 struct Layout {
-  size_t tok, erow, keys, x, n, q, att, m, qkv, part, scores, ml, pv, redo, mml, mpart, total;
+  size_t tok, erow, keys, x, n, q, att, m, qkv, ssq, part, scores, ml, pv, redo, mml, mpart, total;
 };
-
-// The decode step of few sequences (one token each) takes the fused path.
-bool fused_decode(int T) { return T <= 16; }
 
 template <class M>
 Layout layout(int T, int R, int max_context, bool one_per_seq) {
@@ -2004,22 +2039,22 @@ Layout layout(int T, int R, int max_context, bool one_per_seq) {
   take(l.q, (size_t)T * kQS * 2);
   take(l.att, (size_t)T * kQS * 2);
   take(l.m, (size_t)T * Dm::I * 2);
-  if (split_attention(T, max_context, one_per_seq) || (one_per_seq && fused_decode(T))) {
+  if (split_attention(T, max_context, one_per_seq) || (one_per_seq && T <= kRowsMax)) {
     const int nch = split_chunks(max_context);
     take(l.scores, (size_t)T * kNQ * nch * kSplitChunk * 4);
     take(l.ml, (size_t)T * kNQ * nch * 8);
     take(l.pv, (size_t)T * nch * kQS * 4);
   }
-  if (one_per_seq && fused_decode(T)) {
+  if (T <= kRowsMax) {
     take(l.qkv, (size_t)T * kNQKV * 2);
-    l.total = off;
-    return l;
+    take(l.ssq, (size_t)T * (Dm::H / 8) * 4);
+  } else {
+    size_t pf = part_floats(T, kNQKV, Dm::H);
+    pf = std::max(pf, part_floats(T, Dm::H, kQS));
+    pf = std::max(pf, part_floats(T, 2 * Dm::I, Dm::H));
+    pf = std::max(pf, part_floats(T, Dm::H, Dm::I));
+    take(l.part, pf * 4);
   }
-  size_t pf = part_floats(T, kNQKV, Dm::H);
-  pf = std::max(pf, part_floats(T, Dm::H, kQS));
-  pf = std::max(pf, part_floats(T, 2 * Dm::I, Dm::H));
-  pf = std::max(pf, part_floats(T, Dm::H, Dm::I));
-  take(l.part, pf * 4);
   take(l.redo, (size_t)((T + kQT - 1) / kQT) * 4);
   const AttnSplit sp = attn_mfma_split(T, max_context);
   if (mfma_attention(T, max_context, one_per_seq) && sp.nch > 1) {  // attention_mfma's chunks: (max, sum), partials
@@ -2079,42 +2114,37 @@ void launch_lm_head(const uint16_t* N, const int* erow, int R, const uint16_t* W
   hipLaunchKernelGGL(keys_reduce, dim3(R), dim3(256), 0, s, keys, (int)grid.x, erow, tok, out);
 }
 
-// gemm_rows over `tiles` 16-column tiles (NB = 1), NW waves each taking
-// K / NW = 64 * ITERS of the K range; ITERS picked from K.
-template <int EPI, bool NORM, int NW, int ITERS, int MAXT, bool HALF>
-void launch_rows_t(int tiles, const uint16_t* X, const uint16_t* nw, float eps, int T, int K, const Seg& seg,
-                   uint16_t* Y, int ldy, hipStream_t s) {
-  const size_t lds = rows_lds<1, NW, NORM>(T, K);
-  if (lds > 64 * 1024) {
-    // 16 normalised rows of 2048: above the default dynamic LDS limit (gfx950 has 160 KB per CU)
-    static bool raised = false;
-    if (!raised)
-      raised = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_rows<1, EPI, NORM, NW, ITERS, MAXT, HALF>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024) == hipSuccess;
-  }
-  hipLaunchKernelGGL((gemm_rows<1, EPI, NORM, NW, ITERS, MAXT, HALF>), dim3(tiles), dim3(NW * 64), lds, s, X, nw, eps, T,
-                     K, seg, Y, ldy);
+// gemm_rows with RMSNorm over `tiles` tiles of 16 NB product columns, 16 waves: all T rows in every
+// workgroup, so the weights are read once
+template <int K, int NB, int EPI>
+void launch_rows_norm(int tiles, const uint16_t* X, const uint16_t* nw, const float* ssq, float eps, int T,
+                      const Seg& seg, uint16_t* Y, int ldy, hipStream_t s) {
+  constexpr int NW = 16;
+  auto go = [&](auto mt) {
+    constexpr int MT = decltype(mt)::value;
+    constexpr size_t lds = rows_lds<MT, 16 * NB, NW>();
+    static_assert(lds <= 64 * 1024, "the default dynamic LDS limit");
+    hipLaunchKernelGGL((gemm_rows<MT, NB, EPI, true, NW, K, false>), dim3(tiles), dim3(NW * 64), lds, s, X, nw, ssq, eps,
+                       T, seg, Y, ldy, nullptr);
+  };
+  if (T <= 16) go(std::integral_constant<int, 1>{});
+  else go(std::integral_constant<int, 2>{});
 }
 
-// NORM kernels stage the rows in registers sized for T <= 4 (the common batch) or T <= 16.
-template <int EPI, bool NORM, int NW, int ITERS, bool HALF>
-void launch_rows_it(int tiles, const uint16_t* X, const uint16_t* nw, float eps, int T, int K, const Seg& seg,
-                    uint16_t* Y, int ldy, hipStream_t s) {
-  if (!NORM || T <= 4) launch_rows_t<EPI, NORM, NW, ITERS, 4, HALF>(tiles, X, nw, eps, T, K, seg, Y, ldy, s);
-  else launch_rows_t<EPI, NORM, NW, ITERS, 16, HALF>(tiles, X, nw, eps, T, K, seg, Y, ldy, s);
-}
-
-// `tiles` tiles of 16 output columns, or of 8 (HALF)
-template <int EPI, bool NORM, int NW, bool HALF = false>
-void launch_rows(int tiles, const uint16_t* X, const uint16_t* nw, float eps, int T, int K, const Seg& seg,
-                 uint16_t* Y, int ldy, hipStream_t s) {
-  switch (K / (64 * NW)) {
-    case 1: launch_rows_it<EPI, NORM, NW, 1, HALF>(tiles, X, nw, eps, T, K, seg, Y, ldy, s); break;
-    case 2: launch_rows_it<EPI, NORM, NW, 2, HALF>(tiles, X, nw, eps, T, K, seg, Y, ldy, s); break;
-    case 3: launch_rows_it<EPI, NORM, NW, 3, HALF>(tiles, X, nw, eps, T, K, seg, Y, ldy, s); break;
-    case 4: launch_rows_it<EPI, NORM, NW, 4, HALF>(tiles, X, nw, eps, T, K, seg, Y, ldy, s); break;
-    default: launch_rows_it<EPI, NORM, NW, 6, HALF>(tiles, X, nw, eps, T, K, seg, Y, ldy, s); break;
-  }
+// gemm_rows with the residual epilogue into the H columns of X: a workgroup per 16-row tile (a second
+// one finds the weights in its XCD's L2) and 8 columns, or 16 where 8 would make more workgroups
+// than CUs (one of 16 waves fits; H = 2048, 24 rows, 512 workgroups against 256: o 10.0 -> 6.4
+// us, down 22.6 -> 15.2)
+template <int K, int H>
+void launch_rows_residual(const uint16_t* A, int T, const Seg& seg, uint16_t* X, float* ssq, hipStream_t s) {
+  constexpr int NW = 16;
+  const int rt = (T + 15) / 16;
+  if (rt * (H / 8) <= kNumWG)
+    hipLaunchKernelGGL((gemm_rows<1, 1, kEpiResidual, false, NW, K, true>), dim3(H / 8, rt), dim3(NW * 64),
+                       (rows_lds<1, 8, NW>()), s, A, nullptr, nullptr, 0.f, T, seg, X, H, ssq);
+  else
+    hipLaunchKernelGGL((gemm_rows<1, 1, kEpiResidual, false, NW, K, false>), dim3(H / 16, rt), dim3(NW * 64),
+                       (rows_lds<1, 16, NW>()), s, A, nullptr, nullptr, 0.f, T, seg, X, H, ssq);
 }
 
 // The context-split attention of one layer: RAW from the q/k/v projection's output, else from
@@ -2141,41 +2171,80 @@ void launch_attn_chunks(const Args& a, const AttnChunks& ac, const uint16_t* src
   hipLaunchKernelGGL(attn_chunk_merge, dim3(a.T, kNQ), dim3(256), 0, s, tok, ac.nch, ac.pvp, out);
 }
 
+// The attention of one layer whose q rows are finished and K/V appended: the context-split form, the
+// MFMA form (and the row kernel for the tiles that it leaves), or the row kernel.
+void launch_attention(const Args& a, const Layout& l, const uint16_t* Q, const Tok* tok, int L,
+                      const LDGLayerWeights& w, float eps, uint16_t* ATT, hipStream_t s) {
+  const int T = a.T;
+  if (split_attention(T, a.max_context, a.one_per_seq)) {
+    launch_attn_chunks<false>(a, attn_chunks(a, l), Q, tok, L, w, eps, ATT, s);
+    return;
+  }
+  if (!mfma_attention(T, a.max_context, a.one_per_seq)) {
+    hipLaunchKernelGGL(attention_rows, dim3(T, kNKV), dim3(256), 0, s, Q, tok, T, L, a.cache, a.attn_scale, ATT, nullptr);
+    return;
+  }
+  // tiles of one sequence's consecutive tokens on MFMA; any other tile row by row
+  const AttnSplit asp = attn_mfma_split(T, a.max_context);
+  int* redo = reinterpret_cast<int*>(a.ws + l.redo);
+  const int ntiles = (T + kQT - 1) / kQT;
+  if (asp.nch > 1) {
+    float2* aml = reinterpret_cast<float2*>(a.ws + l.mml);
+    float* apart = reinterpret_cast<float*>(a.ws + l.mpart);
+    const dim3 grid(ntiles * asp.nch, kNQ);
+    hipLaunchKernelGGL(attention_mfma_pass1, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache,
+                       a.attn_scale, ATT, redo, asp.nch, asp.ck, aml, apart);
+    hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache,
+                       a.attn_scale, ATT, redo, asp.nch, asp.ck, aml, apart);
+    hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, tok, T, asp.nch, asp.ck, apart, redo,
+                       ATT);
+  } else {
+    hipLaunchKernelGGL(attention_mfma, dim3((ntiles + 1) / 2, kNQ), dim3(kAttnWaves * 64), 0, s, Q,
+                       tok, T, L, a.cache, a.attn_scale, ATT, redo, 1, 0, nullptr, nullptr);
+  }
+  // the tiles attention_mfma left (redo) row by row: 256 x 8 workgroups loop over the tokens
+  hipLaunchKernelGGL(attention_rows, dim3(std::min(T, 256), kNKV), dim3(256), 0, s, Q, tok, T, L, a.cache,
+                     a.attn_scale, ATT, redo);
+}
+
 template <class M>
-int forward_fused(const Args& a, hipStream_t s) {
+int forward_rows(const Args& a, hipStream_t s) {
   using Dm = Dims<M>;
   const int T = a.T, R = a.R;
-  const Layout l = layout<M>(T, R, a.max_context, true);
+  const Layout l = layout<M>(T, R, a.max_context, a.one_per_seq);
   Tok* tok = reinterpret_cast<Tok*>(a.ws + l.tok);
   int* erow = reinterpret_cast<int*>(a.ws + l.erow);
   auto* keys = reinterpret_cast<unsigned long long*>(a.ws + l.keys);
   uint16_t* X = reinterpret_cast<uint16_t*>(a.ws + l.x);
   uint16_t* N = reinterpret_cast<uint16_t*>(a.ws + l.n);
+  uint16_t* Qb = reinterpret_cast<uint16_t*>(a.ws + l.q);
   uint16_t* ATT = reinterpret_cast<uint16_t*>(a.ws + l.att);
   uint16_t* MM = reinterpret_cast<uint16_t*>(a.ws + l.m);
   uint16_t* QKV = reinterpret_cast<uint16_t*>(a.ws + l.qkv);
+  float* ssq = reinterpret_cast<float*>(a.ws + l.ssq);
   const float eps = 1e-6f;
   auto u16 = [](const void* p) { return static_cast<const uint16_t*>(p); };
-  // every K is split into 16 (8 for gate/up) slices of 64 * {1, 2, 3, 4, 6}
-  static_assert(Dm::H == 1024 || Dm::H == 2048, "K splits of the hidden size");
-  static_assert(Dm::I == 3072 || Dm::I == 6144, "K splits of the MLP size");
-  static_assert(kQS == 2048 && Dm::H <= kMaxRowsH, "K splits of the attention output");
-  const AttnChunks ac = attn_chunks(a, l);
-  hipLaunchKernelGGL(prep_tokens, dim3((std::max(T, R) + 255) / 256), dim3(256), 0, s, a.tokens, a.seqs, a.pos, T,
-                     a.emit, R, a.num_seqs, a.max_context, Dm::V, tok, erow);
-  hipLaunchKernelGGL(embed_rows, dim3(T), dim3(256), 0, s, a.embed, tok, Dm::H, X);
+  hipLaunchKernelGGL((embed_tokens<Dm::H, false>), dim3(T), dim3(256), 0, s, a.tokens, a.seqs, a.pos, T, a.emit, R,
+                     a.num_seqs, a.max_context, Dm::V, a.embed, tok, erow, X, nullptr, eps, nullptr, ssq);
   for (int L = 0; L < a.num_layers; L++) {
     const LDGLayerWeights& w = a.layers[L];
     const Seg qkv{{u16(w.q_proj_weight), u16(w.k_proj_weight), u16(w.v_proj_weight)}, {kQS, kNKV * kD, kNKV * kD}};
-    launch_rows<kEpiStore, true, 16>(kNQKV / 16, X, u16(w.input_layernorm_weight), eps, T, Dm::H, qkv, QKV, kNQKV, s);
-    launch_attn_chunks<true>(a, ac, QKV, tok, L, w, eps, ATT, s);
+    launch_rows_norm<Dm::H, 1, kEpiStore>(kNQKV / 16, X, u16(w.input_layernorm_weight), ssq, eps, T, qkv, QKV, kNQKV, s);
+    if (a.one_per_seq) {
+      launch_attn_chunks<true>(a, attn_chunks(a, l), QKV, tok, L, w, eps, ATT, s);
+    } else {
+      const QkvOut qo{tok, L, u16(w.q_norm_weight), u16(w.k_norm_weight), a.cos_t, a.sin_t, a.cache, eps, Qb};
+      hipLaunchKernelGGL(qkv_rows_finish, dim3(T, (kNQ + 2 * kNKV) / 4), dim3(256), 0, s, QKV, qo);
+      launch_attention(a, l, Qb, tok, L, w, eps, ATT, s);
+    }
     const Seg o{{u16(w.o_proj_weight), nullptr, nullptr}, {Dm::H, 0, 0}};
-    launch_rows<kEpiResidual, false, 16, true>(Dm::H / 8, ATT, nullptr, eps, T, kQS, o, X, Dm::H, s);
+    launch_rows_residual<kQS, Dm::H>(ATT, T, o, X, ssq, s);
     const Seg gu{{u16(w.gate_proj_weight), u16(w.up_proj_weight), nullptr}, {Dm::I, Dm::I, 0}};
-    launch_rows<kEpiSiluMul, true, 8>(Dm::I / 8, X, u16(w.post_attn_layernorm_weight), eps, T, Dm::H, gu, MM, Dm::I,
-                                      s);
+    constexpr int GB = Dm::I / 8 / kNumWG;  // 32 or 48 product columns per workgroup: at most one per CU
+    launch_rows_norm<Dm::H, GB < 2 ? 2 : GB, kEpiSiluMul>(Dm::I / (8 * (GB < 2 ? 2 : GB)), X, u16(w.post_attn_layernorm_weight), ssq, eps, T,
+                                                          gu, MM, Dm::I, s);
     const Seg dn{{u16(w.down_proj_weight), nullptr, nullptr}, {Dm::H, 0, 0}};
-    launch_rows<kEpiResidual, false, 16, true>(Dm::H / 8, MM, nullptr, eps, T, Dm::I, dn, X, Dm::H, s);
+    launch_rows_residual<Dm::I, Dm::H>(MM, T, dn, X, ssq, s);
   }
   hipLaunchKernelGGL((residual_norm<Dm::H>), dim3(T), dim3(256), 0, s, nullptr, 0, T, X, a.final_norm, eps, N);
   launch_lm_head<M>(N, erow, R, a.lm_head, keys, a.logits, tok, a.out_tokens, s);
@@ -2186,7 +2255,7 @@ template <class M>
 int forward(const Args& a, hipStream_t s) {
   using Dm = Dims<M>;
   const int T = a.T, R = a.R;
-  if (a.one_per_seq && fused_decode(T)) return forward_fused<M>(a, s);
+  if (T <= kRowsMax) return forward_rows<M>(a, s);
   const Layout l = layout<M>(T, R, a.max_context, a.one_per_seq);
   Tok* tok = reinterpret_cast<Tok*>(a.ws + l.tok);
   int* erow = reinterpret_cast<int*>(a.ws + l.erow);
@@ -2198,53 +2267,20 @@ int forward(const Args& a, hipStream_t s) {
   uint16_t* MM = reinterpret_cast<uint16_t*>(a.ws + l.m);
   float* part = reinterpret_cast<float*>(a.ws + l.part);
   const float eps = 1e-6f;
-  const bool split = split_attention(T, a.max_context, a.one_per_seq);
-  const bool mfma_attn = mfma_attention(T, a.max_context, a.one_per_seq);
-  const AttnSplit asp = attn_mfma_split(T, a.max_context);
   auto blocks = [](size_t n) { return dim3((unsigned)((n + 255) / 256)); };
   auto u16 = [](const void* p) { return static_cast<const uint16_t*>(p); };
   int ks = 1;
 
-  hipLaunchKernelGGL(prep_tokens, blocks(std::max(T, R)), dim3(256), 0, s, a.tokens, a.seqs, a.pos, T, a.emit, R,
-                     a.num_seqs, a.max_context, Dm::V, tok, erow);
-  hipLaunchKernelGGL(embed_rows, dim3(T), dim3(256), 0, s, a.embed, tok, Dm::H, X);
-  hipLaunchKernelGGL((residual_norm<Dm::H>), dim3(T), dim3(256), 0, s, nullptr, 0, T, X,
-                     u16(a.layers[0].input_layernorm_weight), eps, N);
+  hipLaunchKernelGGL((embed_tokens<Dm::H, true>), dim3(T), dim3(256), 0, s, a.tokens, a.seqs, a.pos, T, a.emit, R,
+                     a.num_seqs, a.max_context, Dm::V, a.embed, tok, erow, X, u16(a.layers[0].input_layernorm_weight),
+                     eps, N, nullptr);
   for (int L = 0; L < a.num_layers; L++) {
     const LDGLayerWeights& w = a.layers[L];
     const Seg qkv{{u16(w.q_proj_weight), u16(w.k_proj_weight), u16(w.v_proj_weight)}, {kQS, kNKV * kD, kNKV * kD}};
     const QkvOut qo{tok, L, u16(w.q_norm_weight), u16(w.k_norm_weight), a.cos_t, a.sin_t, a.cache, eps, Qb};
     launch_gemm(N, T, Dm::H, qkv, kNQKV, part, s, &ks, kEpiQkv, &qo);
     if (ks) hipLaunchKernelGGL(qkv_finish, dim3(T, kNQ + 2 * kNKV), dim3(64), 0, s, part, ks, T, qo);
-    if (split) {
-      launch_attn_chunks<false>(a, attn_chunks(a, l), Qb, tok, L, w, eps, ATT, s);
-    } else {
-      if (mfma_attn) {
-        // tiles of one sequence's consecutive tokens on MFMA; any other tile row by row
-        int* redo = reinterpret_cast<int*>(a.ws + l.redo);
-        const int ntiles = (T + kQT - 1) / kQT;
-        if (asp.nch > 1) {
-          float2* aml = reinterpret_cast<float2*>(a.ws + l.mml);
-          float* apart = reinterpret_cast<float*>(a.ws + l.mpart);
-          const dim3 grid(ntiles * asp.nch, kNQ);
-          hipLaunchKernelGGL(attention_mfma_pass1, grid, dim3(kAttnWaves * 64), 0, s, Qb, tok, T, L, a.cache,
-                             a.attn_scale, ATT, redo, asp.nch, asp.ck, aml, apart);
-          hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Qb, tok, T, L, a.cache,
-                             a.attn_scale, ATT, redo, asp.nch, asp.ck, aml, apart);
-          hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, tok, T, asp.nch, asp.ck, apart, redo,
-                             ATT);
-        } else {
-          hipLaunchKernelGGL(attention_mfma, dim3((ntiles + 1) / 2, kNQ), dim3(kAttnWaves * 64), 0, s, Qb,
-                             tok, T, L, a.cache, a.attn_scale, ATT, redo, 1, 0, nullptr, nullptr);
-        }
-        // the tiles attention_mfma left (redo) row by row: 256 x 8 workgroups loop over the tokens
-        hipLaunchKernelGGL(attention_rows, dim3(std::min(T, 256), kNKV), dim3(256), 0, s, Qb, tok, T, L, a.cache,
-                           a.attn_scale, ATT, redo);
-      } else {
-        hipLaunchKernelGGL(attention_rows, dim3(T, kNKV), dim3(256), 0, s, Qb, tok, T, L, a.cache, a.attn_scale, ATT,
-                           nullptr);
-      }
-    }
+    launch_attention(a, l, Qb, tok, L, w, eps, ATT, s);
     const Seg o{{u16(w.o_proj_weight), nullptr, nullptr}, {Dm::H, 0, 0}};
     launch_gemm(ATT, T, kQS, o, Dm::H, part, s, &ks);
     hipLaunchKernelGGL((residual_norm<Dm::H>), dim3(T), dim3(256), 0, s, part, ks, T, X,

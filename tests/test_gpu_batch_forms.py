@@ -93,3 +93,44 @@ def test_lm_head_row_groups(weights_gpu, rows):
             ulp = torch.exp2(torch.floor(torch.log2(y.abs().clamp_min(1e-3))) - 7)
             assert ((x - y).abs() <= 1.01 * ulp).all()
             assert int(out[r0 + r]) == int(torch.argmax(x.cpu()))
+
+
+@pytest.fixture(scope="module")
+def qwen3_1p7b():
+    from oracle.qwen3_exact import ExactWeights
+    from qwen_megakernel.shapes import QWEN3_1_7B
+    from qwen_megakernel.weights import make_weights, to_device
+
+    w = make_weights(QWEN3_1_7B, seed=0, num_layers=2, max_seq_len=256)
+    return QWEN3_1_7B, ExactWeights(w, QWEN3_1_7B, num_layers=2), to_device(w, "cuda")
+
+
+@pytest.mark.parametrize("model,n", [("0.6b", n) for n in (15, 16, 17, 32, 33)] + [("1.7b", n) for n in (9, 17, 32)])
+def test_prompt_row_tiles(request, model, n):
+    """gemm_rows' row tiles (one up to 16 tokens, two up to 32; for the larger model the residual products'
+    16-column tiles at two) and the first count past them: every row of a prompt after 5 positions, 2
+    layers, and its K/V rows."""
+    from qwen_megakernel.weights import make_prompt
+
+    from parity import decoder
+
+    if model == "0.6b":
+        shape, exact, weights = (request.getfixturevalue(f) for f in ("shape", "exact06", "weights_gpu"))
+    else:
+        shape, exact, weights = request.getfixturevalue("qwen3_1p7b")
+    V, start, S = 151936, 5, 256
+    dec = decoder(weights, num_layers=2, max_seq_len=S)
+    dec.prefill(make_prompt(start, shape.vocab, seed=8))
+    ids = make_prompt(n, shape.vocab, seed=n)
+
+    def i32(x):
+        return torch.tensor(x, dtype=torch.int32, device="cuda")
+
+    out = torch.empty(n, dtype=torch.int32, device="cuda")
+    logits = torch.empty(n, V, dtype=torch.float32, device="cuda")
+    dec._forward(i32(ids), i32([0] * n), i32(list(range(start, start + n))), i32(list(range(n))), out, logits,
+                 dec._k_cache, dec._v_cache, start + n)
+    orc = exact_oracle(exact, shape, S, num_layers=2)
+    ref = oracle_steps(orc, dec._k_cache, dec._v_cache, start, ids)
+    print(check_rows(Tally(f"{model} {n} rows"), ref, out.cpu().tolist(), logits.cpu(), bar=LITERAL))
+    check_kv_rows(f"{model} {n} rows", orc, dec._k_cache, dec._v_cache, start, n)
