@@ -1964,18 +1964,17 @@ int split_chunks(int max_context) { return (max_context + kSplitChunk - 1) / kSp
 
 // The context-split attention (three launches, each token's context over workgroups of
 // kSplitChunk positions) for a batched step and for few tokens over a longer context; the row kernel (one launch) for few tokens over
-// a short one.  Qwen3-0.6B prefills, split against rows, same box: from position 0, 1 token 1.31 /
-// 1.21 ms and 31 tokens 1.45 / 1.35; from 96, 1.41 / 1.39; from 192, 1.46 / 1.56; from 500, 1.45 /
-// 2.14.  Its work grows with tokens x context, attention_mfma's with the context alone (a 64-token
-// tile costs the same for 1 token as for 64), so a prompt of one sequence takes attention_mfma
-// from about 6144 tokens x positions (split against attention_mfma with its keys in chunks: 8
-// tokens after 600 positions 1.55 / 1.62 ms; 2 after 1500 1.61 / 1.64, 8 after 1500 1.83 / 1.68;
-// 1 after 4000 2.01 / 2.07, 2 after 4000 2.12 / 2.08; 1 after 7000 2.60 / 2.38; 31 after 7000
-// 17.96 / 2.42).  A batched decode step (one token per sequence, whose tiles hold several
-// sequences and would fall back to the row kernel) takes the split form at any batch: 48 sequences of
-// 100..1000 positions ran attention_mfma over no tile and then the row kernel, 86 us per layer
-// against 35.
-constexpr int kSplitWork = 6144;
+// a short one (Qwen3-0.6B, 31 tokens after 100 positions: 223 us split against 218 rows per 4-layer
+// forward; after 250, 228 against 254).  Its work grows with tokens x context, attention_mfma's with
+// the context alone (a 64-token tile costs the same for 1 token as for 64), so a prompt of one
+// sequence takes attention_mfma from about 32768 tokens x positions (split against attention_mfma
+// with its keys in chunks, us per 4-layer forward: after 700 positions 8 tokens 200 / 225 and 31
+// tokens 244 / 251; after 2000, 4 tokens 199 / 228 and 16 tokens 241 / 243; after 6500, 1 token 202
+// / 267 and 4 tokens 230 / 271).  A batched decode step (one token per sequence, whose tiles hold
+// several sequences and would fall back to the row kernel) takes the split form at any batch: 48
+// sequences of 100..1000 positions ran attention_mfma over no tile and then the row kernel, 86 us
+// per layer against 35.
+constexpr int kSplitWork = 32768;
 bool split_attention(int T, int max_context, bool one_per_seq) {
   return max_context > kSplitContext && (one_per_seq || (T < kSplitBelow && (long long)T * max_context < kSplitWork));
 }
