@@ -49,15 +49,20 @@ struct SampleParams {
   uint64_t seed;
 };
 
-// Device work of one logits row between the launches of a sampling call: the
-// row's radix histogram (counts or fixed-point masses) and selection state.
-// Zero between calls: the call's last launch clears it.
+// Device work of one logits row between the launches of a sampling call: the row's histogram (counts
+// or fixed-point masses), selection state and candidates.  Zero between calls (but for the
+// candidates): the call's last launch clears it.
+constexpr int kSampleBins = 2048, kSampleCand = 8192;
 struct SampleWork {
-  unsigned long long hist[256];  // bins of the current 8-bit radix digit
+  unsigned long long hist[kSampleBins];  // bins of the first digit (256 of them: of one 8-bit radix digit)
   unsigned long long z, target, need, best;  // need: top-k rank still sought / top-p mass above the prefix
   unsigned int maxkey, prefix, mask, kmin, pmin, ticket;
+  unsigned int ncand, candmin, candmax;  // candidates; ~(smallest key), largest key among them
+  unsigned int pad;
+  unsigned long long tied;               // best draw among the candidates, if their keys are all the same
+  unsigned long long cand[kSampleCand];  // key << 32 | token
 };
-constexpr int kSampleRowsMax = 256;  // rows per launch sequence of qmk_sample_rows
+constexpr int kSampleRowsMax = 64;  // rows per launch sequence of qmk_sample_rows (5 MB of work)
 
 // hipMalloc + zero fill of `rows` work blocks.
 int alloc_sample_work(SampleWork** out, int rows);

@@ -10,22 +10,28 @@
 //   draw:  argmax over kept v of s_v + G_v, G_v = -log(-log(U_v)) (Gumbel-max: a draw
 //          from softmax of the kept s), U_v from a counter-based hash of (seed, counter, v)
 //
-// Both thresholds are found by radix descent over the order-preserving 32-bit
-// key of s, 8 bits per pass: top-k over integer counts, top-p over
-// probability masses held as 2^-40 fixed-point integers (exp(s_v - max)
-// rounded once).  Every workgroup histograms its slice of the row in LDS and
-// adds its non-zero bins to the row's histogram with integer atomics; the last
-// workgroup of the pass (a ticket counter) picks the digit and prepares the
-// next pass.  Integer sums and integer maxima do not depend on the order of
-// the atomics, so results are deterministic.  The random numbers use
-// SplitMix64 (G. Steele, D. Lea, C. Flood, "Fast splittable pseudorandom
-// number generators", OOPSLA 2014).
+// Thresholds are exact: top-k over integer counts, top-p over probability masses held as 2^-40
+// fixed-point integers (exp(s_v - max) rounded once).  Integer sums and integer maxima do not depend
+// on the order of the atomics, so results are deterministic.  The random numbers use SplitMix64
+// (G. Steele, D. Lea, C. Flood, "Fast splittable pseudorandom number generators", OOPSLA 2014).
 //
-// Launches per sampling call: greedy or temperature only, 1 (the draw); top-k,
-// 4 + 1; top-p, 1 (the maximum score) + 4 (the first also sums the mass) + 1;
-// both, 10.  In the generate loop the maximum is the decode step's own greedy
-// logit over T, which saves the first launch.  (Three passes of 11 bits were
-// slower: 2048-bin histograms cost more per pass than the launch they save.)
+// With a filter, a call is two launches over the row (three for top-p alone, whose masses need the
+// row's maximum first; in the generate loop that is the decode step's own greedy logit over T):
+// - k_first histograms the slices over 2048 bins in LDS, adds the non-zero bins to the row's with
+//   integer atomics, and the last workgroup of the row (a ticket counter) finds the bin that holds the
+//   threshold.  top-k: counts over the top 11 bits of the order-preserving 32-bit key of s;  top-p
+//   alone: masses over (max - s) in steps of 1/64, so that a bin holds few scores wherever the
+//   threshold lies;
+// - k_finish draws among the scores above that bin, which are kept for certain, and collects the
+//   bin's own (with both filters: every score from that bin up) as candidates; the row's last
+//   workgroup finds the exact thresholds among these by radix descent in LDS, draws among those that
+//   stay and writes the token.
+// Candidates beyond kSampleCand (scores of the threshold's bin within 1/64 of each other by the
+// thousand, but not equal: equal ones need no list) are found again in the logits by the last
+// workgroup, one pass over the row per digit.  top-k above kFinishTopK keeps the general form: radix
+// descent over the whole row, 8 bits per launch (k_hist, 4 launches per threshold, then k_draw).
+// Each launch costs 7-9 us whatever it does, which is what bounds a call: four rows of 151,936
+// scores, top-k 50 + top-p 0.9: 10 launches 84 us -> 2 launches 24.4.
 
 #include <hip/hip_runtime.h>
 
@@ -35,6 +41,7 @@
 
 #include <map>
 #include <mutex>
+#include <type_traits>
 #include <utility>
 
 namespace qmk {
@@ -256,6 +263,315 @@ __global__ void __launch_bounds__(kThreads) k_hist(Args a, int pass) {
   }
 }
 
+// The row's token, and its work cleared for the next call (one thread of the row's last workgroup).
+__device__ __forceinline__ void put_token(const Args& a, const Block& b, int tok) {
+  SampleWork* w = b.w;
+  if (a.st) {
+    DecodeState* st = a.st;
+    st->tok = tok;
+    if (a.log) a.log[st->step - 1] = tok;
+    st->done = (st->eos >= 0 && tok == st->eos) ? 1u : 0u;
+  } else {
+    a.out[b.row] = tok;
+  }
+  w->z = w->target = w->need = w->best = w->tied = 0;
+  w->maxkey = w->prefix = w->mask = w->kmin = w->pmin = 0;
+  w->ncand = w->candmin = w->candmax = 0;
+  w->ticket = 0;
+}
+
+constexpr int kFirstShift = 21;       // top-k: bins are the key's top 11 bits
+constexpr float kStepsPerUnit = 64.f;  // top-p alone: bins are steps of max - s
+constexpr int kFinishTopK = 4096;     // largest top-k whose candidates are expected to fit
+constexpr int kLocalCand = 1024;      // candidates one workgroup collects
+constexpr int kUnroll = 8;            // logits in flight per thread
+static_assert(kSampleBins == 8 * kThreads, "eight bins per thread");
+
+// Bin of a score, larger for larger scores.  LINEAR: 2047 - floor((max - s) * 64), 0 from 32 below the
+// maximum on (whose mass rounds to 0), and for a NaN difference.
+template <bool LINEAR>
+__device__ __forceinline__ uint32_t first_bin(float s, uint32_t key, float mx) {
+  if (!LINEAR) return key >> kFirstShift;
+  const float d = (mx - s) * kStepsPerUnit;
+  return d < (float)(kSampleBins - 1) ? (uint32_t)(kSampleBins - 1) - (uint32_t)(int)fmaxf(d, 0.f) : 0u;
+}
+
+// f(v, logit) for this thread's elements v = v0 + threadIdx.x, + kThreads, .. of [v0, v1), kUnroll
+// loads at a time
+template <class F>
+__device__ __forceinline__ void for_slice(const float* x, int v0, int v1, F&& f) {
+  for (int v = v0 + (int)threadIdx.x; v < v1; v += kThreads * kUnroll) {
+    float l[kUnroll];
+#pragma unroll
+    for (int i = 0; i < kUnroll; i++) l[i] = v + i * kThreads < v1 ? x[v + i * kThreads] : 0.f;
+#pragma unroll
+    for (int i = 0; i < kUnroll; i++)
+      if (v + i * kThreads < v1) f(v + i * kThreads, l[i]);
+  }
+}
+
+// Sum over the threads after this one, of one value each (kThreads of them), and over all in `total`.
+__device__ __forceinline__ unsigned long long block_sum_after(unsigned long long v, unsigned long long& total) {
+  __shared__ unsigned long long ws[kWaves];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  unsigned long long incl = v;  // this lane's and the later ones'
+  for (int o = 1; o < 64; o <<= 1) {
+    const unsigned long long x = __shfl_down(incl, o);
+    if (lane + o < 64) incl += x;
+  }
+  __syncthreads();
+  if (lane == 0) ws[wave] = incl;
+  __syncthreads();
+  unsigned long long after = incl - v;
+  total = 0;
+  for (int q = 0; q < kWaves; q++) {
+    total += ws[q];
+    if (q > wave) after += ws[q];
+  }
+  return after;
+}
+
+// MASS: the masses of the whole row over linear bins (top-p alone); else counts over key bins (top-k).
+// Leaves the threshold's bin in w->prefix, the rank still sought in it (top-k) or the mass above it
+// (top-p) in w->need, and the mass sought in w->target.
+template <bool MASS>
+__global__ void __launch_bounds__(kThreads) k_first(Args a) {
+  typedef typename std::conditional<MASS, unsigned long long, unsigned int>::type bin_t;
+  __shared__ bin_t wh[kSampleBins];
+  __shared__ unsigned int ndig;
+  Block b;
+  if (!setup(a, b)) return;
+  SampleWork* w = b.w;
+  const float T = a.sp.temperature, mx = MASS ? row_max(a, b) : 0.f;
+#pragma unroll
+  for (int i = 0; i < 8; i++) wh[threadIdx.x + kThreads * i] = 0;
+  if (threadIdx.x == 0) ndig = 0;
+  __syncthreads();
+  for_slice(b.x, b.v0, b.v1, [&](int, float l) {
+    const float s = __fdiv_rn(l, T);
+    const bin_t m = MASS ? (bin_t)mass_of(s, mx) : (bin_t)1;
+    if (!MASS || m) atomicAdd(&wh[first_bin<MASS>(s, key32(s), mx)], m);
+  });
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const unsigned long long h = wh[threadIdx.x + kThreads * i];
+    if (h) atomicAdd(&w->hist[threadIdx.x + kThreads * i], h);
+  }
+  if (!last_block(w)) return;
+
+  // suffix sums: this thread holds bins 8t..8t+7.  The bin is the largest d >= 1 whose suffix sum S[d]
+  // reaches what is sought, else 0 (S does not increase with d, so d is the count of such d)
+  const int t = threadIdx.x;
+  unsigned long long h[8], own = 0, total;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    h[i] = load_u64(&w->hist[8 * t + i]);
+    own += h[i];
+  }
+  const unsigned long long after = block_sum_after(own, total);
+  unsigned long long sought = (unsigned long long)a.sp.top_k;
+  if (MASS) {
+    sought = (unsigned long long)((double)a.sp.top_p * (double)total);
+    if (sought < 1) sought = 1;
+  }
+  unsigned long long run = after, above[8];
+  unsigned int n = 0;
+#pragma unroll
+  for (int i = 7; i >= 0; i--) {
+    above[i] = run;  // S[8t + i + 1]
+    run += h[i];
+    n += (8 * t + i >= 1 && run >= sought) ? 1u : 0u;
+    w->hist[8 * t + i] = 0;  // ready for the next call
+  }
+  if (n) atomicAdd(&ndig, n);
+  __syncthreads();
+  const int d = (int)ndig;
+  if (d >> 3 == t) {
+    unsigned long long ab = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) ab = (d & 7) == i ? above[i] : ab;
+    w->prefix = (unsigned int)d;
+    w->need = MASS ? ab : sought - ab;
+    w->target = sought;
+    w->ticket = 0;
+  }
+}
+
+// Whole draw of a filtered call (after k_first): TOPK, TOPP the filters that are on.
+template <bool TOPK, bool TOPP>
+__global__ void __launch_bounds__(kThreads) k_finish(Args a) {
+  constexpr bool LINEAR = !TOPK, BOTH = TOPK && TOPP;
+  __shared__ unsigned long long local[kLocalCand];
+  __shared__ uint32_t ck[kSampleCand];
+  __shared__ unsigned long long hs[128];
+  __shared__ unsigned int nlocal, base, digit;
+  __shared__ unsigned long long s_above;
+  Block b;
+  if (!setup(a, b)) return;
+  SampleWork* w = b.w;
+  const float T = a.sp.temperature;
+  const uint32_t fd = load_u32(&w->prefix);
+  float mx = LINEAR ? row_max(a, b) : 0.f;
+  const uint64_t dbase = draw_base(a.sp.seed, b.counter);
+  if (threadIdx.x == 0) nlocal = 0;
+  __syncthreads();
+  // best: draws of the scores that stay for certain; tied: of the candidates, which all stay if
+  // their keys are the same
+  unsigned long long best = 0, tied = 0;
+  uint32_t kmn = 0xffffffffu, kmx = 0;
+  auto draw = [&](int v, float l) {
+    return ((unsigned long long)gumbel_key(l, T, dbase, v) << 32) | (0xffffffffu - (uint32_t)v);
+  };
+  for_slice(b.x, b.v0, b.v1, [&](int v, float l) {
+    const float s = __fdiv_rn(l, T);
+    const uint32_t k = key32(s), bin = first_bin<LINEAR>(s, k, mx);
+    if (bin < fd) return;
+    if (!BOTH && bin > fd) {
+      const unsigned long long g = draw(v, l);
+      best = g > best ? g : best;
+      return;
+    }
+    kmn = k < kmn ? k : kmn;
+    kmx = k > kmx ? k : kmx;
+    const unsigned long long g = draw(v, l);
+    tied = g > tied ? g : tied;
+    const unsigned int i = atomicAdd(&nlocal, 1u);
+    if (i < (unsigned)kLocalCand) local[i] = ((unsigned long long)k << 32) | (uint32_t)v;
+  });
+  __syncthreads();
+  // more than the workgroup can list: counted as more than the row can
+  if (threadIdx.x == 0 && nlocal) base = atomicAdd(&w->ncand, nlocal <= (unsigned)kLocalCand ? nlocal : (unsigned)kSampleCand + nlocal);
+  auto mx64 = [](unsigned long long p, unsigned long long q) { return p > q ? p : q; };
+  best = block_reduce_u64(best, mx64);
+  __syncthreads();
+  tied = block_reduce_u64(tied, mx64);
+  __syncthreads();
+  const unsigned long long ends = block_reduce_u64(((unsigned long long)(~kmn) << 32), mx64);
+  __syncthreads();
+  kmx = (uint32_t)block_reduce_u64((unsigned long long)kmx, mx64);
+  if (nlocal && nlocal <= (unsigned)kLocalCand)
+    for (unsigned int i = threadIdx.x; i < nlocal; i += kThreads)
+      if (base + i < (unsigned)kSampleCand)
+        __hip_atomic_store(&w->cand[base + i], local[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (threadIdx.x == 0) {
+    if (best) atomicMax(&w->best, best);
+    if (nlocal) {
+      atomicMax(&w->tied, tied);
+      atomicMax(&w->candmin, (unsigned int)(ends >> 32));
+      atomicMax(&w->candmax, kmx);
+    }
+  }
+  if (!last_block(w)) return;
+
+  // ---- the row's last workgroup
+  const unsigned int nc = load_u32(&w->ncand);
+  const bool listed = nc <= (unsigned)kSampleCand;
+  const uint32_t cmin = ~load_u32(&w->candmin), cmax = load_u32(&w->candmax);
+  best = load_u64(&w->best);
+  if (cmin == cmax) {  // one score, however often: it stays
+    const unsigned long long g = load_u64(&w->tied);
+    best = g > best ? g : best;
+  } else {
+    if (listed)
+      for (unsigned int i = threadIdx.x; i < nc; i += kThreads) ck[i] = (uint32_t)(load_u64(&w->cand[i]) >> 32);
+    __syncthreads();
+    // f(key) for every candidate
+    auto each = [&](auto&& f) {
+      if (listed) {
+        for (unsigned int i = threadIdx.x; i < nc; i += kThreads) f(ck[i]);
+      } else {
+        for_slice(b.x, 0, a.V, [&](int, float l) {
+          const float s = __fdiv_rn(l, T);
+          const uint32_t k = key32(s), bin = first_bin<LINEAR>(s, k, mx);
+          if (BOTH ? bin >= fd : bin == fd) f(k);
+        });
+      }
+    };
+    // the largest key with (sum above the prefix +) the sum over candidates >= it reaching `sought`,
+    // among candidates >= kmin that start with `prefix` (bits of `mask`), 7 bits at a time
+    auto descend = [&](bool mass, uint32_t prefix, uint32_t mask, int hi, unsigned long long above,
+                       unsigned long long sought, uint32_t kmin) {
+      while (hi > 0) {
+        const int wd = hi < 7 ? hi : 7, sh = hi - wd;
+        const uint32_t dm = (1u << wd) - 1u;
+        for (int i = threadIdx.x; i < 128; i += kThreads) hs[i] = 0;
+        __syncthreads();
+        each([&](uint32_t k) {
+          if ((k & mask) == prefix && k >= kmin)
+            atomicAdd(&hs[(k >> sh) & dm], mass ? mass_of(from_key32(k), mx) : 1ull);
+        });
+        __syncthreads();
+        if (threadIdx.x < 64) {  // bins 2l, 2l + 1 per lane; suffix sums, then the digit
+          const int lane = threadIdx.x;
+          const unsigned long long h0 = hs[2 * lane], h1 = hs[2 * lane + 1];
+          unsigned long long incl = h0 + h1;
+          for (int o = 1; o < 64; o <<= 1) {
+            const unsigned long long x = __shfl_down(incl, o);
+            if (lane + o < 64) incl += x;
+          }
+          const unsigned long long s0 = above + incl, s1 = above + incl - h0;
+          const unsigned int d = (unsigned)__popcll(__ballot(lane > 0 && s0 >= sought)) +
+                                 (unsigned)__popcll(__ballot(s1 >= sought));
+          if ((int)(d >> 1) == lane) {
+            digit = d;
+            s_above = (d & 1) ? s1 - h1 : s0 - h0;
+          }
+        }
+        __syncthreads();
+        prefix |= digit << sh;
+        mask |= dm << sh;
+        above = s_above;
+        hi = sh;
+        __syncthreads();
+      }
+      return prefix;
+    };
+    uint32_t keep = 0;
+    if (TOPK) {
+      // the rank still sought in the bin: `sought` counts from the bin's top
+      keep = descend(false, fd << kFirstShift, ~0u << kFirstShift, kFirstShift, 0, load_u64(&w->need), 0);
+      if (BOTH) {
+        mx = from_key32(cmax);
+        unsigned long long z = 0;
+        each([&](uint32_t k) {
+          if (k >= keep) z += mass_of(from_key32(k), mx);
+        });
+        z = block_reduce_u64(z, [](unsigned long long p, unsigned long long q) { return p + q; });
+        unsigned long long target = (unsigned long long)((double)a.sp.top_p * (double)z);
+        if (target < 1) target = 1;
+        const uint32_t pmin = descend(true, 0, 0, 32, 0, target, keep);
+        keep = pmin > keep ? pmin : keep;
+      }
+    } else {
+      keep = descend(true, 0, 0, 32, load_u64(&w->need), load_u64(&w->target), 0);
+    }
+    unsigned long long g = 0;
+    if (listed) {
+      for (unsigned int i = threadIdx.x; i < nc; i += kThreads)
+        if (ck[i] >= keep) {
+          const int v = (int)(uint32_t)load_u64(&w->cand[i]);
+          const unsigned long long q = draw(v, b.x[v]);
+          g = q > g ? q : g;
+        }
+    } else {
+      for_slice(b.x, 0, a.V, [&](int v, float l) {
+        const float s = __fdiv_rn(l, T);
+        const uint32_t k = key32(s), bin = first_bin<LINEAR>(s, k, mx);
+        if ((BOTH ? bin >= fd : bin == fd) && k >= keep) {
+          const unsigned long long q = draw(v, l);
+          g = q > g ? q : g;
+        }
+      });
+    }
+    __syncthreads();
+    g = block_reduce_u64(g, mx64);
+    best = g > best ? g : best;
+  }
+  __syncthreads();  // every wave has read the work that put_token clears
+  if (threadIdx.x == 0) put_token(a, b, (int)(0xffffffffu - (uint32_t)best));
+}
+
 // The draw (GREEDY: the first index of the maximum logit); the last workgroup
 // writes the token and clears the row's work for the next call.
 template <bool GREEDY>
@@ -282,20 +598,7 @@ __global__ void __launch_bounds__(kThreads) k_draw(Args a) {
   best = block_reduce_u64(best, [](unsigned long long p, unsigned long long q) { return p > q ? p : q; });
   if (threadIdx.x == 0) atomicMax(&w->best, best);
   if (!last_block(w)) return;
-  if (threadIdx.x == 0) {
-    const int tok = (int)(0xffffffffu - (uint32_t)load_u64(&w->best));
-    if (a.st) {
-      DecodeState* st = a.st;
-      st->tok = tok;
-      if (a.log) a.log[st->step - 1] = tok;
-      st->done = (st->eos >= 0 && tok == st->eos) ? 1u : 0u;
-    } else {
-      a.out[b.row] = tok;
-    }
-    w->z = w->target = w->need = w->best = 0;
-    w->maxkey = w->prefix = w->mask = w->kmin = w->pmin = 0;
-    w->ticket = 0;
-  }
+  if (threadIdx.x == 0) put_token(a, b, (int)(0xffffffffu - (uint32_t)load_u64(&w->best)));
 }
 
 // Workgroups per row: about 128 workgroups in all, at least 8 per row.
@@ -313,7 +616,15 @@ int launch(const Args& a, int rows, hipStream_t stream) {
   } else {
     const bool topk = sp.top_k > 0 && sp.top_k < a.V;
     const bool topp = sp.top_p > 0.f && sp.top_p < 1.f;
-    if (topp && !a.st) hipLaunchKernelGGL(k_max, grid, block, 0, stream, a);
+    if (topp && !a.st && (!topk || sp.top_k > kFinishTopK)) hipLaunchKernelGGL(k_max, grid, block, 0, stream, a);
+    if ((topk || topp) && !(topk && sp.top_k > kFinishTopK)) {
+      if (topk) hipLaunchKernelGGL(k_first<false>, grid, block, 0, stream, a);
+      else hipLaunchKernelGGL(k_first<true>, grid, block, 0, stream, a);
+      if (topk && topp) hipLaunchKernelGGL((k_finish<true, true>), grid, block, 0, stream, a);
+      else if (topk) hipLaunchKernelGGL((k_finish<true, false>), grid, block, 0, stream, a);
+      else hipLaunchKernelGGL((k_finish<false, true>), grid, block, 0, stream, a);
+      return hipGetLastError() == hipSuccess ? QMK_OK : QMK_ERR_HIP;
+    }
     if (topk)
       for (int p = 0; p < sample::kPasses; p++) hipLaunchKernelGGL(k_hist<false>, grid, block, 0, stream, a, p);
     if (topp)
@@ -348,7 +659,8 @@ int stream_work(hipStream_t stream, SampleWork** out) {
 int alloc_sample_work(SampleWork** out, int rows) {
   const size_t bytes = (size_t)rows * sizeof(SampleWork);
   if (hipMalloc(out, bytes) != hipSuccess) return QMK_ERR_HIP;
-  if (hipMemset(*out, 0, bytes) != hipSuccess) {
+  // the fill runs on the null stream: wait for it, since the caller's stream need not
+  if (hipMemset(*out, 0, bytes) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
     (void)hipFree(*out);
     *out = nullptr;
     return QMK_ERR_HIP;
