@@ -107,10 +107,159 @@ __device__ __forceinline__ void block_max2(float (&v)[2], float (*red)[4]) {
 
 // ---------------------------------------------------------------- tokens
 
+// Tiles of the MFMA attention: up to kQT tokens of one sequence at consecutive positions, neighbours in
+// the call.  A run of such tokens (a prompt) is cut into tiles from its own start, so the tiles of one
+// prompt hold no token of the next; tokens past `cap` tiles (hundreds of short runs) and invalid ones
+// are left to the rows at the kernels' end.  (With tiles cut every kQT tokens of the call, those that
+// held two prompts went to attention_rows: four prompts of 411..613 tokens, Qwen3-1.7B, 56 us per
+// layer beside 37 of attention_mfma, now 40 in all.)
+struct AttnPlan {
+  int* hdr;    // {number of tiles, number of left tokens}
+  int2* tile;  // {first token, tokens}, the ones with the most keys first
+  int2* raw;   // the same in token order,
+  int* rank;   // the places of those in `tile`,
+  int* key;    // and their last positions
+  int* where;  // per token: tile * kQT + row, or -1
+  int* left;   // tokens in no tile
+  int cap;     // tiles at most (0: no plan)
+};
+
+// One workgroup of 256 threads, each over T / 256 neighbouring tokens; info(t) = {sequence, position},
+// sequence -1 for an invalid token.
+template <class F>
+__device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& read) {
+  // up to kHeld tokens, everything between the inputs and the plan stays in LDS (2048 tokens: 23 us in
+  // global memory, 17 in LDS, 6 for one run; embedding alone takes 5)
+  constexpr int kHeld = 2048, kTiles = 128;
+  __shared__ int2 held[kHeld], lraw[kTiles];
+  __shared__ int lwhere[kHeld], lrank[kTiles], lkey[kTiles], ws[4], ntiles, nleft;
+  const bool in_lds = T <= kHeld && pl.cap <= kTiles;
+  int2* const raw = in_lds ? lraw : pl.raw;
+  int* const rank = in_lds ? lrank : pl.rank;
+  int* const key = in_lds ? lkey : pl.key;
+  int* const where = in_lds ? lwhere : pl.where;
+  const int th = threadIdx.x, wave = th >> 6, lane = th & 63, per = (T + 255) / 256, a = min(T, th * per),
+            b = min(T, a + per);
+  {  // every load of the thread's tokens before the first use
+    int2 x[kHeld / 256];
+#pragma unroll
+    for (int i = 0; i < kHeld / 256; i++) x[i] = read(min(th + 256 * i, T - 1));
+#pragma unroll
+    for (int i = 0; i < kHeld / 256; i++) held[th + 256 * i] = x[i];
+  }
+  if (th == 0) nleft = 0;
+  __syncthreads();
+  auto info = [&](int t) { return t < kHeld ? held[t] : read(t); };
+  {  // one run (a single prompt): its tiles, the last one first
+    const int2 x0 = info(0);
+    int one = x0.x >= 0;
+    for (int t = th; t < T; t += 256) {
+      const int2 x = info(t);
+      one &= (x.x == x0.x) & (x.y == x0.y + t);
+    }
+    const int nt = (T + kQT - 1) / kQT;
+    if (__syncthreads_and(one) && nt <= pl.cap) {
+      for (int i = th; i < nt; i += 256) pl.tile[nt - 1 - i] = make_int2(i * kQT, min(kQT, T - i * kQT));
+      for (int t = th; t < T; t += 256) pl.where[t] = (nt - 1 - t / kQT) * kQT + t % kQT;
+      if (th == 0) {
+        pl.hdr[0] = nt;
+        pl.hdr[1] = 0;
+      }
+      return;
+    }
+  }
+  auto starts = [&](int t, int2 x) {  // token t (x, valid) does not continue token t - 1's run
+    if (t == 0) return true;
+    const int2 y = info(t - 1);
+    return y.x != x.x || y.y + 1 != x.y;
+  };
+  auto scan = [&](int v, bool sum) {  // exclusive over the threads: sum, or maximum from -1
+    const int none = sum ? 0 : -1;
+    auto op = [&](int x, int y) { return sum ? x + y : max(x, y); };
+    int incl = v;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int x = __shfl_up(incl, o);
+      if (lane >= o) incl = op(incl, x);
+    }
+    const int prev = __shfl_up(incl, 1);
+    if (lane == 63) ws[wave] = incl;
+    __syncthreads();
+    int ex = lane ? prev : none;
+    for (int q = 0; q < wave; q++) ex = op(ex, ws[q]);
+    __syncthreads();
+    return ex;
+  };
+  int last = -1;  // the segment's last run start
+  for (int t = a; t < b; t++) {
+    const int2 x = info(t);
+    if (x.x >= 0 && starts(t, x)) last = t;
+  }
+  const int rs0 = scan(last, false);
+  int rs = rs0, cnt = 0;
+  for (int t = a; t < b; t++) {
+    const int2 x = info(t);
+    if (x.x < 0) continue;
+    if (starts(t, x)) rs = t;
+    cnt += (t - rs) % kQT == 0;
+  }
+  int id = scan(cnt, true) - 1;
+  rs = rs0;
+  for (int t = a; t < b; t++) {
+    const int2 x = info(t);
+    int wh = -1;
+    if (x.x >= 0) {
+      if (starts(t, x)) rs = t;
+      const int row = (t - rs) % kQT;
+      id += row == 0;
+      if (id < pl.cap) {
+        wh = id * kQT + row;
+        if (row == 0) raw[id].x = t;
+        bool end = t + 1 == T || row == kQT - 1;
+        if (!end) {
+          const int2 y = info(t + 1);
+          end = y.x < 0 || starts(t + 1, y);
+        }
+        if (end) {
+          raw[id].y = row + 1;
+          key[id] = x.y;  // the tile's last position
+        }
+      }
+    }
+    where[t] = wh;
+    if (wh < 0) pl.left[atomicAdd(&nleft, 1)] = t;
+  }
+  if (th == 255) ntiles = min(pl.cap, id + 1);  // the last thread's count of tiles is the call's
+  __threadfence_block();
+  __syncthreads();
+  const int nt = ntiles;
+  if (th == 0) {
+    pl.hdr[0] = nt;
+    pl.hdr[1] = nleft;
+  }
+  // the tiles by their last position (keys), largest first, and each token's place among them
+  for (int i = th; i < nt; i += 256) {
+    const int kx = key[i];
+    int r = 0;
+    for (int k = 0; k < nt; k++) {
+      const int ky = key[k];
+      r += ky > kx || (ky == kx && k < i);
+    }
+    pl.tile[r] = raw[i];
+    rank[i] = r;
+  }
+  __threadfence_block();
+  __syncthreads();
+  for (int t = th; t < T; t += 256) {
+    const int wh = where[t];
+    pl.where[t] = wh < 0 ? -1 : rank[wh / kQT] * kQT + wh % kQT;
+  }
+}
+
 // One workgroup per token t: its checked record, X[t] = embed[token], and what the first layer's q/k/v
 // projection needs of it: N[t] = RMSNorm(X[t]) (NORM), or the row's sum of squares for gemm_rows,
-// ssq[t][0] (its other partials 0).  Workgroup 0 also checks the emit rows.  (Token records,
-// embedding and norm as three launches took 4.5 us each.)
+// ssq[t][0] (its other partials 0).  Token 0's also checks the emit rows.  With a plan, a
+// workgroup before them all plans the attention tiles.  (Token records, embedding and norm as three launches took 4.5 us
+// each.)
 template <int H, bool NORM>
 __global__ void __launch_bounds__(256) embed_tokens(const int* __restrict__ tokens, const int* __restrict__ seqs,
                                                     const int* __restrict__ pos, int T, const int* __restrict__ emit,
@@ -118,13 +267,23 @@ __global__ void __launch_bounds__(256) embed_tokens(const int* __restrict__ toke
                                                     const uint16_t* __restrict__ embed, Tok* __restrict__ tok,
                                                     int* __restrict__ erow, uint16_t* __restrict__ X,
                                                     const uint16_t* __restrict__ norm_w, float eps,
-                                                    uint16_t* __restrict__ Nout, float* __restrict__ ssq) {
+                                                    uint16_t* __restrict__ Nout, float* __restrict__ ssq, AttnPlan pl) {
   constexpr int J = H / 256, JW = J / 2;  // elements and bf16 pairs per thread
   typedef unsigned words_t __attribute__((ext_vector_type(JW)));
   __shared__ float red[4];
-  const int t = blockIdx.x, i0 = J * threadIdx.x;
+  const int t = (int)blockIdx.x - (pl.cap ? 1 : 0), i0 = J * threadIdx.x;
+  auto valid = [&](int id, int sq, int p) {
+    return (id >= 0) & (id < vocab) & (sq >= 0) & (sq < num_seqs) & (p >= 0) & (p < max_context);  // no branches
+  };
+  if (t < 0) {
+    plan_attention(T, pl, [&](int u) {
+      const int sq = seqs ? seqs[u] : u, p = pos[u];
+      return make_int2(valid(tokens[u], sq, p) ? sq : -1, p);
+    });
+    return;
+  }
   const int id = tokens[t], sq = seqs ? seqs[t] : t, p = pos[t];
-  const bool ok = id >= 0 && id < vocab && sq >= 0 && sq < num_seqs && p >= 0 && p < max_context;
+  const bool ok = valid(id, sq, p);
   if (threadIdx.x == 0) tok[t] = Tok{ok ? id : 0, ok ? sq : 0, ok ? p : 0, ok ? 1 : 0};
   if (t == 0)
     for (int i = threadIdx.x; i < R; i += 256) {
@@ -721,40 +880,79 @@ __device__ __forceinline__ void attention_row(const uint16_t* __restrict__ Q, co
   dst[threadIdx.x] = (uint16_t)f32_to_bf16(pv_merge_waves(acc, pv));
 }
 
-// One workgroup per (token, KV head), for many tokens (token t = blockIdx.x,
-// blockIdx.x + gridDim.x, ...; a grid narrower than T when attention_mfma ran,
-// so that the workgroups of the tiles it covered cost little: at 2048 tokens
-// a full grid of such exits took 4.9 us).  Contexts longer than kAttnChunk are
-// processed in chunks, recomputing the scores in each of the three passes
-// (max, sum, P@V) instead of keeping them.
+// One workgroup per (token, KV head).  Contexts longer than kAttnChunk are processed in chunks,
+// recomputing the scores in each of the three passes (max, sum, P@V) instead of keeping them.
 __global__ void __launch_bounds__(256) attention_rows(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok,
-                                                      int T, int L, Cache c, float scale, uint16_t* __restrict__ out,
-                                                      const int* __restrict__ redo) {
+                                                      int L, Cache c, float scale, uint16_t* __restrict__ out) {
   __shared__ float sc[2][kAttnChunk];
   __shared__ float red[2][4];
   __shared__ float pv[4][2][kD];
-  const int g = blockIdx.y, t16 = threadIdx.x & 15;
-  for (int t = blockIdx.x; t < T; t += gridDim.x) {
-    if (redo && redo[t / kQT] == 0) continue;  // attention_mfma covered this token's tile
-    __syncthreads();  // the previous token's reads of the shared arrays are done
-    attention_row(Q, tok[t], t, g, t16, L, c, scale, out, sc, red, pv);
-  }
+  const int t = blockIdx.x;
+  attention_row(Q, tok[t], t, blockIdx.y, threadIdx.x & 15, L, c, scale, out, sc, red, pv);
 }
 
-// Prompt prefill attention on MFMA.  Tiles of kQT consecutive tokens; one
-// workgroup of 8 waves per (pair of tiles, query head h): tiles i and nt-1-i
-// (the middle tile alone when nt is odd), one after the other, so that every
-// workgroup's causal work is about the same (the last tile alone has twice
-// the average).  For a tile whose tokens are one sequence at consecutive
-// positions (every prompt prefill) the tile's 64 query rows share each block
+// The attention of one (token, query head) by one wave, without LDS or barriers, for the tokens that
+// are in no tile: HF's two passes, four positions at a time (a lane row of 16 each, 8 dims per lane).
+__device__ __forceinline__ void attention_wave_row(const uint16_t* __restrict__ Q, const Tok tk, int t, int h, int lane,
+                                                   int L, const Cache& c, float scale, uint16_t* __restrict__ out) {
+  const int slot = lane >> 4, t16 = lane & 15;
+  uint16_t* dst = out + (size_t)t * kQS + h * kD + 8 * t16;
+  if (!tk.valid) {
+    if (slot == 0) *reinterpret_cast<u32x4*>(dst) = u32x4{0, 0, 0, 0};
+    return;
+  }
+  const size_t base = cache_base(c, tk, L, h >> 1);
+  const uint16_t* kc = c.k + base + 8 * t16;
+  const uint16_t* vc = c.v + base + 8 * t16;
+  const u32x4 qv = ld16(Q + (size_t)t * kQS + h * kD + 8 * t16);
+  auto score = [&](int p) {  // positions past the token's own load its row; the callers mask them
+    return bf16r(bf16r(row16_sum(dot8(ld16(kc + (size_t)min(p, tk.pos) * kD), qv, 0.f))) * scale);
+  };
+  float m = -INFINITY, l = 0.f;
+  for (int p = slot; p - slot <= tk.pos; p += 4) {
+    const float s = score(p);
+    if (p <= tk.pos) {
+      const float mn = fmaxf(m, s);
+      l = (m == -INFINITY ? 0.f : l * exp_acc(m - mn)) + (s == -INFINITY ? 0.f : exp_acc(s - mn));
+      m = mn;
+    }
+  }
+  const float M = wave_max_all(m);
+  const float inv = __fdiv_rn(1.0f, rows_sum4(m == -INFINITY ? 0.f : l * exp_acc(m - M)));
+  float acc[8];
+#pragma unroll
+  for (int e = 0; e < 8; e++) acc[e] = 0.f;
+  for (int p = slot; p - slot <= tk.pos; p += 4) {
+    const float s = score(p);
+    if (p <= tk.pos) {
+      const float pr = bf16r(exp_acc(s - M) * inv);
+      const u32x4 v = ld16(vc + (size_t)p * kD);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        acc[2 * e] = __builtin_fmaf(pr, lo_bf16(v[e]), acc[2 * e]);
+        acc[2 * e + 1] = __builtin_fmaf(pr, hi_bf16(v[e]), acc[2 * e + 1]);
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; e++) acc[e] = rows_sum4(acc[e]);
+  if (slot == 0)
+    *reinterpret_cast<u32x4*>(dst) = u32x4{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]),
+                                           pack_bf16x2(acc[4], acc[5]), pack_bf16x2(acc[6], acc[7])};
+}
+
+// Prompt prefill attention on MFMA.  Tiles of up to kQT consecutive tokens of a sequence (AttnPlan);
+// workgroups of 8 waves, 256 / 16 of them per query head h (one per CU: it holds 163 registers), share
+// a head's tiles so that each has about the same keys to walk (the last tile of a prompt alone has
+// twice
+// the average).  The tile's 64 query rows share each block
 // of kKB cached keys and values, staged through LDS.  Two passes over the keys,
 // as HF's eager softmax: pass 1 gives each row's max M and sum L of exp(s - M)
 // (online per lane over the blocks, then across lanes and the two waves of a
 // row group); pass 2 recomputes the scores, rounds the probabilities
 // bf16(exp(s - M) / L) and multiplies them with V on MFMA.  Scores are
-// bf16(bf16(q.k) * scale), as in attention_rows.  A tile that is not one such
-// run (several sequences, an invalid token) is marked in redo[tile] and left to
-// attention_rows.
+// bf16(bf16(q.k) * scale), as in attention_rows.  The tokens that are in no tile are taken
+// one wave per (token, head) after the tiles.
 //
 // MFMA 16x16x32 bf16 layout: lane l supplies A[l%16][8(l/16)..+7] and
 // B[8(l/16)..+7][l%16] and receives C[4(l/16)+i][l%16].  Wave w owns query rows
@@ -776,7 +974,7 @@ __device__ __forceinline__ int attn_v_slot(int q) {
   return 32 * half + 8 * ((r & 15) >> 2) + 4 * (r >> 4) + (r & 3);
 }
 
-// Modes: kAttnFull (kernel attention_mfma) runs both passes over a tile's whole context (pairs of
+// Modes: kAttnFull (kernel attention_mfma) runs both passes over a tile's whole context (several
 // tiles per workgroup, as above).  For few tiles over a long context the keys are split into chunks
 // of ck blocks, one workgroup per (tile, chunk, query head): kAttnPass1 (attention_mfma_pass1)
 // writes each row's (max, sum) of its chunk to ml; kAttnPass2 (attention_mfma_pass2) takes every
@@ -793,7 +991,7 @@ __device__ __forceinline__ size_t attn_chunk_row(int tile, int h, int nch, int c
 template <int MODE>
 __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int T,
                                                     int L, Cache c, float scale, uint16_t* __restrict__ out,
-                                                    int* __restrict__ redo, int nch, int ck, float2* __restrict__ ml,
+                                                    const AttnPlan& pl, int nch, int ck, float2* __restrict__ ml,
                                                     float* __restrict__ part) {
   constexpr int NT = kAttnWaves * 64;
   static_assert(kQT == 64 && kKB == 64 && kAttnWaves == 8, "4 row groups of 16 x 2 key halves of 32");
@@ -802,40 +1000,32 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
   constexpr int kKBytes = kKB * kKPad * 2, kVBytes = kD * kVPad * 2, kRedBytes = 4 * 16 * kD * 4;
   static_assert(kKBytes + kVBytes >= kRedBytes, "the partials fit in the K/V buffers");
   __shared__ __align__(16) unsigned char smem[kKBytes + kVBytes];
-  __shared__ int s_ok[2];
   auto Ks = reinterpret_cast<uint16_t(*)[kKPad]>(smem);
   auto Vt = reinterpret_cast<uint16_t(*)[kVPad]>(smem + kKBytes);
   auto Vw = reinterpret_cast<uint32_t(*)[kVPad / 2]>(smem + kKBytes);  // the same rows as 32-bit words
   auto red = reinterpret_cast<float(*)[16][kD]>(smem);
   __shared__ float s_ml[4][2][16][2];  // (max, sum) per row group, key half and row
-  const int nt = (T + kQT - 1) / kQT;
+  const int nt = pl.hdr[0];
   const int h = blockIdx.y, g = h >> 1;
   // the wave index made uniform, so that branches on the wave's rows and keys are scalar
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15,
             lg = lane >> 4;
   const int rg = w >> 1, kh = w & 1;  // rows 16rg..16rg+15, keys 32kh..32kh+31 of each block
-  // kAttnFull: the pair (i, nt - 1 - i); the split passes: tile blockIdx.x / nch, chunk blockIdx.x % nch
-  const int tiles[2] = {MODE == kAttnFull ? (int)blockIdx.x : (int)blockIdx.x / nch,
-                        MODE == kAttnFull ? nt - 1 - (int)blockIdx.x : (int)blockIdx.x / nch};
+  // the split passes: tile blockIdx.x / nch, chunk blockIdx.x % nch.  kAttnFull: of the tiles in order of
+  // their keys, workgroup b of S takes b, 2S - 1 - b, 2S + b, 4S - 1 - b, ..
   const int chunk = MODE == kAttnFull ? 0 : (int)blockIdx.x % nch;
-  const int ntile = tiles[1] == tiles[0] ? 1 : 2;
-  // which of the pair's tiles are one sequence at consecutive positions
-  if (threadIdx.x < 2) s_ok[threadIdx.x] = 1;
-  __syncthreads();
-  for (int u = 0; u < ntile; u++) {
-    const int t0 = tiles[u] * kQT, nrows = min(kQT, T - t0);
-    if ((int)threadIdx.x < nrows) {
-      const Tok first = tok[t0], tk = tok[t0 + threadIdx.x];
-      if (!tk.valid || tk.seq != first.seq || tk.pos != first.pos + (int)threadIdx.x) s_ok[u] = 0;
+  const int S = gridDim.x;
+  for (int u = 0;; u++) {
+    int ti = (int)blockIdx.x / nch;
+    if constexpr (MODE == kAttnFull) {
+      ti = u * S + (u & 1 ? S - 1 - (int)blockIdx.x : (int)blockIdx.x);
+      if (u * S >= nt) break;
+    } else if (u) {
+      break;
     }
-  }
-  __syncthreads();
-  if (MODE != kAttnPass2 && h == 0 && chunk == 0 && threadIdx.x < (unsigned)ntile)
-    redo[tiles[threadIdx.x]] = s_ok[threadIdx.x] ? 0 : 1;
-
-  for (int u = 0; u < ntile; u++) {
-    if (!s_ok[u]) continue;  // uniform over the workgroup
-    const int t0 = tiles[u] * kQT, nrows = min(kQT, T - t0);
+    if (ti >= nt) continue;  // uniform over the workgroup
+    const int2 tl = pl.tile[ti];
+    const int t0 = __builtin_amdgcn_readfirstlane(tl.x), nrows = __builtin_amdgcn_readfirstlane(tl.y);
     const Tok first = tok[t0];
     const int pos0 = __builtin_amdgcn_readfirstlane(first.pos), pmax = pos0 + nrows - 1;
     const size_t base = cache_base(c, first, L, g);
@@ -852,7 +1042,7 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
     const int nkb = (pmax + kKB) / kKB;         // blocks covering positions 0..pmax
     // this workgroup's blocks: all of them, or its chunk's (none past the tile's last key)
     const int kb0 = MODE == kAttnFull ? 0 : chunk * ck, kb1 = MODE == kAttnFull ? nkb : min(kb0 + ck, nkb);
-    if (kb0 >= kb1) continue;  // uniform over the workgroup
+    if (kb0 >= kb1) continue;  // uniform over the workgroup (a chunk past the tile's keys)
     // Block kb: positions kb*kKB + pr; rows past pmax load row pmax (masked below).  Each
     // thread carries kCh 16-byte chunks of K (and of V): block kb+1 is requested into registers
     // before block kb's MFMAs, so its memory latency overlaps them, and written to LDS after
@@ -992,7 +1182,7 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
       const float sm = (m0 == -INFINITY ? 0.f : l0 * exp_acc(m0 - gm)) + (m1 == -INFINITY ? 0.f : l1 * exp_acc(m1 - gm));
       if constexpr (MODE == kAttnPass1) {
         // the chunk's (max, sum) of row 16rg + l16 (-inf, 0 when every key of the chunk follows it)
-        if (kh == 0 && lg == 0) ml[attn_chunk_row(tiles[u], h, nch, chunk, 16 * rg + l16)] = make_float2(gm, sm);
+        if (kh == 0 && lg == 0) ml[attn_chunk_row(ti, h, nch, chunk, 16 * rg + l16)] = make_float2(gm, sm);
         continue;
       }
       ginv = __fdiv_rn(1.0f, sm);
@@ -1003,7 +1193,7 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
       const int nc = (nkb + ck - 1) / ck, row = 16 * rg + l16;
       float2* const s_cml = reinterpret_cast<float2*>(smem);  // [nc][kQT]
       static_assert(kMaxAttnChunks * kQT * sizeof(float2) <= kKBytes + kVBytes, "the chunks' pairs fit in LDS");
-      for (int i = threadIdx.x; i < nc * kQT; i += NT) s_cml[i] = ml[attn_chunk_row(tiles[u], h, nch, i / kQT, i % kQT)];
+      for (int i = threadIdx.x; i < nc * kQT; i += NT) s_cml[i] = ml[attn_chunk_row(ti, h, nch, i / kQT, i % kQT)];
       __syncthreads();
       float mx = -INFINITY;
       for (int q = 0; q < nc; q++) mx = fmaxf(mx, s_cml[q * kQT + row].x);
@@ -1093,7 +1283,7 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
             for (int j = 0; j < 8; j++)
               dst[16 * j + l16] = (uint16_t)f32_to_bf16(acc[j][i] + red[rg][4 * lg + i][16 * j + l16]);
           } else {  // this chunk's fp32 partial of the row
-            float* dst = part + attn_chunk_row(tiles[u], h, nch, chunk, r) * kD;
+            float* dst = part + attn_chunk_row(ti, h, nch, chunk, r) * kD;
 #pragma unroll
             for (int j = 0; j < 8; j++) dst[16 * j + l16] = acc[j][i] + red[rg][4 * lg + i][16 * j + l16];
           }
@@ -1101,43 +1291,51 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
       }
     }
   }
+  if constexpr (MODE != kAttnPass2) {
+    const int nleft = pl.hdr[1], step = gridDim.x * kAttnWaves;
+    for (int i = blockIdx.x * kAttnWaves + w; i < nleft; i += step) {
+      const int t = __builtin_amdgcn_readfirstlane(pl.left[i]);
+      attention_wave_row(Q, tok[t], t, h, lane, L, c, scale, out);
+    }
+  }
 }
 
 #define QMK_ATTN_ARGS                                                                                      \
   const uint16_t *__restrict__ Q, const Tok *__restrict__ tok, int T, int L, Cache c, float scale,                 \
-      uint16_t *__restrict__ out, int *__restrict__ redo, int nch, int ck, float2 *__restrict__ ml,                 \
+      uint16_t *__restrict__ out, AttnPlan pl, int nch, int ck, float2 *__restrict__ ml,                 \
       float *__restrict__ part
 // The pairs, the first pass over key chunks and the second.  (Held to 128 registers, for two
 // workgroups of the second pass per CU, it spilled 18 and ran slower: 32 tokens after 7,000
 // positions 2.57-2.63 against 2.39-2.44 ms per prefill.)
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma(QMK_ATTN_ARGS) {
-  attention_mfma_body<kAttnFull>(Q, tok, T, L, c, scale, out, redo, nch, ck, ml, part);
+  attention_mfma_body<kAttnFull>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
 }
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_pass1(QMK_ATTN_ARGS) {
-  attention_mfma_body<kAttnPass1>(Q, tok, T, L, c, scale, out, redo, nch, ck, ml, part);
+  attention_mfma_body<kAttnPass1>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
 }
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_pass2(QMK_ATTN_ARGS) {
-  attention_mfma_body<kAttnPass2>(Q, tok, T, L, c, scale, out, redo, nch, ck, ml, part);
+  attention_mfma_body<kAttnPass2>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
 }
 #undef QMK_ATTN_ARGS
 
-// The split passes' output: each row of a tile attention_mfma covered (redo 0) is the sum of its
-// chunks' partials in chunk order, rounded to bf16.  One workgroup of kD threads per (token, query
-// head).
-__global__ void __launch_bounds__(kD) attention_mfma_merge(const Tok* __restrict__ tok, int T, int nch, int ck,
-                                                          const float* __restrict__ part,
-                                                          const int* __restrict__ redo, uint16_t* __restrict__ out) {
+// The split passes' output: each row of a tile is the sum of its chunks' partials in chunk order,
+// rounded to bf16.  One workgroup of kD threads per (token, query head).
+__global__ void __launch_bounds__(kD) attention_mfma_merge(const Tok* __restrict__ tok, int nch, int ck,
+                                                          const float* __restrict__ part, AttnPlan pl,
+                                                          uint16_t* __restrict__ out) {
   const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-  const int tile = t / kQT, t0 = tile * kQT, nrows = min(kQT, T - t0);
-  if (redo[tile]) return;
-  const int pmax = tok[t0].pos + nrows - 1;
+  const int wh = pl.where[t];
+  if (wh < 0) return;  // written by the first pass
+  const int tile = wh / kQT, row = wh % kQT;
+  const int2 tl = pl.tile[tile];
+  const int pmax = tok[tl.x].pos + tl.y - 1;
   const int nc = ((pmax + kKB) / kKB + ck - 1) / ck;
   // eight chunks' loads in flight at a time, added in chunk order
   float y = 0.f;
   for (int q0 = 0; q0 < nc; q0 += 8) {
     float v[8];
 #pragma unroll
-    for (int j = 0; j < 8; j++) v[j] = q0 + j < nc ? part[attn_chunk_row(tile, h, nch, q0 + j, t - t0) * kD + d] : 0.f;
+    for (int j = 0; j < 8; j++) v[j] = q0 + j < nc ? part[attn_chunk_row(tile, h, nch, q0 + j, row) * kD + d] : 0.f;
 #pragma unroll
     for (int j = 0; j < 8; j++)
       if (q0 + j < nc) y += v[j];
@@ -2006,17 +2204,28 @@ bool mfma_attention(int T, int max_context, bool one_per_seq) {
 struct AttnSplit {
   int nch, ck;
 };
-AttnSplit attn_mfma_split(int T, int max_context) {
-  const int nt = (T + kQT - 1) / kQT, nkb = (max_context + kKB - 1) / kKB;
-  if ((nt + 1) / 2 * kNQ >= kNumWG || (max_context < 2 * T && nt > 8)) return {1, nkb};
-  const int nch = std::min((nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks) / nt, nkb / 2);
+// tile chunks at most, over all tiles of the plan (0: the pairs)
+int attn_tile_chunks(int T, int max_context) {
+  const int nt = (T + kQT - 1) / kQT;
+  if ((nt + 1) / 2 * kNQ >= kNumWG || (max_context < 2 * T && nt > 8)) return 0;
+  return nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks;
+}
+AttnSplit attn_mfma_split(int T, int max_context, int tiles) {
+  const int nkb = (max_context + kKB - 1) / kKB;
+  const int nch = std::min(attn_tile_chunks(T, max_context) / tiles, nkb / 2);
   if (nch < 2) return {1, nkb};
   const int ck = (nkb + nch - 1) / nch;
   return {(nkb + ck - 1) / ck, ck};
 }
 
+// Tiles planned for a call: each sequence's run may end in a part tile, up to kMoreTiles of them.
+constexpr int kMoreTiles = 63;
+int attn_tiles(int T, int num_seqs) {
+  return std::min(T, (T + kQT - 1) / kQT + std::min(num_seqs - 1, kMoreTiles));
+}
+
 struct Layout {
-  size_t tok, erow, keys, x, n, q, att, m, qkv, ssq, part, scores, ml, pv, redo, mml, mpart, total;
+  size_t tok, erow, keys, x, n, q, att, m, qkv, ssq, part, scores, ml, pv, plan, mml, mpart, total;
 };
 
 template <class M>
@@ -2054,12 +2263,14 @@ Layout layout(int T, int R, int max_context, bool one_per_seq) {
     pf = std::max(pf, part_floats(T, Dm::H, Dm::I));
     take(l.part, pf * 4);
   }
-  take(l.redo, (size_t)((T + kQT - 1) / kQT) * 4);
-  const AttnSplit sp = attn_mfma_split(T, max_context);
-  if (mfma_attention(T, max_context, one_per_seq) && sp.nch > 1) {  // attention_mfma's chunks: (max, sum), partials
-    const size_t rows = (size_t)((T + kQT - 1) / kQT) * kNQ * sp.nch * kQT;
-    take(l.mml, rows * sizeof(float2));
-    take(l.mpart, rows * kD * 4);
+  if (mfma_attention(T, max_context, one_per_seq)) {
+    // header, tiles twice with their ranks and keys, where, left; then the tile chunks' (max, sum) and partials
+    take(l.plan, 16 + (size_t)attn_tiles(T, kMoreTiles + 1) * 24 + (size_t)T * 8);
+    const size_t rows = (size_t)attn_tile_chunks(T, max_context) * kNQ * kQT;
+    if (rows) {
+      take(l.mml, rows * sizeof(float2));
+      take(l.mpart, rows * kD * 4);
+    }
   }
   l.total = off;
   return l;
@@ -2170,8 +2381,20 @@ void launch_attn_chunks(const Args& a, const AttnChunks& ac, const uint16_t* src
   hipLaunchKernelGGL(attn_chunk_merge, dim3(a.T, kNQ), dim3(256), 0, s, tok, ac.nch, ac.pvp, out);
 }
 
+// The attention plan of a call (cap 0 when its attention takes no tiles); embed_tokens fills it.
+AttnPlan attn_plan(const Args& a, const Layout& l) {
+  if (!mfma_attention(a.T, a.max_context, a.one_per_seq)) return AttnPlan{};
+  const int cap = attn_tiles(a.T, a.num_seqs);
+  int* hdr = reinterpret_cast<int*>(a.ws + l.plan);
+  const int most = attn_tiles(a.T, kMoreTiles + 1);
+  int2* tile = reinterpret_cast<int2*>(hdr + 4);
+  int* rank = reinterpret_cast<int*>(tile + 2 * most);
+  int* where = rank + 2 * most;
+  return {hdr, tile, tile + most, rank, rank + most, where, where + a.T, cap};
+}
+
 // The attention of one layer whose q rows are finished and K/V appended: the context-split form, the
-// MFMA form (and the row kernel for the tiles that it leaves), or the row kernel.
+// MFMA form, or the row kernel.
 void launch_attention(const Args& a, const Layout& l, const uint16_t* Q, const Tok* tok, int L,
                       const LDGLayerWeights& w, float eps, uint16_t* ATT, hipStream_t s) {
   const int T = a.T;
@@ -2180,30 +2403,24 @@ void launch_attention(const Args& a, const Layout& l, const uint16_t* Q, const T
     return;
   }
   if (!mfma_attention(T, a.max_context, a.one_per_seq)) {
-    hipLaunchKernelGGL(attention_rows, dim3(T, kNKV), dim3(256), 0, s, Q, tok, T, L, a.cache, a.attn_scale, ATT, nullptr);
+    hipLaunchKernelGGL(attention_rows, dim3(T, kNKV), dim3(256), 0, s, Q, tok, L, a.cache, a.attn_scale, ATT);
     return;
   }
-  // tiles of one sequence's consecutive tokens on MFMA; any other tile row by row
-  const AttnSplit asp = attn_mfma_split(T, a.max_context);
-  int* redo = reinterpret_cast<int*>(a.ws + l.redo);
-  const int ntiles = (T + kQT - 1) / kQT;
+  const AttnPlan pl = attn_plan(a, l);
+  const AttnSplit asp = attn_mfma_split(T, a.max_context, pl.cap);
   if (asp.nch > 1) {
     float2* aml = reinterpret_cast<float2*>(a.ws + l.mml);
     float* apart = reinterpret_cast<float*>(a.ws + l.mpart);
-    const dim3 grid(ntiles * asp.nch, kNQ);
+    const dim3 grid(pl.cap * asp.nch, kNQ);
     hipLaunchKernelGGL(attention_mfma_pass1, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache,
-                       a.attn_scale, ATT, redo, asp.nch, asp.ck, aml, apart);
+                       a.attn_scale, ATT, pl, asp.nch, asp.ck, aml, apart);
     hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache,
-                       a.attn_scale, ATT, redo, asp.nch, asp.ck, aml, apart);
-    hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, tok, T, asp.nch, asp.ck, apart, redo,
-                       ATT);
+                       a.attn_scale, ATT, pl, asp.nch, asp.ck, aml, apart);
+    hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, tok, asp.nch, asp.ck, apart, pl, ATT);
   } else {
-    hipLaunchKernelGGL(attention_mfma, dim3((ntiles + 1) / 2, kNQ), dim3(kAttnWaves * 64), 0, s, Q,
-                       tok, T, L, a.cache, a.attn_scale, ATT, redo, 1, 0, nullptr, nullptr);
+    hipLaunchKernelGGL(attention_mfma, dim3(std::min(pl.cap, kNumWG / kNQ), kNQ), dim3(kAttnWaves * 64), 0, s, Q,
+                       tok, T, L, a.cache, a.attn_scale, ATT, pl, 1, 0, nullptr, nullptr);
   }
-  // the tiles attention_mfma left (redo) row by row: 256 x 8 workgroups loop over the tokens
-  hipLaunchKernelGGL(attention_rows, dim3(std::min(T, 256), kNKV), dim3(256), 0, s, Q, tok, T, L, a.cache,
-                     a.attn_scale, ATT, redo);
 }
 
 template <class M>
@@ -2223,8 +2440,9 @@ int forward_rows(const Args& a, hipStream_t s) {
   float* ssq = reinterpret_cast<float*>(a.ws + l.ssq);
   const float eps = 1e-6f;
   auto u16 = [](const void* p) { return static_cast<const uint16_t*>(p); };
-  hipLaunchKernelGGL((embed_tokens<Dm::H, false>), dim3(T), dim3(256), 0, s, a.tokens, a.seqs, a.pos, T, a.emit, R,
-                     a.num_seqs, a.max_context, Dm::V, a.embed, tok, erow, X, nullptr, eps, nullptr, ssq);
+  const AttnPlan pl = attn_plan(a, l);
+  hipLaunchKernelGGL((embed_tokens<Dm::H, false>), dim3(T + (pl.cap ? 1 : 0)), dim3(256), 0, s, a.tokens, a.seqs, a.pos,
+                     T, a.emit, R, a.num_seqs, a.max_context, Dm::V, a.embed, tok, erow, X, nullptr, eps, nullptr, ssq, pl);
   for (int L = 0; L < a.num_layers; L++) {
     const LDGLayerWeights& w = a.layers[L];
     const Seg qkv{{u16(w.q_proj_weight), u16(w.k_proj_weight), u16(w.v_proj_weight)}, {kQS, kNKV * kD, kNKV * kD}};
@@ -2270,9 +2488,10 @@ int forward(const Args& a, hipStream_t s) {
   auto u16 = [](const void* p) { return static_cast<const uint16_t*>(p); };
   int ks = 1;
 
-  hipLaunchKernelGGL((embed_tokens<Dm::H, true>), dim3(T), dim3(256), 0, s, a.tokens, a.seqs, a.pos, T, a.emit, R,
-                     a.num_seqs, a.max_context, Dm::V, a.embed, tok, erow, X, u16(a.layers[0].input_layernorm_weight),
-                     eps, N, nullptr);
+  const AttnPlan pl = attn_plan(a, l);
+  hipLaunchKernelGGL((embed_tokens<Dm::H, true>), dim3(T + (pl.cap ? 1 : 0)), dim3(256), 0, s, a.tokens, a.seqs, a.pos,
+                     T, a.emit, R, a.num_seqs, a.max_context, Dm::V, a.embed, tok, erow, X,
+                     u16(a.layers[0].input_layernorm_weight), eps, N, nullptr, pl);
   for (int L = 0; L < a.num_layers; L++) {
     const LDGLayerWeights& w = a.layers[L];
     const Seg qkv{{u16(w.q_proj_weight), u16(w.k_proj_weight), u16(w.v_proj_weight)}, {kQS, kNKV * kD, kNKV * kD}};

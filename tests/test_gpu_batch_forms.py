@@ -134,3 +134,60 @@ def test_prompt_row_tiles(request, model, n):
     ref = oracle_steps(orc, dec._k_cache, dec._v_cache, start, ids)
     print(check_rows(Tally(f"{model} {n} rows"), ref, out.cpu().tolist(), logits.cpu(), bar=LITERAL))
     check_kv_rows(f"{model} {n} rows", orc, dec._k_cache, dec._v_cache, start, n)
+
+
+@pytest.mark.parametrize("order", ["interleaved", "ragged", "after-context", "many-short-runs"])
+def test_attention_tiles_of_several_sequences(shape, exact06, weights_gpu, order):
+    """The MFMA attention's tiles over a call of several sequences, 2 layers, every sequence's last rows
+    against the oracle: prompts whose tiles end inside the call, tokens in no tile (two sequences token by
+    token: one run each; 130 runs of which the plan holds 71), an invalid token inside a prompt, and the
+    same over key chunks after a context."""
+    from qwen_megakernel.model import BatchDecoder
+    from qwen_megakernel.weights import make_prompt
+
+    V, layers, S = 151936, 2, 1408
+    start = 900 if order == "after-context" else 0
+    lens = {"interleaved": (170, 170), "ragged": (65, 1, 190, 130), "after-context": (70, 33),
+            "many-short-runs": (3,) * 130}[order]
+    bd = BatchDecoder(weights=weights_gpu, batch_size=len(lens), max_seq_len=S, num_layers=layers, verbose=False)
+    bd._k_cache.fill_(float("nan"))
+    bd._v_cache.fill_(float("nan"))
+    if start:
+        for b in range(len(lens)):
+            bd._forward(*_one(make_prompt(start, V, seed=50 + b), b), bd._k_cache, bd._v_cache, start)
+    prompts = [make_prompt(n, V, seed=90 + b) for b, n in enumerate(lens)]
+    toks = [(b, i) for b, n in enumerate(lens) for i in range(n)]
+    if order == "interleaved":
+        toks.sort(key=lambda x: (x[1], x[0]))
+    ids, seqs, pos = [prompts[b][i] for b, i in toks], [b for b, _ in toks], [start + i for _, i in toks]
+    bad = len(toks) // 2 if order == "ragged" else None
+    if bad is not None:  # an invalid token splits its prompt's run
+        ids.insert(bad, V + 7), seqs.insert(bad, seqs[bad]), pos.insert(bad, 0)
+        toks.insert(bad, (-1, -1))
+    want = sorted(set(toks.index((b, i)) for b, n in enumerate(lens) if b % 20 == 0 or len(lens) < 10
+                      for i in (0, n // 2, n - 1)))
+    out = torch.empty(len(want), dtype=torch.int32, device="cuda")
+    logits = torch.empty(len(want), V, dtype=torch.float32, device="cuda")
+    bd._forward(_t(ids), _t(seqs), _t(pos), _t(want), out, logits, bd._k_cache, bd._v_cache, start + max(lens))
+    assert torch.isfinite(logits).all()
+    t = Tally(f"{order} tiles")
+    for b in sorted(set(toks[w][0] for w in want)):
+        mine = [k for k, w in enumerate(want) if toks[w][0] == b]
+        n = start + lens[b]
+        kc, vc = (torch.zeros_like(x[b]) for x in (bd._k_cache, bd._v_cache))
+        kc[:, :, :n], vc[:, :, :n] = bd._k_cache[b, :, :, :n], bd._v_cache[b, :, :, :n]
+        orc = exact_oracle(exact06, shape, S, num_layers=layers)
+        ref = oracle_steps(orc, kc, vc, start, prompts[b], emit=[toks[want[k]][1] for k in mine])
+        check_rows(t, ref, [int(out[k]) for k in mine], logits[mine].cpu(), bar=LITERAL)
+    print(t)
+
+
+def _t(values):
+    return torch.tensor([int(v) for v in values], dtype=torch.int32, device="cuda")
+
+
+def _one(ids, seq):
+    """Arguments of a forward of one whole prompt from position 0 that emits its last row."""
+    n = len(ids)
+    return (_t(ids), _t([seq] * n), _t(range(n)), _t([n - 1]), torch.empty(1, dtype=torch.int32, device="cuda"),
+            torch.empty(1, 151936, dtype=torch.float32, device="cuda"))
