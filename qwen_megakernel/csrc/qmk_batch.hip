@@ -40,7 +40,8 @@ namespace batch {
 
 constexpr int kD = 128, kNQ = 16, kNKV = 8, kQS = kNQ * kD, kNQKV = (kNQ + 2 * kNKV) * kD;
 constexpr int kAttnChunk = 2048;  // one-kernel attention: scores of this many positions per LDS pass
-constexpr int kQT = 64, kKB = 64, kKPad = kD + 8, kVPad = kKB + 8;  // MFMA prefill attention tiles
+constexpr int kQT = 64;  // MFMA prefill attention: tokens per tile
+constexpr int kKB = 64, kKPad = kD + 8, kVPad = kKB + 8;  // its split passes: keys per block, LDS rows
 constexpr int kMfmaAttnTokens = 320;   // prompts of this many tokens run attention_mfma
 constexpr int kMfmaAttnContext = 256;  // so do fewer tokens over this many positions of context
 constexpr int kMaxAttnChunks = 16;    // attention_mfma over key chunks: tiles x chunks at most
@@ -941,31 +942,297 @@ __device__ __forceinline__ void attention_wave_row(const uint16_t* __restrict__ 
                                            pack_bf16x2(acc[4], acc[5]), pack_bf16x2(acc[6], acc[7])};
 }
 
-// Prompt prefill attention on MFMA.  Tiles of up to kQT consecutive tokens of a sequence (AttnPlan);
-// workgroups of 8 waves, 256 / 16 of them per query head h (one per CU: it holds 163 registers), share
-// a head's tiles so that each has about the same keys to walk (the last tile of a prompt alone has
-// twice
-// the average).  The tile's 64 query rows share each block
-// of kKB cached keys and values, staged through LDS.  Two passes over the keys,
-// as HF's eager softmax: pass 1 gives each row's max M and sum L of exp(s - M)
-// (online per lane over the blocks, then across lanes and the two waves of a
-// row group); pass 2 recomputes the scores, rounds the probabilities
-// bf16(exp(s - M) / L) and multiplies them with V on MFMA.  Scores are
-// bf16(bf16(q.k) * scale), as in attention_rows.  The tokens that are in no tile are taken
-// one wave per (token, head) after the tiles.
+// Prompt prefill attention on MFMA, over tiles of up to kQT consecutive tokens of a sequence (AttnPlan).
+// A tile's query rows of one head share each block of cached keys and values, staged through LDS.  Two
+// passes over the keys, as HF's eager softmax: pass 1 gives each row's max M and sum L of exp(s - M)
+// (online per lane over the blocks, then across lanes and the waves of a row group); pass 2
+// recomputes the scores, rounds the probabilities bf16(exp(s - M) / L) and multiplies them with V on
+// MFMA.  Scores are bf16(bf16(q.k) * scale), as in attention_rows.  The tokens that are in no tile are
+// taken one wave per (token, head) after the tiles.
 //
-// MFMA 16x16x32 bf16 layout: lane l supplies A[l%16][8(l/16)..+7] and
-// B[8(l/16)..+7][l%16] and receives C[4(l/16)+i][l%16].  Wave w owns query rows
-// 16(w/2)..+15 of the tile and keys 32(w%2)..+31 of every block (two waves per
-// row group, each with half of the keys).  Scores are computed transposed (A =
-// 16 keys' K rows, B = the rows' q), so lane (l16, lg) holds row l16's scores of
-// keys 16n + 4lg + i, i = 0..3: every lane carries one query row.  P@V takes A =
-// those probabilities straight from the registers: the 8 k-slots 8lg..8lg+7 of
-// a 32-key step are keys 4lg..4lg+3 and 16+4lg..16+4lg+3 of the wave's half
-// block, and V is stored transposed in LDS in that slot order (B = V^T rows,
-// 16 contiguous bytes per lane).  The two waves of a row group add their P@V
-// partials through LDS at the end (in a fixed order).
+// MFMA 16x16x32 bf16 layout: lane l supplies A[l%16][8(l/16)..+7] and B[8(l/16)..+7][l%16] and receives
+// C[4(l/16)+i][l%16].  A wave owns 16 query rows of the tile and 32 keys of every block.  Scores are
+// computed transposed (A = 16 keys' K rows, B = the rows' q), so lane (l16, lg) holds row l16's scores
+// of keys 16n + 4lg + i, i = 0..3: every lane carries one query row.  P@V takes A = those
+// probabilities straight from the registers: the 8 k-slots 8lg..8lg+7 of a 32-key step are keys
+// 4lg..4lg+3 and 16+4lg..16+4lg+3 of the wave's keys, and V's operand has to come in that order.  The
+// waves of a row group add their P@V partials through LDS at the end (in a fixed order).
+//
+// The kernels share that plan.  attention_mfma walks each tile's whole context: 16 workgroups of 16 waves
+// per head (one per CU) share the head's tiles, in order of their keys, so that each walks about as many
+// (the last tile of a prompt alone has twice the average).  Where that leaves CUs idle, few tiles over
+// a long context, the keys are split into chunks (attention_mfma_pass1, _pass2, _merge below).
+
+// Transposed LDS read (gfx950): 16 lanes read four rows of 16 columns (bf16), 8 bytes each, and lane i
+// receives the four rows' values of column i
+__device__ __forceinline__ uint2 lds_read_tr4(const unsigned char* p) {
+  typedef short short4_t __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) short4_t* lds_t;
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_t)p));
+}
+
+// Blocks of 128 keys, four waves per row group, K and V straight from global memory into LDS: V stays
+// row-major there and is transposed by the reads.  What bounds it is the latency of a block's chain
+// (LDS reads, products, about 100 VALU instructions and 8 exponentials per wave and pass, barrier):
+// VALU work fills 49 % of the cycles, the MFMAs 14 %.  With blocks of 64 keys and 8 waves (two per
+// SIMD, staged through registers, V transposed on the way into LDS) it was 42 %.  Per 4-layer
+// forward, Qwen3-0.6B, us: 768 tokens 459 -> 448, 1024 529 -> 510, 2048 845 -> 805-821.  Measured on the
+// way: 8 waves and two workgroups per CU 85 us per layer at 2048 tokens, 8 waves and four stages 92,
+// this form with the heads in the grid's second dimension 80, as it is 76.
+__global__ void __launch_bounds__(1024) attention_mfma(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int L, Cache c,
+                                                       float scale, uint16_t* __restrict__ out, AttnPlan pl) {
+  constexpr int KQ = 4, NW = 4 * KQ, KB = 32 * KQ;  // key parts of a block, waves, keys per block
+  static_assert(kNQ == 16 && kNKV == 8, "two query heads per KV head and XCD");
+  static_assert(kQT == 64, "4 row groups of 16 x KQ key parts of 32");
+  // two stages of a K block and a V block, [KB][kD] each; after the passes the same bytes hold the P@V
+  // partials of all key parts but the first [KQ - 1][4 row groups][16 rows][kD] fp32 for the first
+  // part's waves to add
+  constexpr int kBlk = KB * kD * 2, kStage = 2 * kBlk;
+  static_assert(2 * kStage >= (KQ - 1) * 4 * 16 * kD * 4, "the partials fit in the stages");
+  __shared__ __align__(1024) unsigned char smem[2 * kStage];
+  __shared__ float s_ml[4][KQ][16][2];  // (max, sum) per row group, key part and row
+  auto red = reinterpret_cast<float(*)[4][16][kD]>(smem);
+  const int nt = pl.hdr[0];
+  // workgroups go to the eight XCDs in turn, so those of KV head g (query heads 2g, 2g+1) share XCD g's
+  // L2: its K and V, read by every tile, stay there (with the heads in the grid's second dimension each
+  // XCD read all of them)
+  const int h = (((int)blockIdx.x & 7) << 1) | ((int)blockIdx.x >> 3), g = h >> 1, by = blockIdx.y;
+  // the wave index made uniform, so that branches on the wave's rows and keys are scalar
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15,
+            lg = lane >> 4;
+  const int rg = w / KQ, kh = w % KQ;  // rows 16rg..16rg+15, keys 32kh..32kh+31 of each block
+  // of the tiles in order of their keys, workgroup by of S takes by, 2S - 1 - by, 2S + by, 4S - 1 - by, ..
+  const int S = gridDim.y;
+  for (int u = 0; u * S < nt; u++) {
+    const int ti = u * S + (u & 1 ? S - 1 - by : by);
+    if (ti >= nt) continue;  // uniform over the workgroup
+    const int2 tl = pl.tile[ti];
+    const int t0 = __builtin_amdgcn_readfirstlane(tl.x), nrows = __builtin_amdgcn_readfirstlane(tl.y);
+    const Tok first = tok[t0];
+    const int pos0 = __builtin_amdgcn_readfirstlane(first.pos), pmax = pos0 + nrows - 1;
+    const size_t base = cache_base(c, first, L, g);
+    const uint16_t* kc = c.k + base;
+    const uint16_t* vc = c.v + base;
+    const int rpos = pos0 + 16 * rg + l16;      // this lane's row position
+    const int wave_first = pos0 + 16 * rg;      // the wave's smallest row position
+    const int wave_last = pos0 + 16 * rg + 15;  // the wave's largest row position
+    const int nkb = (pmax + KB) / KB;         // blocks covering positions 0..pmax
+    // Block kb: positions kb*KB + r; rows past pmax repeat row pmax (masked below).  Wave w moves rows
+    // 8w..8w+7 straight into LDS, four rows (1 KB) per instruction; lane l fills position l % 16 of
+    // row l / 16.  K: 16-byte chunk c of row r at position c ^ (r & 7), so the lanes that read one chunk
+    // of 8 consecutive rows meet every bank once.  V: the 32-byte pairs of chunks at pair ^ (r & 7),
+    // for the transposed reads, which take 32 bytes of 8 consecutive rows per 32 lanes.
+    const int drow = 8 * w + lg;  // and + 4
+    auto issue = [&](int kb, int st, bool v) {
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        const int r = drow + 4 * q;
+        const size_t row = (size_t)min(kb * KB + r, pmax) * kD;
+        unsigned char* dst = smem + st * kStage + (8 * w + 4 * q) * (kD * 2);
+        dma16(kc + row + 8 * (l16 ^ (r & 7)), dst);
+        if (v) dma16(vc + row + 8 * ((((l16 >> 1) ^ (r & 7)) << 1) | (l16 & 1)), dst + kBlk);
+      }
+    };
+    // the blocks in the order in which they are used, those of pass 1, then those of pass 2, each
+    // requested while the one before it is at hand
+    auto request = [&](int it) {
+      if (it < 2 * nkb) issue(it < nkb ? it : it - nkb, it & 1, it >= nkb);
+    };
+    request(0);
+    // B operands: this lane's query row (rows past the tile's tokens repeat its last one)
+    const int tq = t0 + min(16 * rg + l16, nrows - 1);
+    bf16x8 qb[4];
+#pragma unroll
+    for (int kk = 0; kk < 4; kk++) qb[kk] = ld_bf16x8(Q + (size_t)tq * kQS + h * kD + 32 * kk + 8 * lg);
+    // raw q.k of row l16 with keys kb*KB + 32kh + 16n + 4lg + i
+    auto tile_scores = [&](int st, int n) {
+      const unsigned char* kr = smem + st * kStage + (32 * kh + 16 * n + l16) * (kD * 2);
+      f32x4 sc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kk = 0; kk < 4; kk++)
+        sc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+            *reinterpret_cast<const bf16x8*>(kr + 16 * ((4 * kk + lg) ^ (l16 & 7))), qb[kk], sc, 0, 0, 0);
+      return sc;
+    };
+    // the four scores bf16(bf16(q.k) * scale), two roundings per conversion; no branch per
+    // element (the callers mask by select), so the four chains interleave
+    auto scaled = [&](const f32x4& sc, float (&x)[4]) {
+      const uint32_t r01 = pack_bf16x2(sc[0], sc[1]), r23 = pack_bf16x2(sc[2], sc[3]);
+      const uint32_t s01 = pack_bf16x2(lo_bf16(r01) * scale, hi_bf16(r01) * scale);
+      const uint32_t s23 = pack_bf16x2(lo_bf16(r23) * scale, hi_bf16(r23) * scale);
+      x[0] = lo_bf16(s01);
+      x[1] = hi_bf16(s01);
+      x[2] = lo_bf16(s23);
+      x[3] = hi_bf16(s23);
+    };
+    int it = 0;  // the block at hand
+    auto walk = [&](auto&& f) {  // f(block, stage) for each block of a pass
+      for (int kb = 0; kb < nkb; kb++, it++) {
+        ring_barrier<0>();  // the block has landed in every wave, and the other stage is read
+        request(it + 1);
+        f(kb, it & 1);
+      }
+    };
+    // ---- pass 1: per lane, online max and sum of exp over its positions (one exp per score,
+    // one rescale per block)
+    float m = -INFINITY, ls = 0.f;
+    walk([&](int kb, int stg) {
+      const int kbase = kb * KB + 32 * kh;
+      if (kbase > wave_last) return;  // every key of the wave's part follows its rows
+      // MASKED: the part reaches the causal diagonal of the wave's rows (the last one or two
+      // blocks of a tile); every earlier key precedes every row, so neither the mask nor the
+      // clamp of exp_acc is needed (exp_finite gives the same values for finite arguments)
+      auto block = [&](auto masked) {
+        constexpr bool MASKED = decltype(masked)::value;
+        float x[2][4];
+        float mb = -INFINITY;
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+          const f32x4 sc = !MASKED || kbase + 16 * n <= wave_last ? tile_scores(stg, n) : f32x4{0.f, 0.f, 0.f, 0.f};
+          scaled(sc, x[n]);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            if constexpr (MASKED) x[n][i] = kbase + 16 * n + 4 * lg + i <= rpos ? x[n][i] : -INFINITY;
+            mb = fmaxf(mb, x[n][i]);
+          }
+        }
+        // no branch: while every key so far is masked for this lane's row (mn = -inf) the terms
+        // are taken against 0, and exp_acc turns -inf into 0, so ls stays 0
+        const float mn = fmaxf(m, mb);
+        const float ref = MASKED && mn == -INFINITY ? 0.f : mn;
+        float e = 0.f;
+#pragma unroll
+        for (int n = 0; n < 2; n++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) e += MASKED ? exp_acc(x[n][i] - ref) : exp_finite(x[n][i] - ref);
+        ls = ls * exp_acc(m - ref) + e;
+        m = mn;
+      };
+      if (kbase + 31 <= wave_first) block(std::false_type{});
+      else block(std::true_type{});
+    });
+    // row l16's (max, sum): over the 4 lanes of equal l16, then the row group's waves (in the
+    // same order in each, so they hold the same M and 1/L)
+    {
+      float mx = m;
+      mx = fmaxf(mx, __shfl_xor(mx, 16));
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      float sm = m == -INFINITY ? 0.f : ls * exp_acc(m - mx);
+      sm += __shfl_xor(sm, 16);
+      sm += __shfl_xor(sm, 32);
+      if (lg == 0) {
+        s_ml[rg][kh][l16][0] = mx;
+        s_ml[rg][kh][l16][1] = sm;
+      }
+    }
+    __syncthreads();
+    float qm[KQ], ql[KQ];
+#pragma unroll
+    for (int q = 0; q < KQ; q++) {
+      qm[q] = s_ml[rg][q][l16][0];
+      ql[q] = s_ml[rg][q][l16][1];
+    }
+    float gm = qm[0];
+#pragma unroll
+    for (int q = 1; q < KQ; q++) gm = fmaxf(gm, qm[q]);
+    float sm = 0.f;
+#pragma unroll
+    for (int q = 0; q < KQ; q++) sm += qm[q] == -INFINITY ? 0.f : ql[q] * exp_acc(qm[q] - gm);
+    const float ginv = __fdiv_rn(1.0f, sm);
+    // ---- pass 2: probabilities (bf16, as HF rounds them) times V
+    f32x4 acc[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    walk([&](int kb, int stg) {
+      const int kbase = kb * KB + 32 * kh;
+      if (kbase > wave_last) return;
+      // A operand: k-slot 4n + i of this lane is key kbase + 16n + 4lg + i of row l16
+      uint32_t pw[4];
+      auto probs = [&](auto masked) {  // MASKED as in pass 1
+        constexpr bool MASKED = decltype(masked)::value;
+#pragma unroll
+        for (int n = 0; n < 2; n++) {
+          // a 16-key tile wholly past the wave's rows is masked for every row: no MFMA for it
+          const f32x4 sc = !MASKED || kbase + 16 * n <= wave_last ? tile_scores(stg, n) : f32x4{0.f, 0.f, 0.f, 0.f};
+          float x[4], pr[4];
+          scaled(sc, x);
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            // the probability bf16(exp(s - M) / L) (rounded once, by the packing below); masked
+            // keys, whose terms may be anything, take 0
+            if constexpr (MASKED) pr[i] = kbase + 16 * n + 4 * lg + i <= rpos ? exp_acc(x[i] - gm) * ginv : 0.f;
+            else pr[i] = exp_finite(x[i] - gm) * ginv;
+          }
+          pw[2 * n] = pack_bf16x2(pr[0], pr[1]);
+          pw[2 * n + 1] = pack_bf16x2(pr[2], pr[3]);
+        }
+      };
+      if (kbase + 31 <= wave_first) probs(std::false_type{});
+      else probs(std::true_type{});
+      const bf16x8 pa = __builtin_bit_cast(bf16x8, u32x4{pw[0], pw[1], pw[2], pw[3]});
+      // B operand: dim 16j + l16 of those keys.  A transposed read gives each lane of a group of 16 four
+      // consecutive rows' values of its own column; lane i of the group points at row i / 4, columns
+      // 4 (i % 4)..+3
+      const int vr = 32 * kh + 4 * lg + (l16 >> 2);
+      const unsigned char* vrow = smem + stg * kStage + kBlk + vr * (kD * 2) + 8 * (l16 & 3);
+#pragma unroll
+      for (int j = 0; j < 8; j++) {
+        const int o = 32 * (j ^ (vr & 7));  // rows vr and vr + 16 swizzle alike
+        const uint2 lo = lds_read_tr4(vrow + o), hi = lds_read_tr4(vrow + o + 16 * kD * 2);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pa, __builtin_bit_cast(bf16x8, u32x4{lo.x, lo.y, hi.x, hi.y}),
+                                                         acc[j], 0, 0, 0);
+      }
+    });
+    // the row group's partials: all but the first wave's through LDS (over the stages), added to the first
+    // wave's in order
+    ring_barrier<0>();
+    if (kh != 0) {
+#pragma unroll
+      for (int j = 0; j < 8; j++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) red[kh - 1][rg][4 * lg + i][16 * j + l16] = acc[j][i];
+    }
+    __syncthreads();
+    if (kh == 0) {
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int r = 16 * rg + 4 * lg + i;
+        if (r < nrows) {
+          uint16_t* dst = out + (size_t)(t0 + r) * kQS + h * kD;
+#pragma unroll
+          for (int j = 0; j < 8; j++) {
+            const int d = 16 * j + l16;
+            float y = acc[j][i];
+#pragma unroll
+            for (int q = 0; q < KQ - 1; q++) y += red[q][rg][4 * lg + i][d];
+            dst[d] = (uint16_t)f32_to_bf16(y);
+          }
+        }
+      }
+    }
+    __syncthreads();  // the partials are read before the next tile's first block
+  }
+  const int nleft = pl.hdr[1], step = S * NW;
+  for (int i = by * NW + w; i < nleft; i += step) {
+    const int t = __builtin_amdgcn_readfirstlane(pl.left[i]);
+    attention_wave_row(Q, tok[t], t, h, lane, L, c, scale, out);
+  }
+}
+
+// Blocks of kKB = 64 keys and workgroups of 8 waves, two per row group.  The split passes take the keys in
+// chunks of ck blocks, one workgroup per (tile, chunk, query head): kAttnPass1 (attention_mfma_pass1)
+// writes each row's (max, sum) of its chunk to ml; kAttnPass2 (attention_mfma_pass2) takes every chunk's
+// (max, sum) of its rows (in chunk order) for the global max M and sum L, and writes its chunk's P@V
+// partial (fp32) to part; attention_mfma_merge adds the partials in chunk order.  Workgroups of chunks
+// past a tile's last key do nothing.  kAttnFull (attention_mfma_short): both passes over a tile's whole
+// context, shared as attention_mfma's, for short contexts.
+// K and V go through two register sets, so that a request has two blocks of compute to land, and V is
+// transposed on its way into LDS.  For few blocks after a cold start that is the better form:
+// attention_mfma's LDS DMA measured, in us per layer, 100 tokens after 6000 positions, pass 1
+// 17.0-19.4 against 14.8, pass 2 22.0-25.3 against 21.0 (two and four stages); four prompts of
+// 411..613 tokens 46 against 40.
 constexpr int kAttnWaves = 8;
+enum AttnMode : int { kAttnFull = 0, kAttnPass1 = 1, kAttnPass2 = 2 };
 
 // LDS slot of key q (0..kKB-1) of a block in the transposed V: the order in
 // which a wave's P@V k-slots take its keys (see above)
@@ -974,22 +1241,13 @@ __device__ __forceinline__ int attn_v_slot(int q) {
   return 32 * half + 8 * ((r & 15) >> 2) + 4 * (r >> 4) + (r & 3);
 }
 
-// Modes: kAttnFull (kernel attention_mfma) runs both passes over a tile's whole context (several
-// tiles per workgroup, as above).  For few tiles over a long context the keys are split into chunks
-// of ck blocks, one workgroup per (tile, chunk, query head): kAttnPass1 (attention_mfma_pass1)
-// writes each row's (max, sum) of its chunk to ml; kAttnPass2 (attention_mfma_pass2) takes every
-// chunk's (max, sum) of its rows (in chunk order) for the global max M and sum L, and writes its
-// chunk's P@V partial (fp32) to part; attention_mfma_merge adds the partials in chunk order.
-// Workgroups of chunks past a tile's last key do nothing.
-enum AttnMode : int { kAttnFull = 0, kAttnPass1 = 1, kAttnPass2 = 2 };
-
 // Index of (tile, head, chunk)'s row block in the split passes' ml and part buffers
 __device__ __forceinline__ size_t attn_chunk_row(int tile, int h, int nch, int chunk, int row) {
   return (((size_t)tile * kNQ + h) * nch + chunk) * kQT + row;
 }
 
 template <int MODE>
-__device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int T,
+__device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int T,
                                                     int L, Cache c, float scale, uint16_t* __restrict__ out,
                                                     const AttnPlan& pl, int nch, int ck, float2* __restrict__ ml,
                                                     float* __restrict__ part) {
@@ -1011,8 +1269,7 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15,
             lg = lane >> 4;
   const int rg = w >> 1, kh = w & 1;  // rows 16rg..16rg+15, keys 32kh..32kh+31 of each block
-  // the split passes: tile blockIdx.x / nch, chunk blockIdx.x % nch.  kAttnFull: of the tiles in order of
-  // their keys, workgroup b of S takes b, 2S - 1 - b, 2S + b, 4S - 1 - b, ..
+  // the split passes: tile blockIdx.x / nch, chunk blockIdx.x % nch; kAttnFull: as attention_mfma
   const int chunk = MODE == kAttnFull ? 0 : (int)blockIdx.x % nch;
   const int S = gridDim.x;
   for (int u = 0;; u++) {
@@ -1302,19 +1559,18 @@ __device__ __forceinline__ void attention_mfma_body(const uint16_t* __restrict__
 
 #define QMK_ATTN_ARGS                                                                                      \
   const uint16_t *__restrict__ Q, const Tok *__restrict__ tok, int T, int L, Cache c, float scale,                 \
-      uint16_t *__restrict__ out, AttnPlan pl, int nch, int ck, float2 *__restrict__ ml,                 \
+      uint16_t *__restrict__ out, AttnPlan pl, int nch, int ck, float2 *__restrict__ ml,                            \
       float *__restrict__ part
-// The pairs, the first pass over key chunks and the second.  (Held to 128 registers, for two
-// workgroups of the second pass per CU, it spilled 18 and ran slower: 32 tokens after 7,000
-// positions 2.57-2.63 against 2.39-2.44 ms per prefill.)
-__global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma(QMK_ATTN_ARGS) {
-  attention_mfma_body<kAttnFull>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
+// (The second pass held to 128 registers, for two workgroups per CU, spilled 18 and ran slower: 32
+// tokens after 7,000 positions 2.57-2.63 against 2.39-2.44 ms per prefill.)
+__global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_short(QMK_ATTN_ARGS) {
+  attention_chunk_body<kAttnFull>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
 }
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_pass1(QMK_ATTN_ARGS) {
-  attention_mfma_body<kAttnPass1>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
+  attention_chunk_body<kAttnPass1>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
 }
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_pass2(QMK_ATTN_ARGS) {
-  attention_mfma_body<kAttnPass2>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
+  attention_chunk_body<kAttnPass2>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
 }
 #undef QMK_ATTN_ARGS
 
@@ -2187,13 +2443,13 @@ bool mfma_attention(int T, int max_context, bool one_per_seq) {
          (T >= kMfmaAttnTokens || max_context >= kMfmaAttnContext);
 }
 
-// attention_mfma's keys in chunks of ck blocks (nch > 1: the split passes) when its tile pairs would
+// attention_mfma's keys in chunks of ck blocks (nch > 1: the split passes) when its tiles would
 // leave CUs idle and either the context before the prompt is at least as long as the prompt (a
 // prompt of few tiles over a long context, e.g. a new turn appended to a long conversation, where
-// each pair's workgroup would walk the whole context alone: Qwen3-0.6B, pairs against chunks, 128
+// each tile's workgroup would walk the whole context alone: Qwen3-0.6B, whole tiles against chunks, 128
 // tokens after 7000 positions 13.9 / 2.8 ms, 32 tokens after 4000 4.82 / 1.90) or the prompt has
 // at most 8 tiles (from position 0: 384 tokens 2.87-2.90 / 2.82-2.83, 512 tokens 3.32-3.36 /
-// 3.24; with more tiles from position 0 the pairs balance the causal work as well: 768 tokens
+// 3.24; with more tiles from position 0 the whole tiles balance the causal work as well: 768 tokens
 // 3.70-3.74 / 3.75-3.76, 1024 tokens 3.97-4.00 / 3.99).
 // Up to 8 tiles, at most kMaxAttnChunks tile chunks, at least two blocks each: 256 workgroups, so
 // the second pass (one workgroup per CU) runs in one round (at most 32: 32 tokens after 7,000
@@ -2201,10 +2457,14 @@ bool mfma_attention(int T, int max_context, bool one_per_seq) {
 // to 4 x kMaxAttnChunks tile chunks, two or more rounds, rather than one chunk each (1024 tokens
 // after 4000 positions 10.76 -> 7.56 ms, after 6000 14.05 -> 9.17).  The fp32 partials (32 KB per
 // tile chunk and head) stay within 32 MB.
+// Up to this context attention_mfma_short's smaller blocks win (us per 4-layer forward, short against
+// the 128-key form: 640 tokens 418 / 416, 768 456 / 452, 1024 526 / 516; four prompts of 411..613 tokens
+// 1283 / 1313).
+constexpr int kShortAttn = 640;
 struct AttnSplit {
   int nch, ck;
 };
-// tile chunks at most, over all tiles of the plan (0: the pairs)
+// tile chunks at most, over all tiles of the plan (0: whole tiles)
 int attn_tile_chunks(int T, int max_context) {
   const int nt = (T + kQT - 1) / kQT;
   if ((nt + 1) / 2 * kNQ >= kNumWG || (max_context < 2 * T && nt > 8)) return 0;
@@ -2417,9 +2677,12 @@ void launch_attention(const Args& a, const Layout& l, const uint16_t* Q, const T
     hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache,
                        a.attn_scale, ATT, pl, asp.nch, asp.ck, aml, apart);
     hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, tok, asp.nch, asp.ck, apart, pl, ATT);
-  } else {
-    hipLaunchKernelGGL(attention_mfma, dim3(std::min(pl.cap, kNumWG / kNQ), kNQ), dim3(kAttnWaves * 64), 0, s, Q,
+  } else if (a.max_context <= kShortAttn) {
+    hipLaunchKernelGGL(attention_mfma_short, dim3(std::min(pl.cap, kNumWG / kNQ), kNQ), dim3(kAttnWaves * 64), 0, s, Q,
                        tok, T, L, a.cache, a.attn_scale, ATT, pl, 1, 0, nullptr, nullptr);
+  } else {
+    hipLaunchKernelGGL(attention_mfma, dim3(kNQ, std::min(pl.cap, kNumWG / kNQ)), dim3(1024), 0, s, Q, tok, L, a.cache,
+                       a.attn_scale, ATT, pl);
   }
 }
 
