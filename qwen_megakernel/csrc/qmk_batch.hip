@@ -2464,18 +2464,21 @@ constexpr int kShortAttn = 640;
 struct AttnSplit {
   int nch, ck;
 };
-// tile chunks at most, over all tiles of the plan (0: whole tiles)
-int attn_tile_chunks(int T, int max_context) {
-  const int nt = (T + kQT - 1) / kQT;
-  if ((nt + 1) / 2 * kNQ >= kNumWG || (max_context < 2 * T && nt > 8)) return 0;
-  return nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks;
-}
 AttnSplit attn_mfma_split(int T, int max_context, int tiles) {
-  const int nkb = (max_context + kKB - 1) / kKB;
-  const int nch = std::min(attn_tile_chunks(T, max_context) / tiles, nkb / 2);
+  const int nt = (T + kQT - 1) / kQT, nkb = (max_context + kKB - 1) / kKB;
+  if ((nt + 1) / 2 * kNQ >= kNumWG || (max_context < 2 * T && nt > 8)) return {1, nkb};
+  int nch = std::min((nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks) / nt, nkb / 2);
+  // part tiles of further sequences share the tile chunks of nt tiles, for which the workspace is sized
+  nch = nch * nt / tiles;
   if (nch < 2) return {1, nkb};
   const int ck = (nkb + nch - 1) / nch;
   return {(nkb + ck - 1) / ck, ck};
+}
+// the most tile chunks that a call may take, whatever its sequences (0: whole tiles)
+int attn_tile_chunks(int T, int max_context) {
+  const int nt = (T + kQT - 1) / kQT, nkb = (max_context + kKB - 1) / kKB;
+  if (attn_mfma_split(T, max_context, nt).nch < 2) return 0;
+  return std::min((nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks) / nt, nkb / 2) * nt;
 }
 
 // Tiles planned for a call: each sequence's run may end in a part tile, up to kMoreTiles of them.
