@@ -16,8 +16,9 @@
 // Per layer above that (kernels in launch order):
 //   gemm_tiled(qkv)    -> qkv_finish (split-K sum, q/k RMSNorm + RoPE, K/V append;
 //                         in the GEMM's epilogue when K is not split)
-//   attention          (one kernel per (token, KV head) for many tokens; a
-//                       context-split pair + merge for few tokens)
+//   attention          (one workgroup per (token, KV head) over short contexts; MFMA
+//                       tiles of each prompt, over key chunks where they are few;
+//                       128-position chunks per token for a batched step)
 //   gemm_tiled(o)      -> residual_norm (residual add, post-attention RMSNorm)
 //   gemm_tiled(g|u)    -> gate_up_finish (SiLU(g) * u; in the GEMM's epilogue when K
 //                         is not split)
