@@ -45,7 +45,7 @@ constexpr int kQT = 64;  // MFMA prefill attention: tokens per tile
 constexpr int kKB = 64, kKPad = kD + 8, kVPad = kKB + 8;  // its split passes: keys per block, LDS rows
 constexpr int kMfmaAttnTokens = 320;   // prompts of this many tokens run attention_mfma
 constexpr int kMfmaAttnContext = 256;  // so do fewer tokens over this many positions of context
-constexpr int kMaxAttnChunks = 16;    // attention_mfma over key chunks: tiles x chunks at most
+constexpr int kMaxAttnChunks = 16;    // split attention_mfma passes: a tile's key chunks at most
 constexpr int kSplitChunk = 128;  // split attention: positions per workgroup
 constexpr int kSplitBelow = 32;   // fewer tokens than this use the split attention ...
 constexpr int kSplitContext = 128;  // ... over more than this many positions of context
@@ -115,16 +115,31 @@ __device__ __forceinline__ void block_max2(float (&v)[2], float (*red)[4]) {
 // are left to the rows at the kernels' end.  (With tiles cut every kQT tokens of the call, those that
 // held two prompts went to attention_rows: four prompts of 411..613 tokens, Qwen3-1.7B, 56 us per
 // layer beside 37 of attention_mfma, now 40 in all.)
+// The split passes' key chunks are planned here too, from the tiles that there are, not from the sequences
+// that the cache could hold (a turn of 100 tokens after 6000 positions in a cache of 8 sequences, 4 layers:
+// 887 us with the chunks shared by the part tiles of all 8, 376 with those of its own two tiles).
 struct AttnPlan {
-  int* hdr;    // {number of tiles, number of left tokens}
-  int2* tile;  // {first token, tokens}, the ones with the most keys first
-  int2* raw;   // the same in token order,
+  int* hdr;    // {number of tiles, number of left tokens, key chunks per tile, blocks per chunk}
+  int4* tile;  // {first token, tokens, its position, sequence}, the ones with the most keys first
+  int2* raw;   // {first token, tokens} in token order,
   int* rank;   // the places of those in `tile`,
   int* key;    // and their last positions
   int* where;  // per token: tile * kQT + row, or -1
   int* left;   // tokens in no tile
   int cap;     // tiles at most (0: no plan)
+  int budget;  // split passes: tile chunks that the partials hold (0: whole tiles)
+  int nkb;     // and blocks of kKB keys that the call's context may have
 };
+
+// Key chunks of each of `tiles` tiles in a call of nt = ceil(T / kQT): its share of the budget, of two
+// blocks or more.  One chunk (more tiles than half the budget): the whole context.
+__host__ __device__ __forceinline__ int2 attn_key_chunks(int budget, int nkb, int nt, int tiles) {
+  int nch = budget / (tiles > nt ? tiles : nt);
+  nch = nch < nkb / 2 ? nch : nkb / 2;
+  nch = nch > 1 ? nch : 1;
+  const int ck = (nkb + nch - 1) / nch;
+  return make_int2((nkb + ck - 1) / ck, ck);
+}
 
 // One workgroup of 256 threads, each over T / 256 neighbouring tokens; info(t) = {sequence, position},
 // sequence -1 for an invalid token.
@@ -150,6 +165,10 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
     for (int i = 0; i < kHeld / 256; i++) held[th + 256 * i] = x[i];
   }
   if (th == 0) nleft = 0;
+  auto header = [&](int tiles, int left) {
+    const int2 kc = attn_key_chunks(pl.budget, pl.nkb, (T + kQT - 1) / kQT, tiles);
+    *reinterpret_cast<int4*>(pl.hdr) = make_int4(tiles, left, kc.x, kc.y);
+  };
   __syncthreads();
   auto info = [&](int t) { return t < kHeld ? held[t] : read(t); };
   {  // one run (a single prompt): its tiles, the last one first
@@ -161,12 +180,10 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
     }
     const int nt = (T + kQT - 1) / kQT;
     if (__syncthreads_and(one) && nt <= pl.cap) {
-      for (int i = th; i < nt; i += 256) pl.tile[nt - 1 - i] = make_int2(i * kQT, min(kQT, T - i * kQT));
+      for (int i = th; i < nt; i += 256)
+        pl.tile[nt - 1 - i] = make_int4(i * kQT, min(kQT, T - i * kQT), x0.y + i * kQT, x0.x);
       for (int t = th; t < T; t += 256) pl.where[t] = (nt - 1 - t / kQT) * kQT + t % kQT;
-      if (th == 0) {
-        pl.hdr[0] = nt;
-        pl.hdr[1] = 0;
-      }
+      if (th == 0) header(nt, 0);
       return;
     }
   }
@@ -234,10 +251,7 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
   __threadfence_block();
   __syncthreads();
   const int nt = ntiles;
-  if (th == 0) {
-    pl.hdr[0] = nt;
-    pl.hdr[1] = nleft;
-  }
+  if (th == 0) header(nt, nleft);
   // the tiles by their last position (keys), largest first, and each token's place among them
   for (int i = th; i < nt; i += 256) {
     const int kx = key[i];
@@ -246,7 +260,8 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
       const int ky = key[k];
       r += ky > kx || (ky == kx && k < i);
     }
-    pl.tile[r] = raw[i];
+    const int2 tl = raw[i], x = info(tl.x);
+    pl.tile[r] = make_int4(tl.x, tl.y, x.y, x.x);
     rank[i] = r;
   }
   __threadfence_block();
@@ -1007,10 +1022,10 @@ __global__ void __launch_bounds__(1024) attention_mfma(const uint16_t* __restric
   for (int u = 0; u * S < nt; u++) {
     const int ti = u * S + (u & 1 ? S - 1 - by : by);
     if (ti >= nt) continue;  // uniform over the workgroup
-    const int2 tl = pl.tile[ti];
+    const int4 tl = pl.tile[ti];
     const int t0 = __builtin_amdgcn_readfirstlane(tl.x), nrows = __builtin_amdgcn_readfirstlane(tl.y);
-    const Tok first = tok[t0];
-    const int pos0 = __builtin_amdgcn_readfirstlane(first.pos), pmax = pos0 + nrows - 1;
+    const int pos0 = __builtin_amdgcn_readfirstlane(tl.z), pmax = pos0 + nrows - 1;
+    const Tok first{0, __builtin_amdgcn_readfirstlane(tl.w), pos0, 1};
     const size_t base = cache_base(c, first, L, g);
     const uint16_t* kc = c.k + base;
     const uint16_t* vc = c.v + base;
@@ -1225,8 +1240,9 @@ __global__ void __launch_bounds__(1024) attention_mfma(const uint16_t* __restric
 // writes each row's (max, sum) of its chunk to ml; kAttnPass2 (attention_mfma_pass2) takes every chunk's
 // (max, sum) of its rows (in chunk order) for the global max M and sum L, and writes its chunk's P@V
 // partial (fp32) to part; attention_mfma_merge adds the partials in chunk order.  Workgroups of chunks
-// past a tile's last key do nothing.  kAttnFull (attention_mfma_short): both passes over a tile's whole
-// context, shared as attention_mfma's, for short contexts.
+// past a tile's last key do nothing.  A call of many part tiles takes one chunk per tile: then the second
+// pass writes the output and the merge does nothing.  kAttnFull (attention_mfma_short): both passes over a
+// tile's whole context, shared as attention_mfma's, for short contexts.
 // K and V go through two register sets, so that a request has two blocks of compute to land, and V is
 // transposed on its way into LDS.  For few blocks after a cold start that is the better form:
 // attention_mfma's LDS DMA measured, in us per layer, 100 tokens after 6000 positions, pass 1
@@ -1248,9 +1264,9 @@ __device__ __forceinline__ size_t attn_chunk_row(int tile, int h, int nch, int c
 }
 
 template <int MODE>
-__device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int T,
+__device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok,
                                                     int L, Cache c, float scale, uint16_t* __restrict__ out,
-                                                    const AttnPlan& pl, int nch, int ck, float2* __restrict__ ml,
+                                                    const AttnPlan& pl, float2* __restrict__ ml,
                                                     float* __restrict__ part) {
   constexpr int NT = kAttnWaves * 64;
   static_assert(kQT == 64 && kKB == 64 && kAttnWaves == 8, "4 row groups of 16 x 2 key halves of 32");
@@ -1264,28 +1280,24 @@ __device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict_
   auto Vw = reinterpret_cast<uint32_t(*)[kVPad / 2]>(smem + kKBytes);  // the same rows as 32-bit words
   auto red = reinterpret_cast<float(*)[16][kD]>(smem);
   __shared__ float s_ml[4][2][16][2];  // (max, sum) per row group, key half and row
-  const int nt = pl.hdr[0];
+  const int4 hdr = *reinterpret_cast<const int4*>(pl.hdr);
+  const int nch = MODE == kAttnFull ? 1 : hdr.z, ck = hdr.w, items = hdr.x * nch;
   const int h = blockIdx.y, g = h >> 1;
   // the wave index made uniform, so that branches on the wave's rows and keys are scalar
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, l16 = lane & 15,
             lg = lane >> 4;
   const int rg = w >> 1, kh = w & 1;  // rows 16rg..16rg+15, keys 32kh..32kh+31 of each block
-  // the split passes: tile blockIdx.x / nch, chunk blockIdx.x % nch; kAttnFull: as attention_mfma
-  const int chunk = MODE == kAttnFull ? 0 : (int)blockIdx.x % nch;
+  // the (tile, chunk) items are shared as attention_mfma's tiles; with several chunks there are no more
+  // of them than workgroups
   const int S = gridDim.x;
-  for (int u = 0;; u++) {
-    int ti = (int)blockIdx.x / nch;
-    if constexpr (MODE == kAttnFull) {
-      ti = u * S + (u & 1 ? S - 1 - (int)blockIdx.x : (int)blockIdx.x);
-      if (u * S >= nt) break;
-    } else if (u) {
-      break;
-    }
-    if (ti >= nt) continue;  // uniform over the workgroup
-    const int2 tl = pl.tile[ti];
+  for (int u = 0; u * S < items; u++) {
+    const int item = u * S + (u & 1 ? S - 1 - (int)blockIdx.x : (int)blockIdx.x);
+    if (item >= items) continue;  // uniform over the workgroup
+    const int ti = item / nch, chunk = item % nch;
+    const int4 tl = pl.tile[ti];
     const int t0 = __builtin_amdgcn_readfirstlane(tl.x), nrows = __builtin_amdgcn_readfirstlane(tl.y);
-    const Tok first = tok[t0];
-    const int pos0 = __builtin_amdgcn_readfirstlane(first.pos), pmax = pos0 + nrows - 1;
+    const int pos0 = __builtin_amdgcn_readfirstlane(tl.z), pmax = pos0 + nrows - 1;
+    const Tok first{0, __builtin_amdgcn_readfirstlane(tl.w), pos0, 1};
     const size_t base = cache_base(c, first, L, g);
     const uint16_t* kc = c.k + base;
     const uint16_t* vc = c.v + base;
@@ -1535,7 +1547,7 @@ __device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict_
       for (int i = 0; i < 4; i++) {
         const int r = 16 * rg + 4 * lg + i;
         if (r < nrows) {
-          if constexpr (MODE == kAttnFull) {
+          if (MODE == kAttnFull || nch == 1) {
             uint16_t* dst = out + (size_t)(t0 + r) * kQS + h * kD;
 #pragma unroll
             for (int j = 0; j < 8; j++)
@@ -1548,9 +1560,10 @@ __device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict_
         }
       }
     }
+    if constexpr (MODE == kAttnPass2) __syncthreads();  // the partials are read before the next item's pairs
   }
   if constexpr (MODE != kAttnPass2) {
-    const int nleft = pl.hdr[1], step = gridDim.x * kAttnWaves;
+    const int nleft = hdr.y, step = gridDim.x * kAttnWaves;
     for (int i = blockIdx.x * kAttnWaves + w; i < nleft; i += step) {
       const int t = __builtin_amdgcn_readfirstlane(pl.left[i]);
       attention_wave_row(Q, tok[t], t, h, lane, L, c, scale, out);
@@ -1559,33 +1572,32 @@ __device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict_
 }
 
 #define QMK_ATTN_ARGS                                                                                      \
-  const uint16_t *__restrict__ Q, const Tok *__restrict__ tok, int T, int L, Cache c, float scale,                 \
-      uint16_t *__restrict__ out, AttnPlan pl, int nch, int ck, float2 *__restrict__ ml,                            \
-      float *__restrict__ part
+  const uint16_t *__restrict__ Q, const Tok *__restrict__ tok, int L, Cache c, float scale,                         \
+      uint16_t *__restrict__ out, AttnPlan pl, float2 *__restrict__ ml, float *__restrict__ part
 // (The second pass held to 128 registers, for two workgroups per CU, spilled 18 and ran slower: 32
 // tokens after 7,000 positions 2.57-2.63 against 2.39-2.44 ms per prefill.)
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_short(QMK_ATTN_ARGS) {
-  attention_chunk_body<kAttnFull>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
+  attention_chunk_body<kAttnFull>(Q, tok, L, c, scale, out, pl, ml, part);
 }
-__global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_pass1(QMK_ATTN_ARGS) {
-  attention_chunk_body<kAttnPass1>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
+// (six waves per SIMD, three workgroups per CU, for calls of more tile chunks than CUs)
+__global__ void __launch_bounds__(kAttnWaves * 64, 6) attention_mfma_pass1(QMK_ATTN_ARGS) {
+  attention_chunk_body<kAttnPass1>(Q, tok, L, c, scale, out, pl, ml, part);
 }
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_pass2(QMK_ATTN_ARGS) {
-  attention_chunk_body<kAttnPass2>(Q, tok, T, L, c, scale, out, pl, nch, ck, ml, part);
+  attention_chunk_body<kAttnPass2>(Q, tok, L, c, scale, out, pl, ml, part);
 }
 #undef QMK_ATTN_ARGS
 
 // The split passes' output: each row of a tile is the sum of its chunks' partials in chunk order,
 // rounded to bf16.  One workgroup of kD threads per (token, query head).
-__global__ void __launch_bounds__(kD) attention_mfma_merge(const Tok* __restrict__ tok, int nch, int ck,
-                                                          const float* __restrict__ part, AttnPlan pl,
+__global__ void __launch_bounds__(kD) attention_mfma_merge(const float* __restrict__ part, AttnPlan pl,
                                                           uint16_t* __restrict__ out) {
   const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
-  const int wh = pl.where[t];
-  if (wh < 0) return;  // written by the first pass
+  const int wh = pl.where[t], nch = pl.hdr[2], ck = pl.hdr[3];
+  if (wh < 0 || nch == 1) return;  // written by the first pass; by the second
   const int tile = wh / kQT, row = wh % kQT;
-  const int2 tl = pl.tile[tile];
-  const int pmax = tok[tl.x].pos + tl.y - 1;
+  const int4 tl = pl.tile[tile];
+  const int pmax = tl.z + tl.y - 1;
   const int nc = ((pmax + kKB) / kKB + ck - 1) / ck;
   // eight chunks' loads in flight at a time, added in chunk order
   float y = 0.f;
@@ -2444,7 +2456,12 @@ bool mfma_attention(int T, int max_context, bool one_per_seq) {
          (T >= kMfmaAttnTokens || max_context >= kMfmaAttnContext);
 }
 
-// attention_mfma's keys in chunks of ck blocks (nch > 1: the split passes) when its tiles would
+// Up to this context attention_mfma_short's smaller blocks win (us per 4-layer forward, short against
+// the 128-key form: 640 tokens 418 / 416, 768 456 / 452, 1024 526 / 516; four prompts of 411..613 tokens
+// 1283 / 1313).
+constexpr int kShortAttn = 640;
+
+// attention_mfma's keys in chunks (the split passes) when its tiles would
 // leave CUs idle and either the context before the prompt is at least as long as the prompt (a
 // prompt of few tiles over a long context, e.g. a new turn appended to a long conversation, where
 // each tile's workgroup would walk the whole context alone: Qwen3-0.6B, whole tiles against chunks, 128
@@ -2457,36 +2474,18 @@ bool mfma_attention(int T, int max_context, bool one_per_seq) {
 // positions 2.39-2.44 against 2.02-2.07 ms per prefill; at most 8: 2.34-2.38).  More tiles take up
 // to 4 x kMaxAttnChunks tile chunks, two or more rounds, rather than one chunk each (1024 tokens
 // after 4000 positions 10.76 -> 7.56 ms, after 6000 14.05 -> 9.17).  The fp32 partials (32 KB per
-// tile chunk and head) stay within 32 MB.
-// Up to this context attention_mfma_short's smaller blocks win (us per 4-layer forward, short against
-// the 128-key form: 640 tokens 418 / 416, 768 456 / 452, 1024 526 / 516; four prompts of 411..613 tokens
-// 1283 / 1313).
-constexpr int kShortAttn = 640;
-struct AttnSplit {
-  int nch, ck;
-};
-AttnSplit attn_mfma_split(int T, int max_context, int tiles) {
+// tile chunk and head) stay within 32 MB.  The result is the call's budget of tile chunks (0: whole tiles);
+// attn_key_chunks shares it among the tiles that the call turns out to have.
+int attn_chunk_budget(int T, int max_context) {
   const int nt = (T + kQT - 1) / kQT, nkb = (max_context + kKB - 1) / kKB;
-  if ((nt + 1) / 2 * kNQ >= kNumWG || (max_context < 2 * T && nt > 8)) return {1, nkb};
-  int nch = std::min((nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks) / nt, nkb / 2);
-  // part tiles of further sequences share the tile chunks of nt tiles, for which the workspace is sized
-  nch = nch * nt / tiles;
-  if (nch < 2) return {1, nkb};
-  const int ck = (nkb + nch - 1) / nch;
-  return {(nkb + ck - 1) / ck, ck};
-}
-// the most tile chunks that a call may take, whatever its sequences (0: whole tiles)
-int attn_tile_chunks(int T, int max_context) {
-  const int nt = (T + kQT - 1) / kQT, nkb = (max_context + kKB - 1) / kKB;
-  if (attn_mfma_split(T, max_context, nt).nch < 2) return 0;
-  return std::min((nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks) / nt, nkb / 2) * nt;
+  if ((nt + 1) / 2 * kNQ >= kNumWG || (max_context < 2 * T && nt > 8)) return 0;
+  const int budget = nt <= 8 ? kMaxAttnChunks : 4 * kMaxAttnChunks;
+  return attn_key_chunks(budget, nkb, nt, nt).x > 1 ? budget : 0;
 }
 
 // Tiles planned for a call: each sequence's run may end in a part tile, up to kMoreTiles of them.
 constexpr int kMoreTiles = 63;
-int attn_tiles(int T, int num_seqs) {
-  return std::min(T, (T + kQT - 1) / kQT + std::min(num_seqs - 1, kMoreTiles));
-}
+int attn_tiles(int T) { return std::min(T, (T + kQT - 1) / kQT + kMoreTiles); }
 
 struct Layout {
   size_t tok, erow, keys, x, n, q, att, m, qkv, ssq, part, scores, ml, pv, plan, mml, mpart, total;
@@ -2528,12 +2527,12 @@ Layout layout(int T, int R, int max_context, bool one_per_seq) {
     take(l.part, pf * 4);
   }
   if (mfma_attention(T, max_context, one_per_seq)) {
-    // header, tiles twice with their ranks and keys, where, left; then the tile chunks' (max, sum) and partials
-    take(l.plan, 16 + (size_t)attn_tiles(T, kMoreTiles + 1) * 24 + (size_t)T * 8);
-    const size_t rows = (size_t)attn_tile_chunks(T, max_context) * kNQ * kQT;
-    if (rows) {
-      take(l.mml, rows * sizeof(float2));
-      take(l.mpart, rows * kD * 4);
+    // header, tiles twice with their ranks and keys, where, left; then the (max, sum) of the tile chunks or,
+    // with one chunk each, of the tiles, and the tile chunks' partials
+    take(l.plan, 16 + (size_t)attn_tiles(T) * 32 + (size_t)T * 8);
+    if (const int budget = attn_chunk_budget(T, max_context)) {
+      take(l.mml, (size_t)std::max(budget, attn_tiles(T)) * kNQ * kQT * sizeof(float2));
+      take(l.mpart, (size_t)budget * kNQ * kQT * kD * 4);
     }
   }
   l.total = off;
@@ -2648,13 +2647,14 @@ void launch_attn_chunks(const Args& a, const AttnChunks& ac, const uint16_t* src
 // The attention plan of a call (cap 0 when its attention takes no tiles); embed_tokens fills it.
 AttnPlan attn_plan(const Args& a, const Layout& l) {
   if (!mfma_attention(a.T, a.max_context, a.one_per_seq)) return AttnPlan{};
-  const int cap = attn_tiles(a.T, a.num_seqs);
+  const int cap = attn_tiles(a.T);
   int* hdr = reinterpret_cast<int*>(a.ws + l.plan);
-  const int most = attn_tiles(a.T, kMoreTiles + 1);
-  int2* tile = reinterpret_cast<int2*>(hdr + 4);
-  int* rank = reinterpret_cast<int*>(tile + 2 * most);
-  int* where = rank + 2 * most;
-  return {hdr, tile, tile + most, rank, rank + most, where, where + a.T, cap};
+  int4* tile = reinterpret_cast<int4*>(hdr + 4);
+  int2* raw = reinterpret_cast<int2*>(tile + cap);
+  int* rank = reinterpret_cast<int*>(raw + cap);
+  int* where = rank + 2 * cap;
+  return {hdr,   tile,        raw, rank, rank + cap,
+          where, where + a.T, cap, attn_chunk_budget(a.T, a.max_context), (a.max_context + kKB - 1) / kKB};
 }
 
 // The attention of one layer whose q rows are finished and K/V appended: the context-split form, the
@@ -2671,19 +2671,18 @@ void launch_attention(const Args& a, const Layout& l, const uint16_t* Q, const T
     return;
   }
   const AttnPlan pl = attn_plan(a, l);
-  const AttnSplit asp = attn_mfma_split(T, a.max_context, pl.cap);
-  if (asp.nch > 1) {
+  if (pl.budget) {
     float2* aml = reinterpret_cast<float2*>(a.ws + l.mml);
     float* apart = reinterpret_cast<float*>(a.ws + l.mpart);
-    const dim3 grid(pl.cap * asp.nch, kNQ);
-    hipLaunchKernelGGL(attention_mfma_pass1, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache,
-                       a.attn_scale, ATT, pl, asp.nch, asp.ck, aml, apart);
-    hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache,
-                       a.attn_scale, ATT, pl, asp.nch, asp.ck, aml, apart);
-    hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, tok, asp.nch, asp.ck, apart, pl, ATT);
+    const dim3 grid(pl.budget, kNQ);
+    hipLaunchKernelGGL(attention_mfma_pass1, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, L, a.cache, a.attn_scale, ATT,
+                       pl, aml, apart);
+    hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, L, a.cache, a.attn_scale, ATT,
+                       pl, aml, apart);
+    hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, apart, pl, ATT);
   } else if (a.max_context <= kShortAttn) {
     hipLaunchKernelGGL(attention_mfma_short, dim3(std::min(pl.cap, kNumWG / kNQ), kNQ), dim3(kAttnWaves * 64), 0, s, Q,
-                       tok, T, L, a.cache, a.attn_scale, ATT, pl, 1, 0, nullptr, nullptr);
+                       tok, L, a.cache, a.attn_scale, ATT, pl, nullptr, nullptr);
   } else {
     hipLaunchKernelGGL(attention_mfma, dim3(kNQ, std::min(pl.cap, kNumWG / kNQ)), dim3(1024), 0, s, Q, tok, L, a.cache,
                        a.attn_scale, ATT, pl);

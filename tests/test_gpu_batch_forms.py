@@ -136,19 +136,38 @@ def test_prompt_row_tiles(request, model, n):
     check_kv_rows(f"{model} {n} rows", orc, dec._k_cache, dec._v_cache, start, n)
 
 
-@pytest.mark.parametrize("order", ["interleaved", "ragged", "after-context", "many-short-runs"])
+@pytest.mark.parametrize("n,start", [(33, 1400), (100, 1300), (600, 700)])
+def test_prompt_does_not_depend_on_the_cache_slots(weights_gpu, n, start):
+    """One prompt after a context, in a cache of one sequence and in the last of 16 (the others empty): the
+    same calls, so the same logits and K/V rows bit for bit (the key chunks are cut for the call's own tiles)."""
+    from qwen_megakernel.model import BatchDecoder
+    from qwen_megakernel.weights import make_prompt
+
+    V, layers, S = 151936, 2, 1536
+    got = []
+    for slots in (1, 16):
+        bd = BatchDecoder(weights=weights_gpu, batch_size=slots, max_seq_len=S, num_layers=layers, verbose=False)
+        bd.prefill(slots - 1, make_prompt(start, V, seed=3))
+        _, logits = bd.prefill(slots - 1, make_prompt(n, V, seed=4), return_logits=True)
+        got.append((logits.cpu(), bd._k_cache[slots - 1].cpu(), bd._v_cache[slots - 1].cpu()))
+    assert torch.isfinite(got[0][0]).all()
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("order", ["interleaved", "ragged", "after-context", "one-chunk-tiles", "many-short-runs"])
 def test_attention_tiles_of_several_sequences(shape, exact06, weights_gpu, order):
     """The MFMA attention's tiles over a call of several sequences, 2 layers, every sequence's last rows
     against the oracle: prompts whose tiles end inside the call, tokens in no tile (two sequences token by
     token: one run each; 130 runs of which the plan holds 71), an invalid token inside a prompt, and the
-    same over key chunks after a context."""
+    same over key chunks after a context, and after one with more tiles than tile chunks (20 runs of 10)."""
     from qwen_megakernel.model import BatchDecoder
     from qwen_megakernel.weights import make_prompt
 
     V, layers, S = 151936, 2, 1408
-    start = 900 if order == "after-context" else 0
+    start = {"after-context": 900, "one-chunk-tiles": 300}.get(order, 0)
     lens = {"interleaved": (170, 170), "ragged": (65, 1, 190, 130), "after-context": (70, 33),
-            "many-short-runs": (3,) * 130}[order]
+            "one-chunk-tiles": (10,) * 20, "many-short-runs": (3,) * 130}[order]
     bd = BatchDecoder(weights=weights_gpu, batch_size=len(lens), max_seq_len=S, num_layers=layers, verbose=False)
     bd._k_cache.fill_(float("nan"))
     bd._v_cache.fill_(float("nan"))
@@ -164,7 +183,7 @@ def test_attention_tiles_of_several_sequences(shape, exact06, weights_gpu, order
     if bad is not None:  # an invalid token splits its prompt's run
         ids.insert(bad, V + 7), seqs.insert(bad, seqs[bad]), pos.insert(bad, 0)
         toks.insert(bad, (-1, -1))
-    want = sorted(set(toks.index((b, i)) for b, n in enumerate(lens) if b % 20 == 0 or len(lens) < 10
+    want = sorted(set(toks.index((b, i)) for b, n in enumerate(lens) if b % 19 == 0 or len(lens) < 10
                       for i in (0, n // 2, n - 1)))
     out = torch.empty(len(want), dtype=torch.int32, device="cuda")
     logits = torch.empty(len(want), V, dtype=torch.float32, device="cuda")
