@@ -43,6 +43,11 @@ constexpr int kD = 128, kNQ = 16, kNKV = 8, kQS = kNQ * kD, kNQKV = (kNQ + 2 * k
 constexpr int kAttnChunk = 2048;  // one-kernel attention: scores of this many positions per LDS pass
 constexpr int kQT = 64;  // MFMA prefill attention: tokens per tile
 constexpr int kKB = 64, kKPad = kD + 8, kVPad = kKB + 8;  // its split passes: keys per block, LDS rows
+// Tokens of the smallest tile, and of the smallest that starts below kQT.  us per 4-layer forward, as tiles
+// against left tokens: 8 runs of 5 after 2000 positions 392 / 476, 12 of 8 after 1500 476 / 546, 40 of 4
+// after 1500 917 / 773, 100 of 12 from position 0 583 / 529.
+constexpr int kMinTile = 5, kMinTileNear = 16;
+constexpr int kLeftWave = 512;  // left tokens below this position may take a wave each
 constexpr int kMfmaAttnTokens = 320;   // prompts of this many tokens run attention_mfma
 constexpr int kMfmaAttnContext = 256;  // so do fewer tokens over this many positions of context
 constexpr int kMaxAttnChunks = 16;    // split attention_mfma passes: a tile's key chunks at most
@@ -111,21 +116,21 @@ __device__ __forceinline__ void block_max2(float (&v)[2], float (*red)[4]) {
 
 // Tiles of the MFMA attention: up to kQT tokens of one sequence at consecutive positions, neighbours in
 // the call.  A run of such tokens (a prompt) is cut into tiles from its own start, so the tiles of one
-// prompt hold no token of the next; tokens past `cap` tiles (hundreds of short runs) and invalid ones
-// are left to the rows at the kernels' end.  (With tiles cut every kQT tokens of the call, those that
+// prompt hold no token of the next.  What would be a tile of fewer than kMinTile tokens is left to the rows
+// at the kernels' end (attention_left), as are tokens past `cap` tiles and invalid ones.  (With tiles cut every kQT tokens of the call, those that
 // held two prompts went to attention_rows: four prompts of 411..613 tokens, Qwen3-1.7B, 56 us per
 // layer beside 37 of attention_mfma, now 40 in all.)
 // The split passes' key chunks are planned here too, from the tiles that there are, not from the sequences
 // that the cache could hold (a turn of 100 tokens after 6000 positions in a cache of 8 sequences, 4 layers:
 // 887 us with the chunks shared by the part tiles of all 8, 376 with those of its own two tiles).
 struct AttnPlan {
-  int* hdr;    // {number of tiles, number of left tokens, key chunks per tile, blocks per chunk}
+  int* hdr;    // {tiles, left tokens, key chunks per tile, blocks per chunk, left tokens past kLeftWave}
   int4* tile;  // {first token, tokens, its position, sequence}, the ones with the most keys first
   int2* raw;   // {first token, tokens} in token order,
   int* rank;   // the places of those in `tile`,
   int* key;    // and their last positions
   int* where;  // per token: tile * kQT + row, or -1
-  int* left;   // tokens in no tile
+  int* left;   // tokens in no tile: those of positions below kLeftWave from the front, others from the back
   int cap;     // tiles at most (0: no plan)
   int budget;  // split passes: tile chunks that the partials hold (0: whole tiles)
   int nkb;     // and blocks of kKB keys that the call's context may have
@@ -147,9 +152,9 @@ template <class F>
 __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& read) {
   // up to kHeld tokens, everything between the inputs and the plan stays in LDS (2048 tokens: 23 us in
   // global memory, 17 in LDS, 6 for one run; embedding alone takes 5)
-  constexpr int kHeld = 2048, kTiles = 128;
+  constexpr int kHeld = 2048, kTiles = 288;
   __shared__ int2 held[kHeld], lraw[kTiles];
-  __shared__ int lwhere[kHeld], lrank[kTiles], lkey[kTiles], ws[4], ntiles, nleft;
+  __shared__ int lwhere[kHeld], lrank[kTiles], lkey[kTiles], ws[4], ntiles, nleft[2];
   const bool in_lds = T <= kHeld && pl.cap <= kTiles;
   int2* const raw = in_lds ? lraw : pl.raw;
   int* const rank = in_lds ? lrank : pl.rank;
@@ -164,10 +169,11 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
 #pragma unroll
     for (int i = 0; i < kHeld / 256; i++) held[th + 256 * i] = x[i];
   }
-  if (th == 0) nleft = 0;
-  auto header = [&](int tiles, int left) {
+  if (th == 0) nleft[0] = nleft[1] = 0;
+  auto header = [&](int tiles, int left, int far) {
     const int2 kc = attn_key_chunks(pl.budget, pl.nkb, (T + kQT - 1) / kQT, tiles);
     *reinterpret_cast<int4*>(pl.hdr) = make_int4(tiles, left, kc.x, kc.y);
+    pl.hdr[4] = far;
   };
   __syncthreads();
   auto info = [&](int t) { return t < kHeld ? held[t] : read(t); };
@@ -183,7 +189,7 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
       for (int i = th; i < nt; i += 256)
         pl.tile[nt - 1 - i] = make_int4(i * kQT, min(kQT, T - i * kQT), x0.y + i * kQT, x0.x);
       for (int t = th; t < T; t += 256) pl.where[t] = (nt - 1 - t / kQT) * kQT + t % kQT;
-      if (th == 0) header(nt, 0);
+      if (th == 0) header(nt, 0, 0);
       return;
     }
   }
@@ -208,6 +214,38 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
     __syncthreads();
     return ex;
   };
+  // each token's end of run: the next token that is invalid or starts a run
+  {
+    int next = -T;  // minus the first such token after the segment (the scans go forward over threads)
+    int mine = -T;
+    for (int t = b - 1; t >= a; t--) {
+      const int2 x = info(t);
+      if (x.x < 0 || starts(t, x)) mine = -t;
+    }
+    // exclusive maximum over the threads after this one
+    int incl = mine;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int x = __shfl_down(incl, o);
+      if (lane + o < 64) incl = max(incl, x);
+    }
+    const int after = __shfl_down(incl, 1);
+    if (lane == 0) ws[wave] = incl;
+    __syncthreads();
+    if (lane < 63) next = after;
+    for (int q = wave + 1; q < 4; q++) next = max(next, ws[q]);
+    __syncthreads();
+    int end = -next;
+    for (int t = b - 1; t >= a; t--) {
+      where[t] = end;
+      const int2 x = info(t);
+      if (x.x < 0 || starts(t, x)) end = t;
+    }
+  }
+  // rows of the tile whose first token is t (0: left)
+  auto tile_rows = [&](int t, int end) {
+    const int n = min(kQT, end - t);
+    return n < (info(t).y < kQT ? kMinTileNear : kMinTile) ? 0 : n;
+  };
   int last = -1;  // the segment's last run start
   for (int t = a; t < b; t++) {
     const int2 x = info(t);
@@ -219,7 +257,7 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
     const int2 x = info(t);
     if (x.x < 0) continue;
     if (starts(t, x)) rs = t;
-    cnt += (t - rs) % kQT == 0;
+    cnt += (t - rs) % kQT == 0 && tile_rows(t, where[t]) > 0;
   }
   int id = scan(cnt, true) - 1;
   rs = rs0;
@@ -228,30 +266,30 @@ __device__ __forceinline__ void plan_attention(int T, const AttnPlan& pl, F&& re
     int wh = -1;
     if (x.x >= 0) {
       if (starts(t, x)) rs = t;
-      const int row = (t - rs) % kQT;
-      id += row == 0;
-      if (id < pl.cap) {
-        wh = id * kQT + row;
-        if (row == 0) raw[id].x = t;
-        bool end = t + 1 == T || row == kQT - 1;
-        if (!end) {
-          const int2 y = info(t + 1);
-          end = y.x < 0 || starts(t + 1, y);
-        }
-        if (end) {
-          raw[id].y = row + 1;
-          key[id] = x.y;  // the tile's last position
+      const int row = (t - rs) % kQT, rows = tile_rows(t - row, where[t]);
+      if (rows) {
+        id += row == 0;
+        if (id < pl.cap) {
+          wh = id * kQT + row;
+          if (row == 0) {
+            raw[id] = make_int2(t, rows);
+            key[id] = x.y + rows - 1;  // the tile's last position
+          }
         }
       }
     }
     where[t] = wh;
-    if (wh < 0) pl.left[atomicAdd(&nleft, 1)] = t;
+    if (wh < 0) {
+      const bool far = x.x >= 0 && x.y >= kLeftWave;
+      const int i = atomicAdd(&nleft[far], 1);
+      pl.left[far ? T - 1 - i : i] = t;
+    }
   }
   if (th == 255) ntiles = min(pl.cap, id + 1);  // the last thread's count of tiles is the call's
   __threadfence_block();
   __syncthreads();
   const int nt = ntiles;
-  if (th == 0) header(nt, nleft);
+  if (th == 0) header(nt, nleft[0] + nleft[1], nleft[1]);
   // the tiles by their last position (keys), largest first, and each token's place among them
   for (int i = th; i < nt; i += 256) {
     const int kx = key[i];
@@ -908,54 +946,198 @@ __global__ void __launch_bounds__(256) attention_rows(const uint16_t* __restrict
   attention_row(Q, tok[t], t, blockIdx.y, threadIdx.x & 15, L, c, scale, out, sc, red, pv);
 }
 
-// The attention of one (token, query head) by one wave, without LDS or barriers, for the tokens that
-// are in no tile: HF's two passes, four positions at a time (a lane row of 16 each, 8 dims per lane).
-__device__ __forceinline__ void attention_wave_row(const uint16_t* __restrict__ Q, const Tok tk, int t, int h, int lane,
-                                                   int L, const Cache& c, float scale, uint16_t* __restrict__ out) {
-  const int slot = lane >> 4, t16 = lane & 15;
-  uint16_t* dst = out + (size_t)t * kQS + h * kD + 8 * t16;
-  if (!tk.valid) {
-    if (slot == 0) *reinterpret_cast<u32x4*>(dst) = u32x4{0, 0, 0, 0};
+// The attention of one token and KV head (both query heads) by NW waves: whole workgroups, or single waves
+// (NW 1).  Both heads' scores of up to CAP positions are in LDS at once; a lane row of 16 takes a position
+// (8 dims per lane), of K and of V, U of them in flight.  HF's two passes: with more than CAP
+// positions the first keeps the running (max, sum) and the second forms the scores again.
+template <int NW, int CAP>
+struct LeftLds {
+  float sc[2][CAP];
+  float pv[NW > 1 ? NW : 0][2][kD];
+  float2 ml[NW > 1 ? NW : 0][2];
+};
+
+template <int NW, int CAP>
+__device__ __forceinline__ void left_row(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int t, int g, int L,
+                                         const Cache& c, float scale, uint16_t* __restrict__ out,
+                                         LeftLds<NW, CAP>& lds) {
+  constexpr int NT = 64 * NW, U = NW > 1 ? 4 : 8, R = 4 * NW;  // threads, rows in flight per lane row, rows per round
+  const int lane = threadIdx.x & 63, slot = lane >> 4, t16 = lane & 15;
+  const int w = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0, tid = NW > 1 ? (int)threadIdx.x : lane;
+  // a wave's own LDS accesses are in order: only the compiler has to keep them so
+  auto sync = [] {
+    if constexpr (NW > 1) __syncthreads();
+    else asm volatile("" ::: "memory");
+  };
+  const Tok tk = tok[t];
+  const int pos = __builtin_amdgcn_readfirstlane(tk.pos);
+  uint16_t* dst = out + (size_t)t * kQS + 2 * g * kD;  // both heads: 256 contiguous values
+  if (!__builtin_amdgcn_readfirstlane(tk.valid)) {
+    if (tid < 64) *reinterpret_cast<uint2*>(dst + 4 * tid) = make_uint2(0, 0);
     return;
   }
-  const size_t base = cache_base(c, tk, L, h >> 1);
+  const size_t base = cache_base(c, tk, L, g);
   const uint16_t* kc = c.k + base + 8 * t16;
   const uint16_t* vc = c.v + base + 8 * t16;
-  const u32x4 qv = ld16(Q + (size_t)t * kQS + h * kD + 8 * t16);
-  auto score = [&](int p) {  // positions past the token's own load its row; the callers mask them
-    return bf16r(bf16r(row16_sum(dot8(ld16(kc + (size_t)min(p, tk.pos) * kD), qv, 0.f))) * scale);
+  u32x4 qv[2];
+#pragma unroll
+  for (int h = 0; h < 2; h++) qv[h] = ld16(Q + (size_t)t * kQS + (2 * g + h) * kD + 8 * t16);
+  const int nch = pos / CAP + 1;
+  // rows p + R j of the chunk from c0 (past the token's position: its own row)
+  auto rows = [&](const uint16_t* x, int c0, int p, u32x4 (&r)[U]) {
+#pragma unroll
+    for (int j = 0; j < U; j++) r[j] = ld16(x + (size_t)min(c0 + p + R * j, pos) * kD);
   };
-  float m = -INFINITY, l = 0.f;
-  for (int p = slot; p - slot <= tk.pos; p += 4) {
-    const float s = score(p);
-    if (p <= tk.pos) {
-      const float mn = fmaxf(m, s);
-      l = (m == -INFINITY ? 0.f : l * exp_acc(m - mn)) + (s == -INFINITY ? 0.f : exp_acc(s - mn));
-      m = mn;
+  auto scores = [&](int c0, int n) {
+    for (int p = 4 * w + slot; p - slot < n; p += R * U) {
+      u32x4 kx[U];
+      rows(kc, c0, p, kx);
+#pragma unroll
+      for (int j = 0; j < U; j++) {
+        const float s0 = row16_sum(dot8(kx[j], qv[0], 0.f)), s1 = row16_sum(dot8(kx[j], qv[1], 0.f));
+        if (t16 < 2 && p + R * j < n) lds.sc[t16][p + R * j] = bf16r(bf16r(t16 ? s1 : s0) * scale);
+      }
+    }
+  };
+  float m[2] = {-INFINITY, -INFINITY}, l[2] = {0.f, 0.f};  // of this thread's positions
+  for (int ch = 0; ch < nch; ch++) {
+    const int c0 = ch * CAP, n = min(pos + 1 - c0, CAP);
+    sync();  // what was in LDS before these scores is read
+    scores(c0, n);
+    sync();
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+      float mx = m[h], e = 0.f;
+      for (int k = tid; k < n; k += NT) mx = fmaxf(mx, lds.sc[h][k]);
+      for (int k = tid; k < n; k += NT) {
+        const float s = lds.sc[h][k];
+        e += s == -INFINITY ? 0.f : exp_acc(s - mx);
+      }
+      l[h] = (m[h] == -INFINITY ? 0.f : l[h] * exp_acc(m[h] - mx)) + e;
+      m[h] = mx;
     }
   }
-  const float M = wave_max_all(m);
-  const float inv = __fdiv_rn(1.0f, rows_sum4(m == -INFINITY ? 0.f : l * exp_acc(m - M)));
-  float acc[8];
+  u32x4 vx[U];
+  rows(vc, 0, 4 * w + slot, vx);  // the first rows of V, behind the reduction
+  float M[2], inv[2];
 #pragma unroll
-  for (int e = 0; e < 8; e++) acc[e] = 0.f;
-  for (int p = slot; p - slot <= tk.pos; p += 4) {
-    const float s = score(p);
-    if (p <= tk.pos) {
-      const float pr = bf16r(exp_acc(s - M) * inv);
-      const u32x4 v = ld16(vc + (size_t)p * kD);
+  for (int h = 0; h < 2; h++) {
+    M[h] = wave_max_all(m[h]);
+    inv[h] = wave_total(m[h] == -INFINITY ? 0.f : l[h] * exp_acc(m[h] - M[h]));
+    if constexpr (NW > 1) {
+      if (lane == 0) lds.ml[w][h] = make_float2(M[h], inv[h]);
+    }
+  }
+  if constexpr (NW > 1) {
+    sync();
 #pragma unroll
-      for (int e = 0; e < 4; e++) {
-        acc[2 * e] = __builtin_fmaf(pr, lo_bf16(v[e]), acc[2 * e]);
-        acc[2 * e + 1] = __builtin_fmaf(pr, hi_bf16(v[e]), acc[2 * e + 1]);
+    for (int h = 0; h < 2; h++) {
+      M[h] = -INFINITY;
+      for (int q = 0; q < NW; q++) M[h] = fmaxf(M[h], lds.ml[q][h].x);
+      inv[h] = 0.f;
+      for (int q = 0; q < NW; q++) {
+        const float2 e = lds.ml[q][h];
+        inv[h] += e.x == -INFINITY ? 0.f : e.y * exp_acc(e.x - M[h]);
       }
     }
   }
 #pragma unroll
-  for (int e = 0; e < 8; e++) acc[e] = rows_sum4(acc[e]);
-  if (slot == 0)
-    *reinterpret_cast<u32x4*>(dst) = u32x4{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]),
-                                           pack_bf16x2(acc[4], acc[5]), pack_bf16x2(acc[6], acc[7])};
+  for (int h = 0; h < 2; h++) inv[h] = __fdiv_rn(1.0f, inv[h]);
+  float acc[2][8];
+#pragma unroll
+  for (int h = 0; h < 2; h++)
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[h][e] = 0.f;
+  for (int ch = 0; ch < nch; ch++) {
+    const int c0 = ch * CAP, n = min(pos + 1 - c0, CAP);
+    if (nch > 1) {
+      sync();
+      scores(c0, n);
+      sync();
+    }
+    for (int k = tid; k < n; k += NT) {
+      lds.sc[0][k] = bf16r(exp_acc(lds.sc[0][k] - M[0]) * inv[0]);
+      lds.sc[1][k] = bf16r(exp_acc(lds.sc[1][k] - M[1]) * inv[1]);
+    }
+    sync();
+    for (int p = 4 * w + slot; p - slot < n; p += R * U) {
+      if (ch || p >= R) rows(vc, c0, p, vx);
+#pragma unroll
+      for (int j = 0; j < U; j++) {
+        // rows past the chunk's positions count as zeros (their row repeats one that may hold an infinity)
+        const bool live = p + R * j < n;
+        const float p0 = live ? lds.sc[0][p + R * j] : 0.f, p1 = live ? lds.sc[1][p + R * j] : 0.f;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+          const uint32_t v = live ? vx[j][e] : 0u;
+          acc[0][2 * e] = __builtin_fmaf(p0, lo_bf16(v), acc[0][2 * e]);
+          acc[0][2 * e + 1] = __builtin_fmaf(p0, hi_bf16(v), acc[0][2 * e + 1]);
+          acc[1][2 * e] = __builtin_fmaf(p1, lo_bf16(v), acc[1][2 * e]);
+          acc[1][2 * e + 1] = __builtin_fmaf(p1, hi_bf16(v), acc[1][2 * e + 1]);
+        }
+      }
+    }
+  }
+  // the wave's four lane rows, then the waves in order
+#pragma unroll
+  for (int h = 0; h < 2; h++) {
+#pragma unroll
+    for (int e = 0; e < 8; e++) acc[h][e] = rows_sum4(acc[h][e]);
+    if (lane < 16) {
+      if constexpr (NW > 1) {
+        *reinterpret_cast<f32x4*>(&lds.pv[w][h][8 * t16]) = f32x4{acc[h][0], acc[h][1], acc[h][2], acc[h][3]};
+        *reinterpret_cast<f32x4*>(&lds.pv[w][h][8 * t16 + 4]) = f32x4{acc[h][4], acc[h][5], acc[h][6], acc[h][7]};
+      } else {
+        *reinterpret_cast<u32x4*>(dst + h * kD + 8 * t16) =
+            u32x4{pack_bf16x2(acc[h][0], acc[h][1]), pack_bf16x2(acc[h][2], acc[h][3]),
+                  pack_bf16x2(acc[h][4], acc[h][5]), pack_bf16x2(acc[h][6], acc[h][7])};
+      }
+    }
+  }
+  if constexpr (NW > 1) {
+    sync();
+    if (threadIdx.x < 2 * kD) {
+      float y = 0.f;
+#pragma unroll
+      for (int q = 0; q < NW; q++) y += (&lds.pv[q][0][0])[threadIdx.x];
+      dst[threadIdx.x] = (uint16_t)f32_to_bf16(y);
+    }
+  }
+}
+
+// The tokens that are in no tile (hdr[1] of them), shared by the NW-wave workgroups of the launch: a
+// workgroup per (token, KV head), but a wave where more than kLeftFew of them lie below kLeftWave (a
+// workgroup's barriers cost more than such a context: 130 runs of 3 tokens from position 0, 475 us by
+// workgroups, 344 by waves; 256 tokens at 100..2000, 56 of them below 512, 1226 and 1303).  The workgroups that
+// take KV head g sit on one XCD, so tokens of one sequence share its L2.
+// Against one wave per (token, query head), four positions at a time, us per 4-layer forward, and against
+// the separate launch of attention_rows that this replaces in turn: 256 sequences' tokens at 100..2000
+// 4220, 1570, now 1226; 400 of a prompt with 100 sequences' tokens at 1000..3000 6030, 2685, 1138; 100 runs
+// of 4 after 300 987, 735, 618; two prompts of 512 token by token 2110, 778, 900, of 200 after 2000 5410,
+// 2590, 1510.
+constexpr int kLeftFew = 128;
+template <int NW, int CAP>
+__device__ __forceinline__ void attention_left(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int T, int L,
+                                               const Cache& c, float scale, uint16_t* __restrict__ out,
+                                               const AttnPlan& pl, unsigned char* smem) {
+  const int nleft = pl.hdr[1], far = pl.hdr[4], near = nleft - far;
+  if (nleft == 0) return;
+  const int wg = blockIdx.x + gridDim.x * blockIdx.y, g = wg & 7, step = gridDim.x * gridDim.y / 8;
+  auto at = [&](int i) { return __builtin_amdgcn_readfirstlane(pl.left[i]); };
+  LeftLds<NW, CAP>& all = *reinterpret_cast<LeftLds<NW, CAP>*>(smem);
+  for (int i = wg >> 3; i < far; i += step) left_row<NW, CAP>(Q, tok, at(T - 1 - i), g, L, c, scale, out, all);
+  if (near <= kLeftFew) {
+    // (from the workgroups that the far ones leave free)
+    for (int i = (wg >> 3) + (step - far % step); i < near + step; i += step) {
+      if (i >= step) left_row<NW, CAP>(Q, tok, at(i - step), g, L, c, scale, out, all);
+    }
+  } else if (near) {
+    __syncthreads();
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    LeftLds<1, kLeftWave>& own = reinterpret_cast<LeftLds<1, kLeftWave>*>(smem)[w];
+    for (int i = (wg >> 3) + step * w; i < near; i += step * NW)
+      left_row<1, kLeftWave>(Q, tok, at(i), g, L, c, scale, out, own);
+  }
 }
 
 // Prompt prefill attention on MFMA, over tiles of up to kQT consecutive tokens of a sequence (AttnPlan).
@@ -963,8 +1145,8 @@ __device__ __forceinline__ void attention_wave_row(const uint16_t* __restrict__ 
 // passes over the keys, as HF's eager softmax: pass 1 gives each row's max M and sum L of exp(s - M)
 // (online per lane over the blocks, then across lanes and the waves of a row group); pass 2
 // recomputes the scores, rounds the probabilities bf16(exp(s - M) / L) and multiplies them with V on
-// MFMA.  Scores are bf16(bf16(q.k) * scale), as in attention_rows.  The tokens that are in no tile are
-// taken one wave per (token, head) after the tiles.
+// MFMA.  Scores are bf16(bf16(q.k) * scale), as in attention_rows.  The tokens that are in no tile follow
+// after the tiles (attention_left).
 //
 // MFMA 16x16x32 bf16 layout: lane l supplies A[l%16][8(l/16)..+7] and B[8(l/16)..+7][l%16] and receives
 // C[4(l/16)+i][l%16].  A wave owns 16 query rows of the tile and 32 keys of every block.  Scores are
@@ -995,8 +1177,8 @@ __device__ __forceinline__ uint2 lds_read_tr4(const unsigned char* p) {
 // forward, Qwen3-0.6B, us: 768 tokens 459 -> 448, 1024 529 -> 510, 2048 845 -> 805-821.  Measured on the
 // way: 8 waves and two workgroups per CU 85 us per layer at 2048 tokens, 8 waves and four stages 92,
 // this form with the heads in the grid's second dimension 80, as it is 76.
-__global__ void __launch_bounds__(1024) attention_mfma(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int L, Cache c,
-                                                       float scale, uint16_t* __restrict__ out, AttnPlan pl) {
+__global__ void __launch_bounds__(1024) attention_mfma(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int T,
+                                                       int L, Cache c, float scale, uint16_t* __restrict__ out, AttnPlan pl) {
   constexpr int KQ = 4, NW = 4 * KQ, KB = 32 * KQ;  // key parts of a block, waves, keys per block
   static_assert(kNQ == 16 && kNKV == 8, "two query heads per KV head and XCD");
   static_assert(kQT == 64, "4 row groups of 16 x KQ key parts of 32");
@@ -1228,11 +1410,9 @@ __global__ void __launch_bounds__(1024) attention_mfma(const uint16_t* __restric
     }
     __syncthreads();  // the partials are read before the next tile's first block
   }
-  const int nleft = pl.hdr[1], step = S * NW;
-  for (int i = by * NW + w; i < nleft; i += step) {
-    const int t = __builtin_amdgcn_readfirstlane(pl.left[i]);
-    attention_wave_row(Q, tok[t], t, h, lane, L, c, scale, out);
-  }
+  static_assert(sizeof(LeftLds<NW, 8192>) <= sizeof(smem) && NW * sizeof(LeftLds<1, kLeftWave>) <= sizeof(smem),
+                "the left tokens' arrays fit in the stages");
+  attention_left<NW, 8192>(Q, tok, T, L, c, scale, out, pl, smem);
 }
 
 // Blocks of kKB = 64 keys and workgroups of 8 waves, two per row group.  The split passes take the keys in
@@ -1264,7 +1444,7 @@ __device__ __forceinline__ size_t attn_chunk_row(int tile, int h, int nch, int c
 }
 
 template <int MODE>
-__device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok,
+__device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok, int T,
                                                     int L, Cache c, float scale, uint16_t* __restrict__ out,
                                                     const AttnPlan& pl, float2* __restrict__ ml,
                                                     float* __restrict__ part) {
@@ -1562,29 +1742,28 @@ __device__ __forceinline__ void attention_chunk_body(const uint16_t* __restrict_
     }
     if constexpr (MODE == kAttnPass2) __syncthreads();  // the partials are read before the next item's pairs
   }
-  if constexpr (MODE != kAttnPass2) {
-    const int nleft = hdr.y, step = gridDim.x * kAttnWaves;
-    for (int i = blockIdx.x * kAttnWaves + w; i < nleft; i += step) {
-      const int t = __builtin_amdgcn_readfirstlane(pl.left[i]);
-      attention_wave_row(Q, tok[t], t, h, lane, L, c, scale, out);
-    }
+  if constexpr (MODE != kAttnPass1) {
+    static_assert(sizeof(LeftLds<kAttnWaves, 3328>) <= sizeof(smem) &&
+                      kAttnWaves * sizeof(LeftLds<1, kLeftWave>) <= sizeof(smem),
+                  "the left tokens' arrays fit in the K/V buffers");
+    attention_left<kAttnWaves, 3328>(Q, tok, T, L, c, scale, out, pl, smem);
   }
 }
 
 #define QMK_ATTN_ARGS                                                                                      \
-  const uint16_t *__restrict__ Q, const Tok *__restrict__ tok, int L, Cache c, float scale,                         \
+  const uint16_t *__restrict__ Q, const Tok *__restrict__ tok, int T, int L, Cache c, float scale,                  \
       uint16_t *__restrict__ out, AttnPlan pl, float2 *__restrict__ ml, float *__restrict__ part
 // (The second pass held to 128 registers, for two workgroups per CU, spilled 18 and ran slower: 32
 // tokens after 7,000 positions 2.57-2.63 against 2.39-2.44 ms per prefill.)
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_short(QMK_ATTN_ARGS) {
-  attention_chunk_body<kAttnFull>(Q, tok, L, c, scale, out, pl, ml, part);
+  attention_chunk_body<kAttnFull>(Q, tok, T, L, c, scale, out, pl, ml, part);
 }
 // (six waves per SIMD, three workgroups per CU, for calls of more tile chunks than CUs)
 __global__ void __launch_bounds__(kAttnWaves * 64, 6) attention_mfma_pass1(QMK_ATTN_ARGS) {
-  attention_chunk_body<kAttnPass1>(Q, tok, L, c, scale, out, pl, ml, part);
+  attention_chunk_body<kAttnPass1>(Q, tok, T, L, c, scale, out, pl, ml, part);
 }
 __global__ void __launch_bounds__(kAttnWaves * 64) attention_mfma_pass2(QMK_ATTN_ARGS) {
-  attention_chunk_body<kAttnPass2>(Q, tok, L, c, scale, out, pl, ml, part);
+  attention_chunk_body<kAttnPass2>(Q, tok, T, L, c, scale, out, pl, ml, part);
 }
 #undef QMK_ATTN_ARGS
 
@@ -1594,7 +1773,7 @@ __global__ void __launch_bounds__(kD) attention_mfma_merge(const float* __restri
                                                           uint16_t* __restrict__ out) {
   const int t = blockIdx.x, h = blockIdx.y, d = threadIdx.x;
   const int wh = pl.where[t], nch = pl.hdr[2], ck = pl.hdr[3];
-  if (wh < 0 || nch == 1) return;  // written by the first pass; by the second
+  if (wh < 0 || nch == 1) return;  // written by the second pass
   const int tile = wh / kQT, row = wh % kQT;
   const int4 tl = pl.tile[tile];
   const int pmax = tl.z + tl.y - 1;
@@ -2487,7 +2666,7 @@ int attn_chunk_budget(int T, int max_context) {
 }
 
 // Tiles planned for a call: each sequence's run may end in a part tile, up to kMoreTiles of them.
-constexpr int kMoreTiles = 63;
+constexpr int kMoreTiles = 255;
 int attn_tiles(int T) { return std::min(T, (T + kQT - 1) / kQT + kMoreTiles); }
 
 struct Layout {
@@ -2532,7 +2711,7 @@ Layout layout(int T, int R, int max_context, bool one_per_seq) {
   if (mfma_attention(T, max_context, one_per_seq)) {
     // header, tiles twice with their ranks and keys, where, left; then the (max, sum) of the tile chunks or,
     // with one chunk each, of the tiles, and the tile chunks' partials
-    take(l.plan, 16 + (size_t)attn_tiles(T) * 32 + (size_t)T * 8);
+    take(l.plan, 32 + (size_t)attn_tiles(T) * 32 + (size_t)T * 8);
     if (const int budget = attn_chunk_budget(T, max_context)) {
       take(l.mml, (size_t)std::max(budget, attn_tiles(T)) * kNQ * kQT * sizeof(float2));
       take(l.mpart, (size_t)budget * kNQ * kQT * kD * 4);
@@ -2652,7 +2831,7 @@ AttnPlan attn_plan(const Args& a, const Layout& l) {
   if (!mfma_attention(a.T, a.max_context, a.one_per_seq)) return AttnPlan{};
   const int cap = attn_tiles(a.T);
   int* hdr = reinterpret_cast<int*>(a.ws + l.plan);
-  int4* tile = reinterpret_cast<int4*>(hdr + 4);
+  int4* tile = reinterpret_cast<int4*>(hdr + 8);
   int2* raw = reinterpret_cast<int2*>(tile + cap);
   int* rank = reinterpret_cast<int*>(raw + cap);
   int* where = rank + 2 * cap;
@@ -2678,17 +2857,17 @@ void launch_attention(const Args& a, const Layout& l, const uint16_t* Q, const T
     float2* aml = reinterpret_cast<float2*>(a.ws + l.mml);
     float* apart = reinterpret_cast<float*>(a.ws + l.mpart);
     const dim3 grid(pl.budget, kNQ);
-    hipLaunchKernelGGL(attention_mfma_pass1, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, L, a.cache, a.attn_scale, ATT,
-                       pl, aml, apart);
-    hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, L, a.cache, a.attn_scale, ATT,
-                       pl, aml, apart);
+    hipLaunchKernelGGL(attention_mfma_pass1, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache, a.attn_scale,
+                       ATT, pl, aml, apart);
+    hipLaunchKernelGGL(attention_mfma_pass2, grid, dim3(kAttnWaves * 64), 0, s, Q, tok, T, L, a.cache, a.attn_scale,
+                       ATT, pl, aml, apart);
     hipLaunchKernelGGL(attention_mfma_merge, dim3(T, kNQ), dim3(kD), 0, s, apart, pl, ATT);
   } else if (a.max_context <= kShortAttn) {
-    hipLaunchKernelGGL(attention_mfma_short, dim3(std::min(pl.cap, kNumWG / kNQ), kNQ), dim3(kAttnWaves * 64), 0, s, Q,
-                       tok, L, a.cache, a.attn_scale, ATT, pl, nullptr, nullptr);
+    hipLaunchKernelGGL(attention_mfma_short, dim3(kNumWG / kNQ, kNQ), dim3(kAttnWaves * 64), 0, s, Q,
+                       tok, T, L, a.cache, a.attn_scale, ATT, pl, nullptr, nullptr);
   } else {
-    hipLaunchKernelGGL(attention_mfma, dim3(kNQ, std::min(pl.cap, kNumWG / kNQ)), dim3(1024), 0, s, Q, tok, L, a.cache,
-                       a.attn_scale, ATT, pl);
+    hipLaunchKernelGGL(attention_mfma, dim3(kNQ, kNumWG / kNQ), dim3(1024), 0, s, Q, tok, T, L, a.cache, a.attn_scale,
+                       ATT, pl);
   }
 }
 

@@ -159,7 +159,7 @@ def test_prompt_does_not_depend_on_the_cache_slots(weights_gpu, n, start):
 def test_attention_tiles_of_several_sequences(shape, exact06, weights_gpu, order):
     """The MFMA attention's tiles over a call of several sequences, 2 layers, every sequence's last rows
     against the oracle: prompts whose tiles end inside the call, tokens in no tile (two sequences token by
-    token: one run each; 130 runs of which the plan holds 71), an invalid token inside a prompt, and the
+    token: one run each; 130 runs of 3), an invalid token inside a prompt, and the
     same over key chunks after a context, and after one with more tiles than tile chunks (20 runs of 10)."""
     from qwen_megakernel.model import BatchDecoder
     from qwen_megakernel.weights import make_prompt
@@ -198,6 +198,59 @@ def test_attention_tiles_of_several_sequences(shape, exact06, weights_gpu, order
         orc = exact_oracle(exact06, shape, S, num_layers=layers)
         ref = oracle_steps(orc, kc, vc, start, prompts[b], emit=[toks[want[k]][1] for k in mine])
         check_rows(t, ref, [int(out[k]) for k in mine], logits[mine].cpu(), bar=LITERAL)
+    print(t)
+
+
+@pytest.mark.parametrize("n,runs", [
+    (330, [(0, 1), (63, 2), (511, 1), (512, 2), (598, 1)]),
+    (70, [(3326, 1), (3327, 1), (3328, 4), (40, 3), (-1, 1)]),
+    (1990, [(8190, 1), (8191, 1), (8192, 2), (511, 1), (-1, 1)]),
+    (2100, [(100, 3), (700, 1), (5, 20), (-1, 1)]),
+    (330, [(p, 1) for p in list(range(0, 500, 4)) + [508, 509, 510, 511, 512, 570]]),
+], ids=["short", "split", "whole", "long-call", "many"])
+def test_tokens_beside_a_prompt(shape, exact06, weights_gpu, n, runs):
+    """Tokens in no attention tile beside a prompt of n tokens, in each of the three kernels that take them, 2
+    layers: runs of fewer tokens than a tile's smallest count, at the edges of what is taken by a wave
+    (position 511), of the scores that LDS holds at once (3328 positions beside tile chunks, 8192 beside
+    whole tiles), a call of more tokens than the plan holds in LDS, more of them than workgroups take ("many"), and an invalid one (position -1)."""
+    from qwen_megakernel.model import BatchDecoder
+    from qwen_megakernel.weights import make_prompt
+
+    V, layers = 151936, 2
+    S = (max([n] + [p + k for p, k in runs]) + 63) // 64 * 64
+    bd = BatchDecoder(weights=with_rope(weights_gpu, S, "cuda"), batch_size=1 + len(runs), max_seq_len=S,
+                      num_layers=layers, verbose=False)
+    bd._k_cache.fill_(float("nan"))
+    bd._v_cache.fill_(float("nan"))
+    g = torch.Generator("cuda").manual_seed(n + len(runs))
+    for b, (p, _) in enumerate(runs, 1):
+        if p > 0:
+            bd.load_kv(b, torch.randn(layers, 8, p, 128, generator=g, device="cuda").bfloat16(),
+                       torch.randn(layers, 8, p, 128, generator=g, device="cuda").bfloat16(), p)
+    # half of the runs before the prompt, half after it
+    order = list(range(1, 1 + len(runs) // 2)) + [0] + list(range(1 + len(runs) // 2, 1 + len(runs)))
+    own = [make_prompt(n, V, seed=1)] + [make_prompt(k, V, seed=70 + b) for b, (_, k) in enumerate(runs)]
+    start = [0] + [p for p, _ in runs]
+    toks = [(b, i) for b in order for i in range(len(own[b]))]
+    ids, seqs, pos = [own[b][i] for b, i in toks], [b for b, _ in toks], [start[b] + i for b, i in toks]
+    check = [b for b in order if b and (len(runs) < 20 or b % 21 == 0 or start[b] > 500)]
+    want = [k for k, (b, _) in enumerate(toks) if b in check]
+    out = torch.empty(len(want), dtype=torch.int32, device="cuda")
+    logits = torch.empty(len(want), V, dtype=torch.float32, device="cuda")
+    bd._forward(_t(ids), _t(seqs), _t(pos), _t(want), out, logits, bd._k_cache, bd._v_cache, max(pos) + 1)
+    t = Tally(f"{len(runs)} runs beside {n} tokens")
+    for b in check:
+        mine = [k for k, w in enumerate(want) if toks[w][0] == b]
+        if start[b] < 0:
+            assert [int(out[k]) for k in mine] == [-1]
+            continue
+        m = start[b] + len(own[b])
+        kc, vc = (torch.zeros_like(x[b]) for x in (bd._k_cache, bd._v_cache))
+        kc[:, :, :m], vc[:, :, :m] = bd._k_cache[b, :, :, :m], bd._v_cache[b, :, :, :m]
+        orc = exact_oracle(exact06, shape, S, num_layers=layers)
+        ref = oracle_steps(orc, kc, vc, start[b], own[b])
+        check_rows(t, ref, [int(out[k]) for k in mine], logits[mine].cpu(), bar=LITERAL)
+        check_kv_rows(f"sequence {b}", orc, kc, vc, start[b], len(own[b]))
     print(t)
 
 
