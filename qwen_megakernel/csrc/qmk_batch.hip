@@ -1793,7 +1793,8 @@ __global__ void __launch_bounds__(kD) attention_mfma_merge(const float* __restri
 
 // Context-split attention: one token per row of the launch (a batched decode step; a few tokens of a
 // prompt), its context in chunks of kSplitChunk positions, one workgroup of 4 waves per (chunk, KV
-// head, token), in HF's two passes over three launches:
+// head, token), or per every gridDim.x'th chunk (launch_attn_chunks), in HF's two passes over three
+// launches:
 // - attn_chunk_scores requests the chunk's K rows (a lane row of 16 takes one position, so one wave
 //   instruction reads four whole rows), scores them as HF rounds them, stores the scores (fp32)
 //   and the chunk's (max m, sum l of exp(s - m)) per head.  RAW: q, k, v come as the q/k/v
@@ -1813,7 +1814,7 @@ __global__ void __launch_bounds__(kD) attention_mfma_merge(const float* __restri
 // from setting the time.  Qwen3-0.6B, us per layer for the three launches, against the forms it
 // replaced: 8 sequences of 5..1500 positions 32.3 -> 15.6, 3 of 5000..6100 74.7 -> 21.8, 48 of
 // 100..1000 86 -> 35.
-template <bool RAW>
+template <bool RAW, bool SEVERAL>
 __global__ void __launch_bounds__(256) attn_chunk_scores(const uint16_t* __restrict__ src, const Tok* __restrict__ tok,
                                                          int L, const uint16_t* __restrict__ q_norm,
                                                          const uint16_t* __restrict__ k_norm,
@@ -1825,15 +1826,16 @@ __global__ void __launch_bounds__(256) attn_chunk_scores(const uint16_t* __restr
   __shared__ float sc[2][kSplitChunk];
   __shared__ __align__(16) uint16_t qs[2][kD], kn[kD];
   __shared__ float wm[4], wl[4];
-  const int j = blockIdx.x, g = blockIdx.y, t = blockIdx.z;
+  const int g = blockIdx.y, t = blockIdx.z, step = gridDim.x;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, slot = lane >> 4,
             t16 = lane & 15;
   const Tok tk = tok[t];
-  const int pos = tk.pos, c0 = j * kSplitChunk, n = min(pos + 1 - c0, kSplitChunk);
-  if (!tk.valid || n <= 0) return;
+  const int pos = __builtin_amdgcn_readfirstlane(tk.pos);
+  int j = blockIdx.x;
+  if (!tk.valid || j * kSplitChunk > pos) return;
   const size_t base = cache_base(c, tk, L, g);
   const uint16_t* kc = c.k + base;
-  const bool own = RAW && n <= kSplitChunk && pos < c0 + kSplitChunk;  // the chunk of the token's own position
+  const bool own = RAW && (SEVERAL ? pos / kSplitChunk % step : pos / kSplitChunk) == j;  // this workgroup's chunks hold the token's own position
   u32x4 qv[2];
   // waves 0, 1: q heads 2g, 2g+1; wave 2: k head g; wave 3: v head g
   const int h = w < 2 ? 2 * g + w : (w == 2 ? kNQ + g : kNQ + kNKV + g);
@@ -1855,8 +1857,12 @@ __global__ void __launch_bounds__(256) attn_chunk_scores(const uint16_t* __restr
   // in the cache yet (RAW)
   const int plast = RAW ? max(pos - 1, 0) : pos;
   u32x4 kx[NR];
+  auto request = [&](int j) {
 #pragma unroll
-  for (int r = 0; r < NR; r++) kx[r] = ld16(kc + (size_t)min(c0 + 16 * r + 4 * w + slot, plast) * kD + 8 * t16);
+    for (int r = 0; r < NR; r++)
+      kx[r] = ld16(kc + (uint32_t)(min(j * kSplitChunk + 16 * r + 4 * w + slot, plast) * kD + 8 * t16));
+  };
+  request(j);
   u32x4 k_now = u32x4{0, 0, 0, 0};
   if constexpr (RAW) {
     if (w == 3) {
@@ -1886,57 +1892,70 @@ __global__ void __launch_bounds__(256) attn_chunk_scores(const uint16_t* __restr
     for (int hh = 0; hh < 2; hh++) qv[hh] = *reinterpret_cast<const u32x4*>(&qs[hh][8 * t16]);
     k_now = *reinterpret_cast<const u32x4*>(&kn[8 * t16]);
   }
+  for (;;) {
+    const int c0 = j * kSplitChunk, n = min(pos + 1 - c0, kSplitChunk);
 #pragma unroll
-  for (int r = 0; r < NR; r++) {
-    const int i = 16 * r + 4 * w + slot;
-    const u32x4 kr = RAW && c0 + i == pos ? k_now : kx[r];
-    const float s0 = row16_sum(dot8(kr, qv[0], 0.f)), s1 = row16_sum(dot8(kr, qv[1], 0.f));
-    if (t16 < 2) sc[t16][i] = t16 ? s1 : s0;
-  }
-  __syncthreads();
-  // one (head, position) per thread: the score as HF rounds it, the chunk's maximum and sum
-  static_assert(kSplitChunk == 128, "256 threads: 2 heads x 128 positions, two waves per head");
-  const int hh = w >> 1, i = threadIdx.x & (kSplitChunk - 1);
-  const float s = bf16r(bf16r(sc[hh][i]) * scale);
-  if (i < n) scores[((size_t)t * kNQ + 2 * g + hh) * ((size_t)nch * kSplitChunk) + c0 + i] = s;
-  const float m = wave_max_all(i < n ? s : -INFINITY);
-  const float l = wave_total(i < n && m > -INFINITY ? exp_acc(s - m) : 0.f);
-  if (lane == 0) {
-    wm[w] = m;
-    wl[w] = l;
-  }
-  __syncthreads();
-  if (threadIdx.x < 2) {
-    const int q = 2 * threadIdx.x;
-    const float ma = wm[q], mb = wm[q + 1], mx = fmaxf(ma, mb);
-    const float la = ma == -INFINITY ? 0.f : wl[q] * exp_acc(ma - mx);
-    const float lb = mb == -INFINITY ? 0.f : wl[q + 1] * exp_acc(mb - mx);
-    ml[((size_t)t * kNQ + 2 * g + threadIdx.x) * nch + j] = make_float2(mx, la + lb);
+    for (int r = 0; r < NR; r++) {
+      const int i = 16 * r + 4 * w + slot;
+      const u32x4 kr = RAW && c0 + i == pos ? k_now : kx[r];
+      const float s0 = row16_sum(dot8(kr, qv[0], 0.f)), s1 = row16_sum(dot8(kr, qv[1], 0.f));
+      if (t16 < 2) sc[t16][i] = t16 ? s1 : s0;
+    }
+    __syncthreads();
+    // one (head, position) per thread: the score as HF rounds it, the chunk's maximum and sum
+    static_assert(kSplitChunk == 128, "256 threads: 2 heads x 128 positions, two waves per head");
+    const int hh = w >> 1, i = threadIdx.x & (kSplitChunk - 1);
+    const float s = bf16r(bf16r(sc[hh][i]) * scale);
+    if (i < n) scores[((size_t)t * kNQ + 2 * g + hh) * ((size_t)nch * kSplitChunk) + c0 + i] = s;
+    const float m = wave_max_all(i < n ? s : -INFINITY);
+    const float l = wave_total(i < n && m > -INFINITY ? exp_acc(s - m) : 0.f);
+    if (lane == 0) {
+      wm[w] = m;
+      wl[w] = l;
+    }
+    __syncthreads();  // (the next chunk's scores may be written; its pairs come after another barrier)
+    if (threadIdx.x < 2) {
+      const int q = 2 * threadIdx.x;
+      const float ma = wm[q], mb = wm[q + 1], mx = fmaxf(ma, mb);
+      const float la = ma == -INFINITY ? 0.f : wl[q] * exp_acc(ma - mx);
+      const float lb = mb == -INFINITY ? 0.f : wl[q + 1] * exp_acc(mb - mx);
+      ml[((size_t)t * kNQ + 2 * g + threadIdx.x) * nch + j] = make_float2(mx, la + lb);
+    }
+    j += step;
+    if (!SEVERAL || j * kSplitChunk > pos) return;
+    request(j);
   }
 }
 
+template <bool SEVERAL>
 __global__ void __launch_bounds__(256) attn_chunk_pv(const Tok* __restrict__ tok, int L, Cache c, int nch,
                                                      const float* __restrict__ scores, const float2* __restrict__ ml,
                                                      float* __restrict__ pvp) {
   constexpr int NR = kSplitChunk / 16;
   __shared__ float pr[2][kSplitChunk];
   __shared__ float wacc[4][2][kD];
-  const int j = blockIdx.x, g = blockIdx.y, t = blockIdx.z;
+  const int g = blockIdx.y, t = blockIdx.z, step = gridDim.x;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, slot = lane >> 4,
             t16 = lane & 15;
   const Tok tk = tok[t];
-  const int pos = tk.pos, c0 = j * kSplitChunk, n = min(pos + 1 - c0, kSplitChunk);
-  if (!tk.valid || n <= 0) return;
+  const int pos = __builtin_amdgcn_readfirstlane(tk.pos);
+  int j = blockIdx.x;
+  if (!tk.valid || j * kSplitChunk > pos) return;
   const uint16_t* vc = c.v + cache_base(c, tk, L, g);
   // this thread's score (head w / 2, position i of the chunk) and its head's pairs, then the V rows
   const int hh = w >> 1, i = threadIdx.x & (kSplitChunk - 1), used = pos / kSplitChunk + 1;
   const size_t row = (size_t)t * kNQ + 2 * g + hh;
-  const float s = scores[row * ((size_t)nch * kSplitChunk) + c0 + min(i, n - 1)];
+  const float* sch = scores + row * ((size_t)nch * kSplitChunk);
+  float s = sch[min(j * kSplitChunk + i, pos)];
   const float2* mlh = ml + row * nch;
   const float2 first = lane < used ? mlh[lane] : make_float2(-INFINITY, 0.f);
   u32x4 vx[NR];
+  auto request = [&](int j) {
 #pragma unroll
-  for (int r = 0; r < NR; r++) vx[r] = ld16(vc + (size_t)min(c0 + 16 * r + 4 * w + slot, pos) * kD + 8 * t16);
+    for (int r = 0; r < NR; r++)
+      vx[r] = ld16(vc + (uint32_t)(min(j * kSplitChunk + 16 * r + 4 * w + slot, pos) * kD + 8 * t16));
+  };
+  request(j);
   float mx = first.x;
   for (int q = 64 + lane; q < used; q += 64) mx = fmaxf(mx, mlh[q].x);
   mx = wave_max_all(mx);
@@ -1946,43 +1965,50 @@ __global__ void __launch_bounds__(256) attn_chunk_pv(const Tok* __restrict__ tok
     ls += e.x == -INFINITY ? 0.f : e.y * exp_acc(e.x - mx);
   }
   const float inv = __fdiv_rn(1.0f, wave_total(ls));
-  pr[hh][i] = i < n ? bf16r(exp_acc(s - mx) * inv) : 0.f;
-  __syncthreads();
-  float acc[2][8];
+  for (;;) {
+    const int n = min(pos + 1 - j * kSplitChunk, kSplitChunk);
+    pr[hh][i] = i < n ? bf16r(exp_acc(s - mx) * inv) : 0.f;
+    __syncthreads();
+    float acc[2][8];
 #pragma unroll
-  for (int q = 0; q < 2; q++)
+    for (int q = 0; q < 2; q++)
 #pragma unroll
-    for (int e = 0; e < 8; e++) acc[q][e] = 0.f;
+      for (int e = 0; e < 8; e++) acc[q][e] = 0.f;
 #pragma unroll
-  for (int r = 0; r < NR; r++) {
-    const int p = 16 * r + 4 * w + slot;
-    // rows past the last position carry probability 0 and a repeated row; taken as zeros, so that
-    // an infinity in that row is not counted twice (0 * inf)
-    const bool live = p < n;
-    const u32x4 vr = u32x4{live ? vx[r].x : 0u, live ? vx[r].y : 0u, live ? vx[r].z : 0u, live ? vx[r].w : 0u};
-    const float vf[8] = {lo_bf16(vr.x), hi_bf16(vr.x), lo_bf16(vr.y), hi_bf16(vr.y),
-                         lo_bf16(vr.z), hi_bf16(vr.z), lo_bf16(vr.w), hi_bf16(vr.w)};
-    const float p0 = pr[0][p], p1 = pr[1][p];
+    for (int r = 0; r < NR; r++) {
+      const int p = 16 * r + 4 * w + slot;
+      // rows past the last position carry probability 0 and a repeated row; taken as zeros, so that
+      // an infinity in that row is not counted twice (0 * inf)
+      const bool live = p < n;
+      const u32x4 vr = u32x4{live ? vx[r].x : 0u, live ? vx[r].y : 0u, live ? vx[r].z : 0u, live ? vx[r].w : 0u};
+      const float vf[8] = {lo_bf16(vr.x), hi_bf16(vr.x), lo_bf16(vr.y), hi_bf16(vr.y),
+                           lo_bf16(vr.z), hi_bf16(vr.z), lo_bf16(vr.w), hi_bf16(vr.w)};
+      const float p0 = pr[0][p], p1 = pr[1][p];
 #pragma unroll
-    for (int e = 0; e < 8; e++) {
-      acc[0][e] = __builtin_fmaf(p0, vf[e], acc[0][e]);
-      acc[1][e] = __builtin_fmaf(p1, vf[e], acc[1][e]);
+      for (int e = 0; e < 8; e++) {
+        acc[0][e] = __builtin_fmaf(p0, vf[e], acc[0][e]);
+        acc[1][e] = __builtin_fmaf(p1, vf[e], acc[1][e]);
+      }
     }
-  }
-  // the wave's four lane rows, then the four waves in order
+    // the wave's four lane rows, then the four waves in order
 #pragma unroll
-  for (int q = 0; q < 2; q++) {
+    for (int q = 0; q < 2; q++) {
 #pragma unroll
-    for (int e = 0; e < 8; e++) acc[q][e] = rows_sum4(acc[q][e]);
-    if (lane < 16) {
-      *reinterpret_cast<f32x4*>(&wacc[w][q][8 * t16]) = f32x4{acc[q][0], acc[q][1], acc[q][2], acc[q][3]};
-      *reinterpret_cast<f32x4*>(&wacc[w][q][8 * t16 + 4]) = f32x4{acc[q][4], acc[q][5], acc[q][6], acc[q][7]};
+      for (int e = 0; e < 8; e++) acc[q][e] = rows_sum4(acc[q][e]);
+      if (lane < 16) {
+        *reinterpret_cast<f32x4*>(&wacc[w][q][8 * t16]) = f32x4{acc[q][0], acc[q][1], acc[q][2], acc[q][3]};
+        *reinterpret_cast<f32x4*>(&wacc[w][q][8 * t16 + 4]) = f32x4{acc[q][4], acc[q][5], acc[q][6], acc[q][7]};
+      }
     }
+    __syncthreads();  // (the next chunk's probabilities may be written; its sums come after another barrier)
+    const int d = threadIdx.x & 127, ho = threadIdx.x >> 7;  // 256 threads: both heads' dims
+    pvp[(((size_t)t * nch + j) * kNQ + 2 * g) * kD + threadIdx.x] =
+        ((wacc[0][ho][d] + wacc[1][ho][d]) + wacc[2][ho][d]) + wacc[3][ho][d];
+    j += step;
+    if (!SEVERAL || j * kSplitChunk > pos) return;
+    s = sch[min(j * kSplitChunk + i, pos)];
+    request(j);
   }
-  __syncthreads();
-  const int d = threadIdx.x & 127, ho = threadIdx.x >> 7;  // 256 threads: both heads' dims
-  pvp[(((size_t)t * nch + j) * kNQ + 2 * g) * kD + threadIdx.x] =
-      ((wacc[0][ho][d] + wacc[1][ho][d]) + wacc[2][ho][d]) + wacc[3][ho][d];
 }
 
 // The output of (token t, head): its used chunks' partials added, rounded to bf16 (zeros for an invalid
@@ -2815,14 +2841,29 @@ AttnChunks attn_chunks(const Args& a, const Layout& l) {
           reinterpret_cast<float2*>(a.ws + l.ml), reinterpret_cast<float*>(a.ws + l.pv)};
 }
 
+// Workgroups of a launch at most: the call's context is a bound that its tokens may lie far below, and a
+// workgroup without a chunk still costs 2 ns, so above this each takes several chunks (one step, 4 layers,
+// us, one chunk each / several: 128 sequences at 100..200 with a bound of 4096 1010 / 423, of 201 430 both;
+// where the bound is the context, 256 sequences at 1000..1100 1295 / 1340, 64 at 1000..4000 790 / 790).
+// An odd number per (token, head), since workgroups go to the eight XCDs in turn: with eight, every token's
+// first chunk falls on the same one (48 sequences at 100..200, bound 4096: 354 us with 8, 300 with 10 and 9).
+constexpr int kChunkWGs = 3072;
+
 template <bool RAW>
 void launch_attn_chunks(const Args& a, const AttnChunks& ac, const uint16_t* src, const Tok* tok, int L,
                         const LDGLayerWeights& w, float eps, uint16_t* out, hipStream_t s) {
-  const dim3 grid(ac.nch, kNKV, a.T);
-  hipLaunchKernelGGL(attn_chunk_scores<RAW>, grid, dim3(256), 0, s, src, tok, L,
-                     static_cast<const uint16_t*>(w.q_norm_weight), static_cast<const uint16_t*>(w.k_norm_weight),
-                     a.cos_t, a.sin_t, a.cache, eps, a.attn_scale, ac.nch, ac.scores, ac.ml);
-  hipLaunchKernelGGL(attn_chunk_pv, grid, dim3(256), 0, s, tok, L, a.cache, ac.nch, ac.scores, ac.ml, ac.pvp);
+  auto go = [&](auto several, int per_head) {
+    constexpr bool SEVERAL = decltype(several)::value;
+    const dim3 grid(per_head, kNKV, a.T);
+    hipLaunchKernelGGL((attn_chunk_scores<RAW, SEVERAL>), grid, dim3(256), 0, s, src, tok, L,
+                       static_cast<const uint16_t*>(w.q_norm_weight), static_cast<const uint16_t*>(w.k_norm_weight),
+                       a.cos_t, a.sin_t, a.cache, eps, a.attn_scale, ac.nch, ac.scores, ac.ml);
+    hipLaunchKernelGGL(attn_chunk_pv<SEVERAL>, grid, dim3(256), 0, s, tok, L, a.cache, ac.nch, ac.scores, ac.ml,
+                       ac.pvp);
+  };
+  const int most = std::max(1, kChunkWGs / (kNKV * a.T));
+  if (ac.nch <= most) go(std::false_type{}, ac.nch);
+  else go(std::true_type{}, most - 1 + most % 2);
   hipLaunchKernelGGL(attn_chunk_merge, dim3(a.T, kNQ), dim3(256), 0, s, tok, ac.nch, ac.pvp, out);
 }
 

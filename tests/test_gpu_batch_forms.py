@@ -53,6 +53,37 @@ def test_decode_batch_attention_chunk_edges(shape, exact06, weights_gpu, c0s):
     _decode_steps(shape, exact06, weights_gpu, c0s, layers=2, max_seq=(max(c0s) + 2 + 63) // 64 * 64)
 
 
+def test_decode_batch_several_chunks(shape, exact06, weights_gpu):
+    """More chunks than workgroups (40 sequences, a context bound of 12 chunks: 9 workgroups per head, some of
+    which take two), contexts at the edges of the chunks taken second, against the oracle."""
+    c0s = tuple(range(3, 31)) + (1151, 1152, 1153, 1278, 1279, 1280, 1400, 1498, 127, 128, 1023, 700)
+    _decode_steps(shape, exact06, weights_gpu, c0s, layers=2, max_seq=1536, steps=1)
+
+
+@pytest.mark.parametrize("batch", [5, 40])
+def test_decode_batch_does_not_depend_on_the_bound(weights_gpu, batch):
+    """The same step with max_context at its longest sequence and far above it (each workgroup several
+    chunks, nearly all of which no token reaches): the same bits."""
+    from qwen_megakernel.model import _Forward, _ops
+
+    V, layers, S = 151936, 2, 16384 if batch == 5 else 4096
+    w = with_rope(weights_gpu, S, "cuda")
+    fwd = _Forward(_ops(), w, layers)
+    g = torch.Generator("cuda").manual_seed(batch)
+    k0 = torch.randn(batch, layers, 8, S, 128, generator=g, device="cuda").bfloat16()
+    v0 = torch.randn(batch, layers, 8, S, 128, generator=g, device="cuda").bfloat16()
+    pos = [(37 * b) % 300 for b in range(batch)]
+    got = []
+    for bound in (max(pos) + 1, S):
+        k, v = k0.clone(), v0.clone()
+        out = torch.empty(batch, dtype=torch.int32, device="cuda")
+        logits = torch.empty(batch, V, dtype=torch.float32, device="cuda")
+        fwd.decode(_t(range(batch)), _t(pos), out, logits, k, v, bound)
+        got.append((out, logits, k, v))
+    for a, b in zip(*got):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("rows", [17, 32, 33, 64, 65, 200])
 def test_lm_head_row_groups(weights_gpu, rows):
     """lm_head_tiled (more than 16 emitted rows, groups of 32 or 64): logits within one bf16 ulp of the
