@@ -49,28 +49,41 @@ struct SampleParams {
   uint64_t seed;
 };
 
-// Device work of one logits row between the launches of a sampling call: the row's histogram (counts
-// or fixed-point masses), selection state and candidates.  Zero between calls (but for the
-// candidates): the call's last launch clears it.
+// Device work of one logits row between the launches of a sampling call: its selection state, and the
+// histogram of one 8-bit radix digit (counts or fixed-point masses).  Zero between calls: the call's last
+// launch clears it.
 constexpr int kSampleBins = 2048, kSampleCand = 8192;
 struct SampleWork {
-  unsigned long long hist[kSampleBins];  // bins of the first digit (256 of them: of one 8-bit radix digit)
+  unsigned long long hist[256];
   unsigned long long z, target, need, best;  // need: top-k rank still sought / top-p mass above the prefix
   unsigned int maxkey, prefix, mask, kmin, pmin, ticket;
   unsigned int ncand, candmin, candmax;  // candidates; ~(smallest key), largest key among them
   unsigned int pad;
   unsigned long long tied;               // best draw among the candidates, if their keys are all the same
+};
+// What the two-launch form of a filtered draw needs besides, per row of its launches: the first digit's
+// histogram (zero between calls) and the candidates.
+struct SampleLists {
+  unsigned long long hist[kSampleBins];
   unsigned long long cand[kSampleCand];  // key << 32 | token
 };
-constexpr int kSampleRowsMax = 64;  // rows per launch sequence of qmk_sample_rows (5 MB of work)
+// Rows per launch sequence of qmk_sample_rows (0.5 MB of work); of the two-launch form, whose lists would
+// make that 21 MB (5 MB).  A draw of 256 rows without a filter takes 34-83 us in one sequence and 107-167 in
+// four.
+constexpr int kSampleRowsMax = 256, kSampleListRows = 64;
 
-// hipMalloc + zero fill of `rows` work blocks.
+// The work of up to `rows` rows, in one allocation: `rows` SampleWork, then the lists.
+__host__ __device__ inline SampleLists* sample_lists(SampleWork* work, int rows) {
+  return reinterpret_cast<SampleLists*>(work + rows);
+}
+
+// hipMalloc + zero fill of the work of `rows` rows.
 int alloc_sample_work(SampleWork** out, int rows);
 
 // Persistent-mode sampler of the generate loop: when the decode step just run
 // produced `logits`, replace its greedy token in the state and the log by a
 // sampled one (counter = the step's position) and set `done` for the stop token.
-// `work`: one zeroed SampleWork owned by the caller's stream.
+// `work`: one row's zeroed work, owned by the caller's stream.
 int launch_sample_state(const float* logits, int vocab, const SampleParams& sp, DecodeState* st, int* log,
                         SampleWork* work, hipStream_t stream);
 

@@ -39,6 +39,7 @@
 #include "qmk_device.h"
 #include "qmk_sample.h"
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <type_traits>
@@ -62,6 +63,7 @@ struct Args {
   DecodeState* st;            // state mode (one row): counter = st->pos - 1; the token replaces st->tok
   int* log;
   SampleWork* work;           // one per row, zero between calls
+  SampleLists* lists;         // one per row (two-launch form)
 };
 
 __device__ __forceinline__ float from_key32(uint32_t k) {
@@ -78,6 +80,7 @@ struct Block {
   int v0, v1;           // this workgroup's slice of the row
   uint64_t counter;
   SampleWork* w;
+  SampleLists* ls;
   uint32_t greedy_tok;  // state mode: the decode step's greedy token (its logit is the row maximum)
 };
 
@@ -105,6 +108,7 @@ __device__ bool setup(const Args& a, Block& b) {
   b.v1 = min(a.V, b.v0 + chunk);
   b.counter = (uint64_t)ctr;
   b.w = a.work + b.row;
+  b.ls = a.lists + b.row;
   b.greedy_tok = a.st ? (uint32_t)tok : 0u;
   return run != 0;
 }
@@ -356,7 +360,7 @@ __global__ void __launch_bounds__(kThreads) k_first(Args a) {
 #pragma unroll
   for (int i = 0; i < 8; i++) {
     const unsigned long long h = wh[threadIdx.x + kThreads * i];
-    if (h) atomicAdd(&w->hist[threadIdx.x + kThreads * i], h);
+    if (h) atomicAdd(&b.ls->hist[threadIdx.x + kThreads * i], h);
   }
   if (!last_block(w)) return;
 
@@ -366,7 +370,7 @@ __global__ void __launch_bounds__(kThreads) k_first(Args a) {
   unsigned long long h[8], own = 0, total;
 #pragma unroll
   for (int i = 0; i < 8; i++) {
-    h[i] = load_u64(&w->hist[8 * t + i]);
+    h[i] = load_u64(&b.ls->hist[8 * t + i]);
     own += h[i];
   }
   const unsigned long long after = block_sum_after(own, total);
@@ -382,7 +386,7 @@ __global__ void __launch_bounds__(kThreads) k_first(Args a) {
     above[i] = run;  // S[8t + i + 1]
     run += h[i];
     n += (8 * t + i >= 1 && run >= sought) ? 1u : 0u;
-    w->hist[8 * t + i] = 0;  // ready for the next call
+    b.ls->hist[8 * t + i] = 0;  // ready for the next call
   }
   if (n) atomicAdd(&ndig, n);
   __syncthreads();
@@ -453,7 +457,7 @@ __global__ void __launch_bounds__(kThreads) k_finish(Args a) {
   if (nlocal && nlocal <= (unsigned)kLocalCand)
     for (unsigned int i = threadIdx.x; i < nlocal; i += kThreads)
       if (base + i < (unsigned)kSampleCand)
-        __hip_atomic_store(&w->cand[base + i], local[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __hip_atomic_store(&b.ls->cand[base + i], local[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   if (threadIdx.x == 0) {
     if (best) atomicMax(&w->best, best);
     if (nlocal) {
@@ -474,7 +478,7 @@ __global__ void __launch_bounds__(kThreads) k_finish(Args a) {
     best = g > best ? g : best;
   } else {
     if (listed)
-      for (unsigned int i = threadIdx.x; i < nc; i += kThreads) ck[i] = (uint32_t)(load_u64(&w->cand[i]) >> 32);
+      for (unsigned int i = threadIdx.x; i < nc; i += kThreads) ck[i] = (uint32_t)(load_u64(&b.ls->cand[i]) >> 32);
     __syncthreads();
     // f(key) for every candidate
     auto each = [&](auto&& f) {
@@ -550,7 +554,7 @@ __global__ void __launch_bounds__(kThreads) k_finish(Args a) {
     if (listed) {
       for (unsigned int i = threadIdx.x; i < nc; i += kThreads)
         if (ck[i] >= keep) {
-          const int v = (int)(uint32_t)load_u64(&w->cand[i]);
+          const int v = (int)(uint32_t)load_u64(&b.ls->cand[i]);
           const unsigned long long q = draw(v, b.x[v]);
           g = q > g ? q : g;
         }
@@ -608,6 +612,12 @@ int groups_for(int rows) {
   return g;
 }
 
+// Draws that take the two-launch form
+bool two_launches(const SampleParams& sp, int V) {
+  const bool topk = sp.top_k > 0 && sp.top_k < V, topp = sp.top_p > 0.f && sp.top_p < 1.f;
+  return sp.temperature > 0.f && (topk || topp) && !(topk && sp.top_k > kFinishTopK);
+}
+
 int launch(const Args& a, int rows, hipStream_t stream) {
   const dim3 grid(groups_for(rows), rows), block(kThreads);
   const SampleParams& sp = a.sp;
@@ -617,7 +627,7 @@ int launch(const Args& a, int rows, hipStream_t stream) {
     const bool topk = sp.top_k > 0 && sp.top_k < a.V;
     const bool topp = sp.top_p > 0.f && sp.top_p < 1.f;
     if (topp && !a.st && (!topk || sp.top_k > kFinishTopK)) hipLaunchKernelGGL(k_max, grid, block, 0, stream, a);
-    if ((topk || topp) && !(topk && sp.top_k > kFinishTopK)) {
+    if (two_launches(sp, a.V)) {
       if (topk) hipLaunchKernelGGL(k_first<false>, grid, block, 0, stream, a);
       else hipLaunchKernelGGL(k_first<true>, grid, block, 0, stream, a);
       if (topk && topp) hipLaunchKernelGGL((k_finish<true, true>), grid, block, 0, stream, a);
@@ -657,7 +667,8 @@ int stream_work(hipStream_t stream, SampleWork** out) {
 }  // namespace sample
 
 int alloc_sample_work(SampleWork** out, int rows) {
-  const size_t bytes = (size_t)rows * sizeof(SampleWork);
+  static_assert(sizeof(SampleWork) % alignof(SampleLists) == 0, "the lists follow the rows' work");
+  const size_t bytes = (size_t)rows * sizeof(SampleWork) + (size_t)std::min(rows, kSampleListRows) * sizeof(SampleLists);
   if (hipMalloc(out, bytes) != hipSuccess) return QMK_ERR_HIP;
   // the fill runs on the null stream: wait for it, since the caller's stream need not
   if (hipMemset(*out, 0, bytes) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) {
@@ -670,7 +681,7 @@ int alloc_sample_work(SampleWork** out, int rows) {
 
 int launch_sample_state(const float* logits, int vocab, const SampleParams& sp, DecodeState* st, int* log,
                         SampleWork* work, hipStream_t stream) {
-  sample::Args a{logits, vocab, sp, nullptr, nullptr, st, log, work};
+  sample::Args a{logits, vocab, sp, nullptr, nullptr, st, log, work, sample_lists(work, 1)};
   return sample::launch(a, 1, stream);
 }
 
@@ -687,9 +698,11 @@ extern "C" int qmk_sample_rows(const float* logits, int rows, int vocab, float t
   SampleWork* work = nullptr;
   int s = sample::stream_work(stream, &work);
   if (s != QMK_OK) return s;
-  for (int r0 = 0; r0 < rows && s == QMK_OK; r0 += kSampleRowsMax) {
-    const int n = rows - r0 < kSampleRowsMax ? rows - r0 : kSampleRowsMax;
-    sample::Args a{logits + (size_t)r0 * vocab, vocab, sp, counters + r0, out_tokens + r0, nullptr, nullptr, work};
+  const int most = sample::two_launches(sp, vocab) ? kSampleListRows : kSampleRowsMax;
+  for (int r0 = 0; r0 < rows && s == QMK_OK; r0 += most) {
+    const int n = std::min(rows - r0, most);
+    sample::Args a{logits + (size_t)r0 * vocab, vocab, sp, counters + r0, out_tokens + r0, nullptr, nullptr, work,
+                   sample_lists(work, kSampleRowsMax)};
     s = sample::launch(a, n, stream);
   }
   return s;

@@ -52,6 +52,19 @@ def test_filtered_draw_small_vocabularies(n):
         _compare(rows, 1.1, k, p, 5, list(range(5)))
 
 
+@pytest.mark.parametrize("rows", [64, 65, 256, 257])
+def test_row_groups(rows):
+    """Rows at the edges of a launch sequence's rows (64 of the two-launch form, 256 of the others): every
+    form draws what it draws for each row alone, and leaves the work clear."""
+    rng = np.random.default_rng(rows)
+    x = rng.normal(0, 2, (rows, 700)).astype(np.float32)
+    ctr = list(range(rows))
+    for T, k, p in ((0.0, 0, 1.0), (0.9, 0, 1.0), (0.9, 30, 1.0), (0.9, 0, 0.8), (0.9, 30, 0.8), (0.9, 5000, 1.0)):
+        got = _compare(x, T, k, p, 11, ctr)
+        some = [0, 63, 64 % rows, rows - 1]
+        assert [got[r] for r in some] == [_gpu_sample(x[r:r + 1], T, k, p, 11, [ctr[r]])[0] for r in some]
+
+
 def test_work_is_clear_after_every_form():
     """A call of each form after each other form on one stream gives what it gives alone."""
     rng = np.random.default_rng(9)
