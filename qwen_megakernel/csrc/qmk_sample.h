@@ -36,10 +36,12 @@ __device__ __forceinline__ uint32_t key32(float f) {
   return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
 
-// Key of token v's Gumbel-perturbed score: key32(logit / T + G), G = -log(-log(U)).
-__device__ __forceinline__ uint32_t gumbel_key(float logit, float temperature, uint64_t base, int v) {
-  const float s = __fdiv_rn(logit, temperature);
+// Key of token v's Gumbel-perturbed score s: key32(s + G), G = -log(-log(U)).
+__device__ __forceinline__ uint32_t gumbel_key_score(float s, uint64_t base, int v) {
   return key32(s + -logf(-logf(draw_uniform(base, v))));
+}
+__device__ __forceinline__ uint32_t gumbel_key(float logit, float temperature, uint64_t base, int v) {
+  return gumbel_key_score(__fdiv_rn(logit, temperature), base, v);
 }
 
 struct SampleParams {
@@ -52,25 +54,29 @@ struct SampleParams {
 // Device work of one logits row between the launches of a sampling call: its selection state, and the
 // histogram of one 8-bit radix digit (counts or fixed-point masses).  Zero between calls: the call's last
 // launch clears it.
-constexpr int kSampleBins = 2048, kSampleCand = 8192;
+constexpr int kSampleBins = 2048, kSampleCand = 4096;
 struct SampleWork {
   unsigned long long hist[256];
   unsigned long long z, target, need, best;  // need: top-k rank still sought / top-p mass above the prefix
   unsigned int maxkey, prefix, mask, kmin, pmin, ticket;
-  unsigned int ncand, candmin, candmax;  // candidates; ~(smallest key), largest key among them
-  unsigned int pad;
-  unsigned long long tied;               // best draw among the candidates, if their keys are all the same
+  // two-launch form: scores above the threshold's bin (both filters) and in it, ~(smallest key) and largest
+  // key in the bin, largest key above it, whether the bin is one of the finer ones (and is to be cut so)
+  unsigned int nabove, nbin, binmin, binmax, abovemax, finer;
+  unsigned long long tied;  // best draw in the bin, if its keys are all the same
 };
-// What the two-launch form of a filtered draw needs besides, per row of its launches: the first digit's
-// histogram (zero between calls) and the candidates.
+// What the two-launch form of a filtered draw needs besides, per row of its launches: a histogram (zero
+// between calls) and, after it, the tokens in the threshold's bin; those above the bin; up to kSampleCand of each.
 struct SampleLists {
-  unsigned long long hist[kSampleBins];
-  unsigned long long cand[kSampleCand];  // key << 32 | token
+  union {
+    unsigned long long hist[kSampleBins];
+    unsigned int bin[kSampleCand];
+  };
+  unsigned int above[kSampleCand];
 };
 // Rows per launch sequence of qmk_sample_rows (0.5 MB of work); of the two-launch form, whose lists would
-// make that 21 MB (5 MB).  A draw of 256 rows without a filter takes 34-83 us in one sequence and 107-167 in
-// four.
-constexpr int kSampleRowsMax = 256, kSampleListRows = 64;
+// make that 8 MB, 128 (4 MB).  A draw of 256 rows without a filter takes 33-84 us in one sequence and 107-167
+// in four.
+constexpr int kSampleRowsMax = 256, kSampleListRows = 128;
 
 // The work of up to `rows` rows, in one allocation: `rows` SampleWork, then the lists.
 __host__ __device__ inline SampleLists* sample_lists(SampleWork* work, int rows) {

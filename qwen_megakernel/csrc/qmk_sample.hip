@@ -16,22 +16,29 @@
 // (G. Steele, D. Lea, C. Flood, "Fast splittable pseudorandom number generators", OOPSLA 2014).
 //
 // With a filter, a call is two launches over the row (three for top-p alone, whose masses need the
-// row's maximum first; in the generate loop that is the decode step's own greedy logit over T):
+// row's maximum first; in the generate loop that is the decode step's own greedy logit over T), and one
+// between them that rarely does anything:
 // - k_first histograms the slices over 2048 bins in LDS, adds the non-zero bins to the row's with
 //   integer atomics, and the last workgroup of the row (a ticket counter) finds the bin that holds the
 //   threshold.  top-k: counts over the top 11 bits of the order-preserving 32-bit key of s;  top-p
-//   alone: masses over (max - s) in steps of 1/64, so that a bin holds few scores wherever the
-//   threshold lies;
-// - k_finish draws among the scores above that bin, which are kept for certain, and collects the
-//   bin's own (with both filters: every score from that bin up) as candidates; the row's last
-//   workgroup finds the exact thresholds among these by radix descent in LDS, draws among those that
-//   stay and writes the token.
-// Candidates beyond kSampleCand (scores of the threshold's bin within 1/64 of each other by the
-// thousand, but not equal: equal ones need no list) are found again in the logits by the last
-// workgroup, one pass over the row per digit.  top-k above kFinishTopK keeps the general form: radix
-// descent over the whole row, 8 bits per launch (k_hist, 4 launches per threshold, then k_draw).
-// Each launch costs 7-9 us whatever it does, which is what bounds a call: four rows of 151,936
-// scores, top-k 50 + top-p 0.9: 10 launches 84 us -> 2 launches 24.4.
+//   alone: masses over (max - s) in steps of 1/64;
+// - k_finer does the same within that bin, 2048 finer ones, where it holds more than kFinerAbove scores: a
+//   key bin is up to a quarter of the score wide, so logits far from 0 for their spread fill it, and so
+//   do flat ones at a high temperature;
+// - k_finish draws among the scores above the bin, which are kept for certain (with both filters it
+//   lists them, fewer than top_k), and lists the bin's own; the row's last workgroup finds the exact
+//   thresholds among these by radix descent in LDS, draws among those that stay and writes the token.
+//   A bin of equal scores, however many (a mask's -inf, bf16 logits), needs no list: they stay or go as one.
+// A bin of more than kSampleCand scores even so, not equal but closer than 2^-13 of their value (top-p
+// alone: 2^-17), is found again in the logits by the last workgroup, one pass over the row per digit.
+// top-k above kFinishTopK keeps the general form: radix descent over the whole row, 8 bits per launch
+// (k_hist, 4 launches per threshold, then k_draw).
+// A launch that works costs 7-9 us whatever it does, which is what bounds a call; k_finer without work 2.3.
+// Four rows of 151,936 scores, T 0.8, us, general form -> two launches without k_finer -> now: N(0,2) with a
+// few raised, top-k 50 + top-p 0.9 83 -> 24.6 -> 28.2, top-k 4096 + top-p 0.95 91 -> 836 -> 59; N(10,2), top-k
+// 200 + top-p 0.9 84 -> 727 -> 36; all but ten masked, top-k 50 + top-p 0.9 91 -> 1005 -> 43; N(0,0.01), top-p
+// 0.9 60 -> 673 -> 44.  The general form is faster for 152,000 distinct scores within 0.01 (one row, top-k
+// 4096: 36 against 44).
 
 #include <hip/hip_runtime.h>
 
@@ -280,25 +287,17 @@ __device__ __forceinline__ void put_token(const Args& a, const Block& b, int tok
   }
   w->z = w->target = w->need = w->best = w->tied = 0;
   w->maxkey = w->prefix = w->mask = w->kmin = w->pmin = 0;
-  w->ncand = w->candmin = w->candmax = 0;
+  w->nabove = w->nbin = w->binmin = w->binmax = w->abovemax = w->finer = 0;
   w->ticket = 0;
 }
 
 constexpr int kFirstShift = 21;       // top-k: bins are the key's top 11 bits
 constexpr float kStepsPerUnit = 64.f;  // top-p alone: bins are steps of max - s
-constexpr int kFinishTopK = 4096;     // largest top-k whose candidates are expected to fit
-constexpr int kLocalCand = 1024;      // candidates one workgroup collects
+constexpr int kFinerBits = 11;          // finer bins: the next 11, steps of 1/2048 of those
+constexpr int kFinishTopK = kSampleCand;  // largest top-k whose scores above the threshold's bin fit the list
+constexpr unsigned long long kFinerAbove = 512;  // scores in the bin from which k_finer pays
 constexpr int kUnroll = 8;            // logits in flight per thread
 static_assert(kSampleBins == 8 * kThreads, "eight bins per thread");
-
-// Bin of a score, larger for larger scores.  LINEAR: 2047 - floor((max - s) * 64), 0 from 32 below the
-// maximum on (whose mass rounds to 0), and for a NaN difference.
-template <bool LINEAR>
-__device__ __forceinline__ uint32_t first_bin(float s, uint32_t key, float mx) {
-  if (!LINEAR) return key >> kFirstShift;
-  const float d = (mx - s) * kStepsPerUnit;
-  return d < (float)(kSampleBins - 1) ? (uint32_t)(kSampleBins - 1) - (uint32_t)(int)fmaxf(d, 0.f) : 0u;
-}
 
 // f(v, logit) for this thread's elements v = v0 + threadIdx.x, + kThreads, .. of [v0, v1), kUnroll
 // loads at a time
@@ -335,26 +334,77 @@ __device__ __forceinline__ unsigned long long block_sum_after(unsigned long long
   return after;
 }
 
+// Bin of a score, larger for larger scores.  Key bins: the key's top bits.  LINEAR: the steps of max - s,
+// counted down from the top bin, 0 from 32 below the maximum on (whose mass rounds to 0), and for a NaN
+// difference.  Scaling by powers of two is exact, so a finer bin lies in one first one.
+// Level 0: the first 2048 bins, 1: the 2048 in each of those (22 bits).
+template <bool LINEAR>
+__device__ __forceinline__ uint32_t level_bin(float s, uint32_t key, float mx, int level) {
+  uint32_t b = key >> (kFirstShift - kFinerBits);
+  if (LINEAR) {
+    const float d = (mx - s) * (kStepsPerUnit * kSampleBins);
+    b = d < (float)(kSampleBins - 1) * kSampleBins ? kSampleBins * kSampleBins - 1 - (uint32_t)(int)fmaxf(d, 0.f) : 0u;
+  }
+  return level ? b : b >> kFinerBits;
+}
+
+// The last workgroup's end of a histogram pass.  Suffix sums: a thread holds bins 8t..8t+7.  The bin is the
+// largest d >= 1 whose sum above + S[d] reaches what is sought, else 0 (S does not increase with d, so d is
+// the count of such d); sought(total) says what.  Clears the histogram, and calls f(d, S[d + 1], h[d], sought)
+// in one thread.
+template <class P, class F>
+__device__ __forceinline__ void select_bin(unsigned long long* hist, unsigned long long above, P&& sought_of, F&& f) {
+  __shared__ unsigned int ndig;
+  const int t = threadIdx.x;
+  if (t == 0) ndig = 0;
+  unsigned long long h[8], own = 0, total;
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    h[i] = load_u64(&hist[8 * t + i]);
+    own += h[i];
+  }
+  const unsigned long long after = block_sum_after(own, total), sought = sought_of(total);
+  unsigned long long run = after, over[8];
+  unsigned int n = 0;
+#pragma unroll
+  for (int i = 7; i >= 0; i--) {
+    over[i] = run;  // S[8t + i + 1]
+    run += h[i];
+    n += (8 * t + i >= 1 && above + run >= sought) ? 1u : 0u;
+    hist[8 * t + i] = 0;  // ready for the next pass
+  }
+  if (n) atomicAdd(&ndig, n);
+  __syncthreads();
+  const int d = (int)ndig;
+  if (d >> 3 == t) {
+    unsigned long long ov = 0, hd = 0;
+#pragma unroll
+    for (int i = 0; i < 8; i++) {
+      ov = (d & 7) == i ? over[i] : ov;
+      hd = (d & 7) == i ? h[i] : hd;
+    }
+    f(d, ov, hd, sought);
+  }
+}
+
 // MASS: the masses of the whole row over linear bins (top-p alone); else counts over key bins (top-k).
 // Leaves the threshold's bin in w->prefix, the rank still sought in it (top-k) or the mass above it
-// (top-p) in w->need, and the mass sought in w->target.
+// (top-p) in w->need, the mass sought in w->target, and in w->finer whether k_finer is to cut the bin.
 template <bool MASS>
 __global__ void __launch_bounds__(kThreads) k_first(Args a) {
   typedef typename std::conditional<MASS, unsigned long long, unsigned int>::type bin_t;
   __shared__ bin_t wh[kSampleBins];
-  __shared__ unsigned int ndig;
   Block b;
   if (!setup(a, b)) return;
   SampleWork* w = b.w;
   const float T = a.sp.temperature, mx = MASS ? row_max(a, b) : 0.f;
 #pragma unroll
   for (int i = 0; i < 8; i++) wh[threadIdx.x + kThreads * i] = 0;
-  if (threadIdx.x == 0) ndig = 0;
   __syncthreads();
   for_slice(b.x, b.v0, b.v1, [&](int, float l) {
     const float s = __fdiv_rn(l, T);
     const bin_t m = MASS ? (bin_t)mass_of(s, mx) : (bin_t)1;
-    if (!MASS || m) atomicAdd(&wh[first_bin<MASS>(s, key32(s), mx)], m);
+    if (!MASS || m) atomicAdd(&wh[level_bin<MASS>(s, key32(s), mx, 0)], m);
   });
   __syncthreads();
 #pragma unroll
@@ -363,89 +413,110 @@ __global__ void __launch_bounds__(kThreads) k_first(Args a) {
     if (h) atomicAdd(&b.ls->hist[threadIdx.x + kThreads * i], h);
   }
   if (!last_block(w)) return;
-
-  // suffix sums: this thread holds bins 8t..8t+7.  The bin is the largest d >= 1 whose suffix sum S[d]
-  // reaches what is sought, else 0 (S does not increase with d, so d is the count of such d)
-  const int t = threadIdx.x;
-  unsigned long long h[8], own = 0, total;
-#pragma unroll
-  for (int i = 0; i < 8; i++) {
-    h[i] = load_u64(&b.ls->hist[8 * t + i]);
-    own += h[i];
-  }
-  const unsigned long long after = block_sum_after(own, total);
-  unsigned long long sought = (unsigned long long)a.sp.top_k;
-  if (MASS) {
-    sought = (unsigned long long)((double)a.sp.top_p * (double)total);
-    if (sought < 1) sought = 1;
-  }
-  unsigned long long run = after, above[8];
-  unsigned int n = 0;
-#pragma unroll
-  for (int i = 7; i >= 0; i--) {
-    above[i] = run;  // S[8t + i + 1]
-    run += h[i];
-    n += (8 * t + i >= 1 && run >= sought) ? 1u : 0u;
-    b.ls->hist[8 * t + i] = 0;  // ready for the next call
-  }
-  if (n) atomicAdd(&ndig, n);
-  __syncthreads();
-  const int d = (int)ndig;
-  if (d >> 3 == t) {
-    unsigned long long ab = 0;
-#pragma unroll
-    for (int i = 0; i < 8; i++) ab = (d & 7) == i ? above[i] : ab;
-    w->prefix = (unsigned int)d;
-    w->need = MASS ? ab : sought - ab;
-    w->target = sought;
-    w->ticket = 0;
-  }
+  select_bin(
+      b.ls->hist, 0,
+      [&](unsigned long long total) {
+        if (!MASS) return (unsigned long long)a.sp.top_k;
+        const unsigned long long p = (unsigned long long)((double)a.sp.top_p * (double)total);
+        return p < 1 ? 1ull : p;
+      },
+      [&](int d, unsigned long long over, unsigned long long h, unsigned long long sought) {
+        w->prefix = (unsigned int)d;
+        w->need = MASS ? over : sought - over;
+        w->target = sought;
+        // scores in the bin: its count; for a mass at most that over the smallest one's
+        const unsigned long long least = MASS ? mass_of(-(float)(kSampleBins - d) / kStepsPerUnit, 0.f) : 1ull;
+        w->finer = (MASS && (d == 0 || least == 0)) || h > kFinerAbove * least;
+        w->ticket = 0;
+      });
 }
 
-// Whole draw of a filtered call (after k_first): TOPK, TOPP the filters that are on.
+// The threshold's bin among the 2048 finer ones within k_first's, as k_first (if that asked for it).
+template <bool MASS>
+__global__ void __launch_bounds__(kThreads) k_finer(Args a) {
+  typedef typename std::conditional<MASS, unsigned long long, unsigned int>::type bin_t;
+  __shared__ bin_t wh[kSampleBins];
+  if (load_u32(&a.work[blockIdx.y].finer) == 0) return;
+  Block b;
+  if (!setup(a, b)) return;
+  SampleWork* w = b.w;
+  const float T = a.sp.temperature, mx = MASS ? row_max(a, b) : 0.f;
+  const uint32_t fd = load_u32(&w->prefix);
+#pragma unroll
+  for (int i = 0; i < 8; i++) wh[threadIdx.x + kThreads * i] = 0;
+  __syncthreads();
+  for_slice(b.x, b.v0, b.v1, [&](int, float l) {
+    const float s = __fdiv_rn(l, T);
+    const uint32_t bin = level_bin<MASS>(s, key32(s), mx, 1);
+    if (bin >> kFinerBits == fd) atomicAdd(&wh[bin & (kSampleBins - 1)], MASS ? (bin_t)mass_of(s, mx) : (bin_t)1);
+  });
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < 8; i++) {
+    const unsigned long long h = wh[threadIdx.x + kThreads * i];
+    if (h) atomicAdd(&b.ls->hist[threadIdx.x + kThreads * i], h);
+  }
+  if (!last_block(w)) return;
+  const unsigned long long need = load_u64(&w->need), target = load_u64(&w->target);
+  __syncthreads();  // read by every thread before one of them writes them
+  select_bin(
+      b.ls->hist, MASS ? need : 0, [&](unsigned long long) { return MASS ? target : need; },
+      [&](int d, unsigned long long over, unsigned long long, unsigned long long) {
+        w->prefix = fd << kFinerBits | (unsigned int)d;
+        w->need = MASS ? need + over : need - over;
+        w->ticket = 0;
+      });
+}
+
+// Whole draw of a filtered call (after k_first and k_finer): TOPK, TOPP the filters that are on.
 template <bool TOPK, bool TOPP>
 __global__ void __launch_bounds__(kThreads) k_finish(Args a) {
   constexpr bool LINEAR = !TOPK, BOTH = TOPK && TOPP;
-  __shared__ unsigned long long local[kLocalCand];
-  __shared__ uint32_t ck[kSampleCand];
+  // tokens above the bin and in it: this workgroup's, then, in the row's last one, the row's, with their keys
+  __shared__ uint32_t tk[2][kSampleCand], ck[2 * kSampleCand];
   __shared__ unsigned long long hs[128];
-  __shared__ unsigned int nlocal, base, digit;
+  __shared__ unsigned int nlocal[2], base[2], digit;
   __shared__ unsigned long long s_above;
   Block b;
   if (!setup(a, b)) return;
   SampleWork* w = b.w;
   const float T = a.sp.temperature;
   const uint32_t fd = load_u32(&w->prefix);
+  const int level = load_u32(&w->finer) ? 1 : 0;
   float mx = LINEAR ? row_max(a, b) : 0.f;
   const uint64_t dbase = draw_base(a.sp.seed, b.counter);
-  if (threadIdx.x == 0) nlocal = 0;
+  if (threadIdx.x < 2) nlocal[threadIdx.x] = 0;
   __syncthreads();
-  // best: draws of the scores that stay for certain; tied: of the candidates, which all stay if
-  // their keys are the same
+  // best: draws of the scores that stay for certain; tied: of the bin's, which stay or go as one if their
+  // keys are the same
   unsigned long long best = 0, tied = 0;
-  uint32_t kmn = 0xffffffffu, kmx = 0;
-  auto draw = [&](int v, float l) {
-    return ((unsigned long long)gumbel_key(l, T, dbase, v) << 32) | (0xffffffffu - (uint32_t)v);
+  uint32_t kmn = 0xffffffffu, kmx = 0, amx = 0;
+  auto draw = [&](int v, float s) {
+    return ((unsigned long long)gumbel_key_score(s, dbase, v) << 32) | (0xffffffffu - (uint32_t)v);
   };
   for_slice(b.x, b.v0, b.v1, [&](int v, float l) {
     const float s = __fdiv_rn(l, T);
-    const uint32_t k = key32(s), bin = first_bin<LINEAR>(s, k, mx);
+    const uint32_t k = key32(s), bin = level_bin<LINEAR>(s, k, mx, level);
     if (bin < fd) return;
-    if (!BOTH && bin > fd) {
-      const unsigned long long g = draw(v, l);
-      best = g > best ? g : best;
-      return;
+    const int in = bin == fd;
+    if (!BOTH || in) {
+      const unsigned long long g = draw(v, s);
+      if (in) tied = g > tied ? g : tied;
+      else best = g > best ? g : best;
     }
-    kmn = k < kmn ? k : kmn;
-    kmx = k > kmx ? k : kmx;
-    const unsigned long long g = draw(v, l);
-    tied = g > tied ? g : tied;
-    const unsigned int i = atomicAdd(&nlocal, 1u);
-    if (i < (unsigned)kLocalCand) local[i] = ((unsigned long long)k << 32) | (uint32_t)v;
+    if (in) {
+      kmn = k < kmn ? k : kmn;
+      kmx = k > kmx ? k : kmx;
+    } else {
+      amx = k > amx ? k : amx;
+      if (!BOTH) return;
+    }
+    const unsigned int i = atomicAdd(&nlocal[in], 1u);
+    if (i < (unsigned)kSampleCand) tk[in][i] = (uint32_t)v;
   });
   __syncthreads();
-  // more than the workgroup can list: counted as more than the row can
-  if (threadIdx.x == 0 && nlocal) base = atomicAdd(&w->ncand, nlocal <= (unsigned)kLocalCand ? nlocal : (unsigned)kSampleCand + nlocal);
+  if (threadIdx.x < 2 && nlocal[threadIdx.x])
+    base[threadIdx.x] = atomicAdd(threadIdx.x ? &w->nbin : &w->nabove, nlocal[threadIdx.x]);
   auto mx64 = [](unsigned long long p, unsigned long long q) { return p > q ? p : q; };
   best = block_reduce_u64(best, mx64);
   __syncthreads();
@@ -454,57 +525,75 @@ __global__ void __launch_bounds__(kThreads) k_finish(Args a) {
   const unsigned long long ends = block_reduce_u64(((unsigned long long)(~kmn) << 32), mx64);
   __syncthreads();
   kmx = (uint32_t)block_reduce_u64((unsigned long long)kmx, mx64);
-  if (nlocal && nlocal <= (unsigned)kLocalCand)
-    for (unsigned int i = threadIdx.x; i < nlocal; i += kThreads)
-      if (base + i < (unsigned)kSampleCand)
-        __hip_atomic_store(&b.ls->cand[base + i], local[i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (BOTH) {
+    __syncthreads();
+    amx = (uint32_t)block_reduce_u64((unsigned long long)amx, mx64);
+  }
+  for (int q = 0; q < 2; q++) {
+    uint32_t* const list = q ? b.ls->bin : b.ls->above;
+    const unsigned int n = min(nlocal[q], (unsigned)kSampleCand);
+    for (unsigned int i = threadIdx.x; i < n; i += kThreads)
+      if (base[q] + i < (unsigned)kSampleCand)
+        __hip_atomic_store(&list[base[q] + i], tk[q][i], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
   if (threadIdx.x == 0) {
     if (best) atomicMax(&w->best, best);
-    if (nlocal) {
+    if (BOTH && nlocal[0]) atomicMax(&w->abovemax, amx);
+    if (nlocal[1]) {
       atomicMax(&w->tied, tied);
-      atomicMax(&w->candmin, (unsigned int)(ends >> 32));
-      atomicMax(&w->candmax, kmx);
+      atomicMax(&w->binmin, (unsigned int)(ends >> 32));
+      atomicMax(&w->binmax, kmx);
     }
   }
   if (!last_block(w)) return;
 
   // ---- the row's last workgroup
-  const unsigned int nc = load_u32(&w->ncand);
-  const bool listed = nc <= (unsigned)kSampleCand;
-  const uint32_t cmin = ~load_u32(&w->candmin), cmax = load_u32(&w->candmax);
+  const unsigned int na = BOTH ? load_u32(&w->nabove) : 0u, nb = load_u32(&w->nbin);  // na < top_k <= kSampleCand
+  const uint32_t bmin = ~load_u32(&w->binmin), bmax = load_u32(&w->binmax);
+  const bool same = bmin == bmax, listed = nb <= (unsigned)kSampleCand;  // one score, however often; all in the list
   best = load_u64(&w->best);
-  if (cmin == cmax) {  // one score, however often: it stays
-    const unsigned long long g = load_u64(&w->tied);
-    best = g > best ? g : best;
+  tied = load_u64(&w->tied);
+  if (same && !BOTH) {  // the threshold is that score: it stays
+    best = tied > best ? tied : best;
   } else {
-    if (listed)
-      for (unsigned int i = threadIdx.x; i < nc; i += kThreads) ck[i] = (uint32_t)(load_u64(&b.ls->cand[i]) >> 32);
+    // the listed scores: those above the bin, then its own
+    uint32_t* const rtk = &tk[0][0];
+    const unsigned int nl = na + (listed && !same ? nb : 0u);
+    for (unsigned int i = threadIdx.x; i < nl; i += kThreads) {
+      const uint32_t v = load_u32(i < na ? &b.ls->above[i] : &b.ls->bin[i - na]);
+      rtk[i] = v;
+      ck[i] = key32(__fdiv_rn(b.x[v], T));
+    }
     __syncthreads();
-    // f(key) for every candidate
-    auto each = [&](auto&& f) {
-      if (listed) {
-        for (unsigned int i = threadIdx.x; i < nc; i += kThreads) f(ck[i]);
-      } else {
-        for_slice(b.x, 0, a.V, [&](int, float l) {
+    // f(key, how many, token or -1) for the scores of the bin, or also for those above it (the list from 0)
+    auto each = [&](bool all, auto&& f) {
+      for (unsigned int i = threadIdx.x + (all ? 0u : na); i < nl; i += kThreads) f(ck[i], 1u, (int)rtk[i]);
+      if (same) {
+        if (threadIdx.x == 0) f(bmin, nb, -1);
+      } else if (!listed) {
+        for_slice(b.x, 0, a.V, [&](int v, float l) {
           const float s = __fdiv_rn(l, T);
-          const uint32_t k = key32(s), bin = first_bin<LINEAR>(s, k, mx);
-          if (BOTH ? bin >= fd : bin == fd) f(k);
+          const uint32_t k = key32(s);
+          if (level_bin<LINEAR>(s, k, mx, level) == fd) f(k, 1u, v);
         });
       }
     };
-    // the largest key with (sum above the prefix +) the sum over candidates >= it reaching `sought`,
-    // among candidates >= kmin that start with `prefix` (bits of `mask`), 7 bits at a time
-    auto descend = [&](bool mass, uint32_t prefix, uint32_t mask, int hi, unsigned long long above,
-                       unsigned long long sought, uint32_t kmin) {
+    // the largest key with (a sum above +) the sum over the bin's scores, or all, of keys >= it reaching
+    // `sought`, among the keys from kmin to kmax: 7 bits at a time of those in which the two differ
+    auto descend = [&](bool mass, bool all, uint32_t kmin, uint32_t kmax, unsigned long long above,
+                       unsigned long long sought) {
+      int hi = kmin == kmax ? 0 : 32 - __clz((int)(kmin ^ kmax));
+      uint32_t mask = hi == 32 ? 0u : ~0u << hi, prefix = kmax & mask;
       while (hi > 0) {
         const int wd = hi < 7 ? hi : 7, sh = hi - wd;
         const uint32_t dm = (1u << wd) - 1u;
         for (int i = threadIdx.x; i < 128; i += kThreads) hs[i] = 0;
         __syncthreads();
-        each([&](uint32_t k) {
+        auto count = [&](uint32_t k, unsigned int n, int) {
           if ((k & mask) == prefix && k >= kmin)
-            atomicAdd(&hs[(k >> sh) & dm], mass ? mass_of(from_key32(k), mx) : 1ull);
-        });
+            atomicAdd(&hs[(k >> sh) & dm], mass ? mass_of(from_key32(k), mx) * n : (unsigned long long)n);
+        };
+        each(all, count);
         __syncthreads();
         if (threadIdx.x < 64) {  // bins 2l, 2l + 1 per lane; suffix sums, then the digit
           const int lane = threadIdx.x;
@@ -533,45 +622,36 @@ __global__ void __launch_bounds__(kThreads) k_finish(Args a) {
     };
     uint32_t keep = 0;
     if (TOPK) {
-      // the rank still sought in the bin: `sought` counts from the bin's top
-      keep = descend(false, fd << kFirstShift, ~0u << kFirstShift, kFirstShift, 0, load_u64(&w->need), 0);
+      // the rank still sought in the bin: it counts from the bin's top
+      keep = descend(false, false, bmin, bmax, 0, load_u64(&w->need));
       if (BOTH) {
-        mx = from_key32(cmax);
+        const uint32_t kmax = na ? load_u32(&w->abovemax) : bmax;
+        mx = from_key32(kmax);
         unsigned long long z = 0;
-        each([&](uint32_t k) {
-          if (k >= keep) z += mass_of(from_key32(k), mx);
+        each(true, [&](uint32_t k, unsigned int n, int) {
+          if (k >= keep) z += mass_of(from_key32(k), mx) * n;
         });
         z = block_reduce_u64(z, [](unsigned long long p, unsigned long long q) { return p + q; });
         unsigned long long target = (unsigned long long)((double)a.sp.top_p * (double)z);
         if (target < 1) target = 1;
-        const uint32_t pmin = descend(true, 0, 0, 32, 0, target, keep);
+        const uint32_t pmin = descend(true, true, keep, kmax, 0, target);
         keep = pmin > keep ? pmin : keep;
       }
     } else {
-      keep = descend(true, 0, 0, 32, load_u64(&w->need), load_u64(&w->target), 0);
+      keep = descend(true, false, bmin, bmax, load_u64(&w->need), load_u64(&w->target));
     }
     unsigned long long g = 0;
-    if (listed) {
-      for (unsigned int i = threadIdx.x; i < nc; i += kThreads)
-        if (ck[i] >= keep) {
-          const int v = (int)(uint32_t)load_u64(&b.ls->cand[i]);
-          const unsigned long long q = draw(v, b.x[v]);
-          g = q > g ? q : g;
-        }
-    } else {
-      for_slice(b.x, 0, a.V, [&](int v, float l) {
-        const float s = __fdiv_rn(l, T);
-        const uint32_t k = key32(s), bin = first_bin<LINEAR>(s, k, mx);
-        if ((BOTH ? bin >= fd : bin == fd) && k >= keep) {
-          const unsigned long long q = draw(v, l);
-          g = q > g ? q : g;
-        }
-      });
-    }
+    each(true, [&](uint32_t k, unsigned int, int v) {
+      if (k < keep) return;
+      const unsigned long long q = v < 0 ? tied : draw(v, from_key32(k));
+      g = q > g ? q : g;
+    });
     __syncthreads();
     g = block_reduce_u64(g, mx64);
     best = g > best ? g : best;
   }
+  // the bin's list lies where the next call's histogram does
+  for (unsigned int i = threadIdx.x; i < min(nb, (unsigned)kSampleCand); i += kThreads) b.ls->bin[i] = 0;
   __syncthreads();  // every wave has read the work that put_token clears
   if (threadIdx.x == 0) put_token(a, b, (int)(0xffffffffu - (uint32_t)best));
 }
@@ -628,8 +708,13 @@ int launch(const Args& a, int rows, hipStream_t stream) {
     const bool topp = sp.top_p > 0.f && sp.top_p < 1.f;
     if (topp && !a.st && (!topk || sp.top_k > kFinishTopK)) hipLaunchKernelGGL(k_max, grid, block, 0, stream, a);
     if (two_launches(sp, a.V)) {
-      if (topk) hipLaunchKernelGGL(k_first<false>, grid, block, 0, stream, a);
-      else hipLaunchKernelGGL(k_first<true>, grid, block, 0, stream, a);
+      if (topk) {
+        hipLaunchKernelGGL(k_first<false>, grid, block, 0, stream, a);
+        hipLaunchKernelGGL(k_finer<false>, grid, block, 0, stream, a);
+      } else {
+        hipLaunchKernelGGL(k_first<true>, grid, block, 0, stream, a);
+        hipLaunchKernelGGL(k_finer<true>, grid, block, 0, stream, a);
+      }
       if (topk && topp) hipLaunchKernelGGL((k_finish<true, true>), grid, block, 0, stream, a);
       else if (topk) hipLaunchKernelGGL((k_finish<true, false>), grid, block, 0, stream, a);
       else hipLaunchKernelGGL((k_finish<false, true>), grid, block, 0, stream, a);
