@@ -193,9 +193,8 @@ def test_batch_generate_matches_oracle_streams(shape, exact06, weights_cpu, weig
 
 
 def test_long_two_sequence_prefill_mfma_attention(shape, exact06, weights_gpu):
-    """1100 tokens of two sequences (600 + 500) in one forward, 2 layers: the MFMA attention
-    (1024+ tokens) over 64-token tiles, a partial last tile and the tile holding the end of
-    sequence 0 and the start of sequence 1 (row-by-row fallback); every 50th row of each
+    """1100 tokens of two sequences (600 + 500) in one forward, 2 layers: the MFMA attention over
+    64-token tiles, each sequence's cut from its own start, with a partial last one; every 50th row of each
     sequence and each sequence's last row against its own oracle, and a repeat bit-exact."""
     from qwen_megakernel.model import BatchDecoder
     from qwen_megakernel.weights import make_prompt
@@ -229,8 +228,8 @@ def test_long_two_sequence_prefill_mfma_attention(shape, exact06, weights_gpu):
 
 
 def test_long_single_sequence_prefill_mfma_attention(shape, exact06, weights_gpu):
-    """A 2048-token prompt of one sequence, 2 layers: the MFMA attention's 32 tiles in 16 pairs
-    (tiles i and 31 - i in one workgroup per query head), rows 0..2047 in every tile; every 97th
+    """A 2048-token prompt of one sequence, 2 layers: the MFMA attention's 32 tiles shared by 16
+    workgroups per query head (the longest with the shortest), rows 0..2047 in every tile; every 97th
     row and the last against the oracle, and a repeat bit-exact."""
     from qwen_megakernel.model import BatchDecoder
     from qwen_megakernel.weights import make_prompt
@@ -280,11 +279,12 @@ def test_prefill_all_matches_per_sequence_prefill(shape, weights_gpu):
         check_row(t, ("step", b), l2[b].cpu(), s1[b], l1[b], bar=LAYERS28)
 
 
-@pytest.mark.parametrize("n", [2, 8, 40, 150],
-                         ids=["2tok-split", "8tok-mfma-chunks", "40tok-mfma-chunks", "150tok-mfma-chunks"])
+@pytest.mark.parametrize("n", [2, 8, 20, 40, 150],
+                         ids=["2tok-split", "8tok-split", "20tok-mfma-chunks", "40tok-mfma-chunks",
+                              "150tok-mfma-chunks"])
 def test_long_context_prefill(shape, exact06, weights_gpu, n):
-    """Prefill after an injected N(0,1) cache of 2100 positions: 2 tokens take the split attention
-    (34 workgroups per head and token); 8, 40 and 150 tokens (one, one and three 64-token tiles,
+    """Prefill after an injected N(0,1) cache of 2100 positions: 2 and 8 tokens take the split attention
+    (17 chunks per head and token); 20, 40 and 150 tokens (one, one and three 64-token tiles,
     the last partial) the MFMA attention with its keys in chunks over the context (too few tiles
     to fill the chip)."""
     from qwen_megakernel.weights import make_kv_prefill, make_prompt
@@ -345,13 +345,15 @@ def test_long_prompt_after_long_context(shape, exact06, weights_gpu):
 
 @pytest.mark.parametrize(
     "n,start",
-    [(31, 190), (32, 100), (33, 300), (320, 0), (700, 0), (64, 2000), (1, 3000), (3, 3000)],
-    ids=["split-31@190", "rows-32@100", "mfma-chunks-33@300", "mfma-chunks-320@0", "mfma-pairs-700@0",
-         "mfma-chunks-64@2000", "split-1@3000", "mfma-chunks-3@3000"])
+    [(31, 190), (32, 100), (33, 300), (320, 0), (640, 0), (700, 0), (64, 2000), (1, 3000), (3, 3000), (10, 3000),
+     (11, 3000)],
+    ids=["split-31@190", "rows-32@100", "mfma-chunks-33@300", "mfma-chunks-320@0", "mfma-short-640@0",
+         "mfma-tiles-700@0", "mfma-chunks-64@2000", "split-1@3000", "split-3@3000", "split-10@3000",
+         "mfma-chunks-11@3000"])
 def test_attention_form_matrix(shape, exact06, weights_gpu, n, start):
     """One prompt of n tokens after `start` prefilled positions, 2 layers, for each attention form
-    the forward picks (the row kernel, the per-token context split, the MFMA attention in tile pairs
-    or over key chunks) around the thresholds between them: the first, middle and last rows and
+    the forward picks (the row kernel, the per-token context split, the MFMA attention over whole tiles
+    or key chunks) around the thresholds between them: the first, middle and last rows and
     every 100th against the exact oracle at the literal bar, and the K/V rows."""
     from qwen_megakernel.weights import make_prompt
 
@@ -376,9 +378,9 @@ def test_attention_form_matrix(shape, exact06, weights_gpu, n, start):
 
 def test_long_context_prefill_rows_two_sequences(shape, exact06, weights_gpu):
     """Two sequences of 20 tokens each after injected N(0,1) caches of 2100 and 2060 positions, in
-    one forward with their tokens interleaved: no 64-token tile is one sequence, so every row takes
-    the row attention, which covers the contexts in two 2048-position chunks (scores recomputed per
-    pass).  Every row against its sequence's oracle."""
+    one forward with their tokens interleaved: every token is a run of its own, too short for a tile,
+    so each takes a workgroup per KV head beside the tile chunks.  Every row against its sequence's
+    oracle."""
     from dataclasses import replace
 
     from qwen_megakernel.model import BatchDecoder
@@ -413,8 +415,8 @@ def test_long_context_prefill_rows_two_sequences(shape, exact06, weights_gpu):
 @pytest.mark.parametrize("n,start", [(1, 0), (2, 0), (3, 0), (1, 150), (3, 150)],
                          ids=["1tok", "2tok", "3tok", "1tok-after-150", "3tok-after-150"])
 def test_prefill_few_tokens(shape, exact06, weights_gpu, n, start):
-    """Prompts of 1-3 tokens, 4 layers: the tiled GEMM's 128-row tile almost all repeats of the last
-    row (rows past T), the row attention from position 0 and the split attention after a
+    """Prompts of 1-3 tokens, 4 layers: a 16-row tile almost all repeats of the last row (rows past
+    T), the row attention from position 0 and the split attention after a
     150-token prefix; every row against the oracle at the literal bar, and the K/V rows."""
     from qwen_megakernel.weights import make_prompt
 
@@ -502,7 +504,7 @@ def test_invalid_entries_emit_minus_one(weights_gpu):
 def test_invalid_entries_in_a_long_prompt(weights_gpu):
     """A 1024-token prompt (the fused q/k/v and gate/up epilogues, the MFMA attention) with a token
     id outside the vocabulary at row 300 and a position outside max_context at row 700: those rows
-    emit -1 and write no cache row, the tiles holding them are redone row by row, the other rows
+    emit -1 and write no cache row, the tokens before and after them form tiles of their own, the other rows
     emit tokens, and a second identical forward gives the same tokens and logits."""
     from qwen_megakernel.weights import make_prompt
 
@@ -575,7 +577,7 @@ def test_decode_batch_16_sequences(shape, exact06, weights_gpu):
 
 
 def test_decode_batch_long_context_general_path(shape, exact06, weights_gpu):
-    """Contexts beyond the fused step's 4096 positions take the general path (split attention); two
+    """Contexts beyond the persistent kernel's take the multi-launch step, here 40 attention chunks; two
     sequences after injected N(0,1) caches of 5000 and 4200 positions, 2 layers, three steps."""
     from qwen_megakernel.model import BatchDecoder
     from qwen_megakernel.weights import make_kv_prefill
@@ -603,12 +605,10 @@ def test_decode_batch_long_context_general_path(shape, exact06, weights_gpu):
 
 
 @pytest.mark.parametrize("c0s", [(3900,), (3000, 17), (2900, 1, 2500, 40)],
-                         ids=["batch1-32splits", "batch2-16splits", "batch4-8splits"])
+                         ids=["batch1-31chunks", "batch2-24chunks", "batch4-23chunks"])
 def test_decode_batch_fused_split_attention_contexts(shape, exact06, weights_gpu, c0s):
-    """The fused step's attention splits each (sequence, KV head) over S = 256 / (8 B) workgroups.
-    Injected N(0,1) caches: 2900-3900 positions give a split two or three 128-position batches
-    (its running-maximum rescale), and 1, 17 or 40 positions leave some of the S splits empty.
-    2 layers, three steps, every sequence against the exact oracle on its own cache."""
+    """The multi-launch step's attention over 128-position chunks, as many for every sequence as the longest
+    has: 1, 17 or 40 positions beside 2500-3900 leave all but one chunk empty.  Injected N(0,1) caches, 2 layers, three steps, every sequence against the exact oracle on its own cache."""
     from qwen_megakernel.model import BatchDecoder
     from qwen_megakernel.weights import make_kv_prefill
 
@@ -634,7 +634,7 @@ def test_decode_batch_fused_split_attention_contexts(shape, exact06, weights_gpu
 
 
 def test_decode_batch_equals_general_forward(weights_gpu):
-    """The fused decode step and forward_tokens (general path) on the same inputs: logits within
+    """The batched step and forward_tokens on the same inputs (one token per sequence): logits within
     the bar of each other and the same tokens up to near-ties."""
     from qwen_megakernel.model import BatchDecoder
     from qwen_megakernel.weights import make_prompt
@@ -673,7 +673,7 @@ def test_long_prefill_tiled_gemm(shape, exact06, weights_gpu, n):
     the oracle, 2 layers, and a second identical forward bit-exact.  128 tokens: 64-column tiles
     for all four projections, o and down split 16 ways over K; 200 tokens: 128-column tiles with
     a partial last row tile; 300 tokens: 128-column tiles and 64-column tiles for down; 450 tokens:
-    the MFMA attention (8 tiles in 4 pairs, a partial last tile)."""
+    the MFMA attention (8 tiles over key chunks, a partial last tile)."""
     from qwen_megakernel.weights import make_prompt
 
     layers = 2
@@ -698,7 +698,7 @@ def test_long_prefill_tiled_gemm(shape, exact06, weights_gpu, n):
 
 def test_prefill_emits_the_maximum_rows(shape, exact06, weights_gpu):
     """A 256-token prefill that emits every row: num_emit = 256, the most one forward takes (the
-    LM-head GEMM over 16 row tiles), 2 layers; every row's token and logits against the exact
+    LM head over four groups of 64 rows), 2 layers; every row's token and logits against the exact
     oracle at the literal bar, and the rows in any order (emit reversed) give the same rows."""
     from qwen_megakernel.weights import make_prompt
 

@@ -45,12 +45,47 @@ def _decode_steps(shape, exact06, weights_gpu, c0s, layers, max_seq, steps=2):
 
 
 @pytest.mark.parametrize("c0s", [(0, 1, 126, 127, 128), (255, 256, 300, 0, 129, 64),
-                                 tuple(range(110, 146, 2)), (383, 8200)],
-                         ids=["5seq-first-chunk-edge", "6seq-second-chunk-edge", "18seq-general", "2seq-65-chunks"])
+                                 tuple(range(110, 146, 2)), (383, 8200), tuple(range(112, 144)),
+                                 tuple(range(112, 144)) + (256,), tuple(range(0, 126, 3))[:34]],
+                         ids=["5seq-first-chunk-edge", "6seq-second-chunk-edge", "18seq-two-row-tiles", "2seq-65-chunks",
+                              "32seq-raw", "33seq-finished-q", "34seq-rows"])
 def test_decode_batch_attention_chunk_edges(shape, exact06, weights_gpu, c0s):
     """attn_chunk_*: contexts ending at, before and after a chunk's edge, a token in a chunk of its own,
-    more than 64 chunks (two rounds of pairs), from raw projections (up to 16 sequences) and finished q."""
+    more than 64 chunks (two rounds of pairs), from raw projections (up to 32 sequences, the most of gemm_rows)
+    and finished q (33, the first of the general projections), and contexts of at most 128 positions above
+    32 sequences (attention_rows)."""
     _decode_steps(shape, exact06, weights_gpu, c0s, layers=2, max_seq=(max(c0s) + 2 + 63) // 64 * 64)
+
+
+@pytest.mark.parametrize("batch", [32, 36])
+def test_decode_batch_invalid_entries(weights_gpu, batch):
+    """A token id outside the vocabulary and a position outside max_context among valid sequences, on both
+    sides of gemm_rows' limit: they emit -1 and write no cache row, and the other sequences' logits and rows are
+    the bits of the same step without them (every row of a batch is computed alike)."""
+    from qwen_megakernel.model import _Forward, _ops
+
+    V, layers, S = 151936, 2, 256
+    fwd = _Forward(_ops(), weights_gpu, layers)
+    g = torch.Generator("cuda").manual_seed(batch)
+    k0 = torch.randn(batch, layers, 8, S, 128, generator=g, device="cuda").bfloat16()
+    v0 = torch.randn(batch, layers, 8, S, 128, generator=g, device="cuda").bfloat16()
+    ids, pos = [31 * b for b in range(batch)], [(29 * b) % 200 for b in range(batch)]
+    got = []
+    for bad in (False, True):
+        i, p = list(ids), list(pos)
+        if bad:
+            i[3], p[batch - 2] = V, 200
+        k, v = k0.clone(), v0.clone()
+        out = torch.empty(batch, dtype=torch.int32, device="cuda")
+        logits = torch.empty(batch, V, dtype=torch.float32, device="cuda")
+        fwd.decode(_t(i), _t(p), out, logits, k, v, 200)
+        got.append((out, logits, k, v))
+    rest = [b for b in range(batch) if b not in (3, batch - 2)]
+    for a, b in zip(*got):
+        assert torch.equal(a[rest], b[rest])
+    out, _, k, v = got[1]
+    for b in (3, batch - 2):
+        assert int(out[b]) == -1 and torch.equal(k[b], k0[b]) and torch.equal(v[b], v0[b])
 
 
 def test_decode_batch_several_chunks(shape, exact06, weights_gpu):
