@@ -40,7 +40,6 @@ namespace batch {
 
 
 constexpr int kD = 128, kNQ = 16, kNKV = 8, kQS = kNQ * kD, kNQKV = (kNQ + 2 * kNKV) * kD;
-constexpr int kAttnChunk = 2048;  // one-kernel attention: scores of this many positions per LDS pass
 constexpr int kQT = 64;  // MFMA prefill attention: tokens per tile
 constexpr int kKB = 64, kKPad = kD + 8, kVPad = kKB + 8;  // its split passes: keys per block, LDS rows
 // Tokens of the smallest tile, and of the smallest that starts below kQT.  us per 4-layer forward, as tiles
@@ -49,7 +48,7 @@ constexpr int kKB = 64, kKPad = kD + 8, kVPad = kKB + 8;  // its split passes: k
 constexpr int kMinTile = 5, kMinTileNear = 16;
 constexpr int kLeftWave = 512;  // left tokens below this position may take a wave each
 constexpr int kMfmaAttnTokens = 320;   // prompts of this many tokens run attention_mfma
-constexpr int kMfmaAttnContext = 256;  // so do fewer tokens over this many positions of context
+constexpr int kMfmaAttnContext = 256;  // so do fewer tokens over this many positions of context; attention_rows below
 constexpr int kMaxAttnChunks = 16;    // split attention_mfma passes: a tile's key chunks at most
 constexpr int kSplitChunk = 128;  // split attention: positions per workgroup
 constexpr int kSplitBelow = 32;   // fewer tokens than this use the split attention ...
@@ -831,25 +830,25 @@ __global__ void __launch_bounds__(256) gate_up_finish(const float* __restrict__ 
 // bf16(bf16(q.k) * scale), softmax in fp32 with the global max, probabilities
 // rounded to bf16, P@V summed in fp32 and rounded to bf16.
 
-// Scores of positions [c0, cend) into sc[h][p - c0]; running max in m.
+// Scores of positions [0, n) into sc[h][p]; running max in m.
 // Each 16-lane row takes one position (16 lanes x 8 dims); a wave four.
-__device__ __forceinline__ void score_chunk(const uint16_t* kc, const u32x4 (&qv)[2], float scale, int c0, int cend,
+__device__ __forceinline__ void score_chunk(const uint16_t* kc, const u32x4 (&qv)[2], float scale, int n,
                                             float* sc0, float* sc1, float (&m)[2]) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, slot = lane >> 4, t16 = lane & 15;
-  for (int p = c0 + wave * 4 + slot; p < cend; p += 16) {
+  for (int p = wave * 4 + slot; p < n; p += 16) {
     const u32x4 kx = ld16(kc + (size_t)p * kD + 8 * t16);
     const float s0 = bf16r(bf16r(row16_sum(dot8(kx, qv[0], 0.f))) * scale);
     const float s1 = bf16r(bf16r(row16_sum(dot8(kx, qv[1], 0.f))) * scale);
     if (t16 == 0) {
-      sc0[p - c0] = s0;
-      sc1[p - c0] = s1;
+      sc0[p] = s0;
+      sc1[p] = s1;
     }
     m[0] = fmaxf(m[0], s0);
     m[1] = fmaxf(m[1], s1);
   }
 }
 
-// Probability-weighted V rows [0, n) of the chunk, dims 2*lane..+1 of both
+// Probability-weighted V rows [0, n), dims 2*lane..+1 of both
 // heads, wave w taking rows w, w+4, ...
 __device__ __forceinline__ void pv_chunk(const uint16_t* vc, const float* p0, const float* p1, int n,
                                          float (&acc)[2][2]) {
@@ -880,10 +879,18 @@ __device__ __forceinline__ float pv_merge_waves(const float (&acc)[2][2], float 
   return ((pv[0][h][d] + pv[1][h][d]) + pv[2][h][d]) + pv[3][h][d];
 }
 
-// attention_rows' work for token t and KV head g (both query heads)
-__device__ __forceinline__ void attention_row(const uint16_t* __restrict__ Q, const Tok tk, int t, int g, int t16,
-                                              int L, const Cache& c, float scale, uint16_t* __restrict__ out,
-                                              float (*sc)[kAttnChunk], float (*red)[4], float (*pv)[2][kD]) {
+// One workgroup per (token, KV head), both query heads, for contexts below kMfmaAttnContext.  It reserves LDS
+// for more scores than those need, so that seven workgroups run on a CU: with eight, 255 tokens take 358 us per
+// 4-layer forward, with seven 351 (100 and 200 tokens the same).
+constexpr int kRowScores = 2048;
+static_assert(kRowScores >= kMfmaAttnContext, "the scores of one context");
+__global__ void __launch_bounds__(256) attention_rows(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok,
+                                                      int L, Cache c, float scale, uint16_t* __restrict__ out) {
+  __shared__ float sc[2][kRowScores];
+  __shared__ float red[2][4];
+  __shared__ float pv[4][2][kD];
+  const int t = blockIdx.x, g = blockIdx.y, t16 = threadIdx.x & 15;
+  const Tok tk = tok[t];
   uint16_t* dst = out + (size_t)t * kQS + 2 * g * kD;  // both heads: 256 contiguous values
   if (!tk.valid) {
     dst[threadIdx.x] = 0;
@@ -896,54 +903,24 @@ __device__ __forceinline__ void attention_row(const uint16_t* __restrict__ Q, co
   u32x4 qv[2];
 #pragma unroll
   for (int h = 0; h < 2; h++) qv[h] = ld16(Q + (size_t)t * kQS + (2 * g + h) * kD + 8 * t16);
-  const int nch = (C + kAttnChunk - 1) / kAttnChunk;
   float M[2] = {-INFINITY, -INFINITY};
-  for (int ch = 0; ch < nch; ch++)
-    score_chunk(kc, qv, scale, ch * kAttnChunk, min(C, (ch + 1) * kAttnChunk), sc[0], sc[1], M);
+  score_chunk(kc, qv, scale, C, sc[0], sc[1], M);
   block_max2(M, red);
   float S[2] = {0.f, 0.f};
-  float dummy[2];
-  for (int ch = 0; ch < nch; ch++) {
-    const int c0 = ch * kAttnChunk, n = min(C - c0, kAttnChunk);
-    if (nch > 1) {
-      __syncthreads();
-      score_chunk(kc, qv, scale, c0, c0 + n, sc[0], sc[1], dummy);
-      __syncthreads();
-    }
-    for (int i = threadIdx.x; i < n; i += 256) {
-      S[0] += exp_acc(sc[0][i] - M[0]);
-      S[1] += exp_acc(sc[1][i] - M[1]);
-    }
+  for (int i = threadIdx.x; i < C; i += 256) {
+    S[0] += exp_acc(sc[0][i] - M[0]);
+    S[1] += exp_acc(sc[1][i] - M[1]);
   }
   block_sum2(S, red);
   const float inv0 = __fdiv_rn(1.0f, S[0]), inv1 = __fdiv_rn(1.0f, S[1]);
-  float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-  for (int ch = 0; ch < nch; ch++) {
-    const int c0 = ch * kAttnChunk, n = min(C - c0, kAttnChunk);
-    __syncthreads();
-    if (nch > 1) {
-      score_chunk(kc, qv, scale, c0, c0 + n, sc[0], sc[1], dummy);
-      __syncthreads();
-    }
-    for (int i = threadIdx.x; i < n; i += 256) {
-      sc[0][i] = bf16r(exp_acc(sc[0][i] - M[0]) * inv0);
-      sc[1][i] = bf16r(exp_acc(sc[1][i] - M[1]) * inv1);
-    }
-    __syncthreads();
-    pv_chunk(vc + (size_t)c0 * kD, sc[0], sc[1], n, acc);
+  for (int i = threadIdx.x; i < C; i += 256) {
+    sc[0][i] = bf16r(exp_acc(sc[0][i] - M[0]) * inv0);
+    sc[1][i] = bf16r(exp_acc(sc[1][i] - M[1]) * inv1);
   }
+  __syncthreads();
+  float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
+  pv_chunk(vc, sc[0], sc[1], C, acc);
   dst[threadIdx.x] = (uint16_t)f32_to_bf16(pv_merge_waves(acc, pv));
-}
-
-// One workgroup per (token, KV head).  Contexts longer than kAttnChunk are processed in chunks,
-// recomputing the scores in each of the three passes (max, sum, P@V) instead of keeping them.
-__global__ void __launch_bounds__(256) attention_rows(const uint16_t* __restrict__ Q, const Tok* __restrict__ tok,
-                                                      int L, Cache c, float scale, uint16_t* __restrict__ out) {
-  __shared__ float sc[2][kAttnChunk];
-  __shared__ float red[2][4];
-  __shared__ float pv[4][2][kD];
-  const int t = blockIdx.x;
-  attention_row(Q, tok[t], t, blockIdx.y, threadIdx.x & 15, L, c, scale, out, sc, red, pv);
 }
 
 // The attention of one token and KV head (both query heads) by NW waves: whole workgroups, or single waves
@@ -2548,11 +2525,11 @@ struct Gemm {
   int ksplit, tn;  // K splits, tile width (128 or 64 columns)
 };
 
-// Every projection of both models takes the LDS-tiled GEMM at any token count: N a multiple of the
+// Above kRowsMax tokens every projection of both models takes the LDS-tiled GEMM: N a multiple of the
 // 128-column tile and K a multiple of four 64-wide steps.  (A register-staged MFMA GEMM, one wave
 // per 16-row tile, ran below 96 tokens before; the tiled kernel on a 128-row tile whose rows past
-// T repeat the last one was faster at every count measured: 4 tokens 1.55 -> 1.34 ms per 0.6B
-// prefill, 64 tokens 2.09 -> 1.55, 80 tokens 2.43 -> 1.65.)
+// T repeat the last one was faster at every count measured: 64 tokens 2.09 -> 1.55 ms per 0.6B
+// prefill, 80 tokens 2.43 -> 1.65.)
 template <class M>
 constexpr bool tiled_shapes() {
   using Dm = Dims<M>;
@@ -2572,14 +2549,13 @@ int tiled_splits(int T, int N, int K) {
 }
 
 // 64-column tiles, for problems whose 128-column plan leaves CUs idle (narrow N at a few hundred
-// rows or fewer): K split (at most 16 ways, >= 2 steps of 64 each) until 256 workgroups run (512
-// for at most 16 rows, whose partials are small: 4-token prefill 1.245 -> 1.20 ms, 16 tokens 1.266
-// -> 1.245; at 64 tokens 512 was slower, 1.535 -> 1.585), while the fp32 partials
+// rows or fewer): K split (at most 16 ways, >= 2 steps of 64 each) until 256 workgroups run (at 64
+// tokens 512 was slower, a prefill 1.535 -> 1.585 ms), while the fp32 partials
 // (ksplit * T * N * 4 bytes) stay within twice the weight bytes (N * K * 2).
 int narrow_splits(int T, int N, int K) {
-  const long long tiles = (long long)((T + kTM - 1) / kTM) * (N / 64), target = T <= 16 ? 512 : 256;
+  const long long tiles = (long long)((T + kTM - 1) / kTM) * (N / 64);
   int ks = 1;
-  while (tiles * ks < target && ks * 2 <= kMaxSplit && K % (ks * 2 * kTK) == 0 && K / (ks * 2) >= 2 * kTK &&
+  while (tiles * ks < 256 && ks * 2 <= kMaxSplit && K % (ks * 2 * kTK) == 0 && K / (ks * 2) >= 2 * kTK &&
          (long long)ks * 2 * T * 4 <= 2LL * K * 2)
     ks *= 2;
   return ks;
@@ -2661,7 +2637,9 @@ bool mfma_attention(int T, int max_context, bool one_per_seq) {
          (T >= kMfmaAttnTokens || max_context >= kMfmaAttnContext);
 }
 
-// Up to this context attention_mfma_short's smaller blocks win (us per 4-layer forward, short against
+// Up to this context attention_mfma_short's smaller blocks win: a tile of five blocks of 128 keys or fewer has
+// too little to hide the first one's arrival and the sum of the four key parts behind, and half of its last
+// block is past the diagonal (us per 4-layer forward, short against
 // the 128-key form: 640 tokens 418 / 416, 768 456 / 452, 1024 526 / 516; four prompts of 411..613 tokens
 // 1283 / 1313).
 constexpr int kShortAttn = 640;
