@@ -1149,8 +1149,8 @@ __device__ __forceinline__ uint2 lds_read_tr4(const unsigned char* p) {
 // Blocks of 128 keys, four waves per row group, K and V straight from global memory into LDS: V stays
 // row-major there and is transposed by the reads.  What bounds it is the latency of a block's chain
 // (LDS reads, products, about 100 VALU instructions and 8 exponentials per wave and pass, barrier):
-// VALU work fills 49 % of the cycles, the MFMAs 14 %.  With blocks of 64 keys and 8 waves (two per
-// SIMD, staged through registers, V transposed on the way into LDS) it was 42 %.  Per 4-layer
+// VALU work fills 57 % of the cycles in which a CU has waves, the MFMAs 16 %.  Against blocks of 64 keys and 8
+// waves (two per SIMD, staged through registers, V transposed on the way into LDS), per 4-layer
 // forward, Qwen3-0.6B, us: 768 tokens 459 -> 448, 1024 529 -> 510, 2048 845 -> 805-821.  Measured on the
 // way: 8 waves and two workgroups per CU 85 us per layer at 2048 tokens, 8 waves and four stages 92,
 // this form with the heads in the grid's second dimension 80, as it is 76.
