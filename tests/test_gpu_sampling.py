@@ -72,8 +72,8 @@ def test_sample_rows_match_oracle_full_vocab(T, k, p):
 
 
 def test_sample_rows_beyond_one_launch_sequence_and_repeatable():
-    """300 rows: more than one launch sequence (256 rows each, the per-row work is reused and must
-    be left zeroed); every row matches the oracle, and a second call gives the same tokens."""
+    """300 rows: more than one launch sequence (128 rows each of a filtered draw, the per-row work is
+    reused and must be left zeroed); every row matches the oracle, and a second call gives the same tokens."""
     rng = np.random.default_rng(4)
     logits = (rng.standard_normal((300, 1000)) * 3).astype(np.float32)
     first = _compare(logits, 0.9, 20, 0.9, 99, list(range(300)))
