@@ -2822,7 +2822,8 @@ AttnChunks attn_chunks(const Args& a, const Layout& l) {
 // Workgroups of a launch at most: the call's context is a bound that its tokens may lie far below, and a
 // workgroup without a chunk still costs 2 ns, so above this each takes several chunks (one step, 4 layers,
 // us, one chunk each / several: 128 sequences at 100..200 with a bound of 4096 1010 / 423, of 201 430 both;
-// where the bound is the context, 256 sequences at 1000..1100 1295 / 1340, 64 at 1000..4000 790 / 790).
+// where the bound is the context, 16 sequences at 3000..8000 475 / 500, 32 at 100..7000 563 / 585, 256 at
+// 1000..1100 1276 / 1326: a chunk's rows are requested when the one before is done).
 // An odd number per (token, head), since workgroups go to the eight XCDs in turn: with eight, every token's
 // first chunk falls on the same one (48 sequences at 100..200, bound 4096: 354 us with 8, 300 with 10 and 9).
 constexpr int kChunkWGs = 3072;
